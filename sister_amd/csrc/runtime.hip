@@ -307,6 +307,10 @@ struct sister_ctx {
         hipEvent_t done;
     };
     PinnedPool pinned;
+    // pinned staging of sister_compute_rig, kept between calls up to kStageKeep
+    char* stage = nullptr;
+    size_t stage_bytes = 0;
+    static constexpr size_t kStageKeep = (size_t)256 << 20;
     std::thread server;
     std::mutex smu;
     std::condition_variable scv;
@@ -712,6 +716,7 @@ void sister_destroy(sister_ctx* c)
     c->timer.collect();
     c->pool.release_all();
     c->pinned.release_all();
+    if (c->stage) (void)hipHostFree(c->stage);
     (void)hipEventDestroy(c->ev_fork);
     for (int k = 0; k < sister_ctx::kMaxParts; k++) {
         if (c->ev_stage[k]) (void)hipEventDestroy(c->ev_stage[k]);
@@ -753,6 +758,19 @@ size_t sister_workspace_bytes(int W, int H, int D)
 
 int sister_outside_reference_domain(int D) { return D > 256 ? 1 : 0; }
 
+// Build the plan of a batch and issue it; the context stream's previous plan
+// is done (under mu, the device current).
+static int run_batch(sister_ctx* c, const sister_rig* rigs, int n, int modes)
+{
+    free_plan(c, c->last);
+    const int rc = build_plan_compact(c, rigs, n, c->last);
+    if (rc) return rc;
+    // profiling times every kernel on its own: the SGM families then run in sequence
+    enqueue(c, c->last, modes, c->stream, c->profiling ? nullptr : &c->fam[0], c->profiling ? &c->timer : nullptr);
+    HIPCHK(c, hipGetLastError());
+    return SISTER_OK;
+}
+
 int sister_run_device(sister_ctx* c, const sister_rig* rigs, int n, int modes)
 {
     if (!c || !rigs || n <= 0) return fail(c, SISTER_EINVAL, "bad arguments");
@@ -761,13 +779,7 @@ int sister_run_device(sister_ctx* c, const sister_rig* rigs, int n, int modes)
     std::lock_guard<std::mutex> lk(c->mu);
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipStreamSynchronize(c->stream));   // the previous plan may still be in use
-    free_plan(c, c->last);
-    rc = build_plan_compact(c, rigs, n, c->last);
-    if (rc) return rc;
-    // profiling times every kernel on its own: the SGM families then run in sequence
-    enqueue(c, c->last, modes, c->stream, c->profiling ? nullptr : &c->fam[0], c->profiling ? &c->timer : nullptr);
-    HIPCHK(c, hipGetLastError());
-    return SISTER_OK;
+    return run_batch(c, rigs, n, modes);
 }
 
 int sister_run_device_noalloc(sister_ctx* c, const sister_rig* rigs, int n, int modes)
@@ -801,6 +813,25 @@ int sister_sync(sister_ctx* c)
     return SISTER_OK;
 }
 
+// rows of a view <-> packed rows
+static void copy_rows(char* dst, const char* src, size_t w, size_t h, size_t stride)
+{
+    if (stride == w) {
+        std::memcpy(dst, src, w * h);
+        return;
+    }
+    for (size_t y = 0; y < h; y++) std::memcpy(dst + y * w, src + y * stride, w);
+}
+
+// The caller's pageable buffers go through pinned staging: a copy from or to
+// pageable memory is staged by the runtime itself, row by row for a 2D copy
+// (about 10 us per row: 24 of the 31 ms of a 640x480 three-mode call), while
+// the CPU moves 10 GB/s or more into a buffer that one asynchronous copy
+// takes.  Below kStageSplit bytes a view, one copy carries all five views (the
+// submission costs more than the copy); above, each view's copy runs while
+// the CPU packs the next one, and each output's while it unpacks the one before.
+constexpr size_t kStageSplit = (size_t)256 << 10;
+
 int sister_compute_rig(sister_ctx* c, const sister_rig* r, int modes)
 {
     if (!c || !r) return fail(c, SISTER_EINVAL, "bad arguments");
@@ -809,50 +840,99 @@ int sister_compute_rig(sister_ctx* c, const sister_rig* r, int modes)
     if (!valid_dims(r->width, r->height, r->disp_count))
         return fail(c, SISTER_EINVAL, "need W,H multiples of 4, D a multiple of 8 in [8,512], W+2D and H+2D at most 16384");
     if (r->stride < r->width) return fail(c, SISTER_EINVAL, "stride < width");
-    const size_t WH = (size_t)r->width * r->height;
+    for (int v = 0; v < 5; v++)
+        if (!r->view[v]) return fail(c, SISTER_EINVAL, "null view");
+    const size_t WH = (size_t)r->width * r->height, view_b = align_up(WH), map_b = align_up(WH * 2);
+    const size_t bytes = io_bytes(WH);
+    HIPCHK(c, hipSetDevice(c->device));
+    HIPCHK(c, hipStreamSynchronize(c->stream));   // the previous plan and staging may still be in use
+    if (c->stage_bytes < bytes) {
+        if (c->stage) (void)hipHostFree(c->stage);
+        c->stage = nullptr;
+        c->stage_bytes = 0;
+        if (hipHostMalloc((void**)&c->stage, bytes, hipHostMallocDefault) == hipSuccess) {
+            c->stage_bytes = bytes;
+        } else {
+            (void)hipGetLastError();
+            c->stage = nullptr;
+        }
+    }
+    char* const hs = c->stage;   // null: the copies run on the caller's buffers
     Block io;
     {
         std::lock_guard<std::mutex> lk(c->mu);
-        HIPCHK(c, hipSetDevice(c->device));
-        if (c->pool.get(io_bytes(WH), io) != 0)
-            return fail(c, SISTER_ENOMEM, "staging allocation failed");
+        if (c->pool.get(bytes, io) != 0) return fail(c, SISTER_ENOMEM, "staging allocation failed");
     }
-    char* p = io.ptr;
+    hipError_t e = hipSuccess;
     sister_rig d = *r;
     d.stride = r->width;
-    for (int v = 0; v < 5; v++) {
-        if (!r->view[v]) { c->pool.put(io); return fail(c, SISTER_EINVAL, "null view"); }
-        hipError_t e = hipMemcpy2DAsync(p, r->width, r->view[v], r->stride, r->width, r->height, hipMemcpyHostToDevice, c->stream);
-        if (e != hipSuccess) { c->pool.put(io); return fail(c, SISTER_EDEVICE, hipGetErrorString(e)); }
+    for (int v = 0; v < 5 && e == hipSuccess; v++) {
+        char* const p = io.ptr + v * view_b;
         d.view[v] = (const uint8_t*)p;
-        p += align_up(WH);
+        if (!hs) {
+            e = hipMemcpy2DAsync(p, r->width, r->view[v], r->stride, r->width, r->height, hipMemcpyHostToDevice, c->stream);
+            continue;
+        }
+        copy_rows(hs + v * view_b, (const char*)r->view[v], r->width, r->height, r->stride);
+        if (WH >= kStageSplit) e = hipMemcpyAsync(p, hs + v * view_b, WH, hipMemcpyHostToDevice, c->stream);
+        else if (v == 4) e = hipMemcpyAsync(io.ptr, hs, 4 * view_b + WH, hipMemcpyHostToDevice, c->stream);
     }
-    uint16_t* dm = (uint16_t*)p; p += align_up(WH * 2);
-    uint16_t* dh = (uint16_t*)p; p += align_up(WH * 2);
-    uint16_t* dv = (uint16_t*)p; p += align_up(WH * 2);
-    uint16_t* dd = (uint16_t*)p; p += align_up(WH * 2);
-    float* dsp = (float*)p;
-    d.out_multiview = (modes & 1) ? dm : nullptr;
-    d.out_horizontal = (modes & 2) ? dh : nullptr;
-    d.out_vertical = (modes & 4) ? dv : nullptr;
-    d.out_disp = r->out_disp ? dd : nullptr;
-    d.out_subpix = r->out_subpix ? dsp : nullptr;
-    rc = sister_run_device(c, &d, 1, modes);
-    if (rc == SISTER_OK) {
-        hipError_t e = hipSuccess;
-        if (modes & 1) e = hipMemcpyAsync(r->out_multiview, dm, WH * 2, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess && (modes & 2)) e = hipMemcpyAsync(r->out_horizontal, dh, WH * 2, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess && (modes & 4)) e = hipMemcpyAsync(r->out_vertical, dv, WH * 2, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess && r->out_disp) e = hipMemcpyAsync(r->out_disp, dd, WH * 2, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess && r->out_subpix) e = hipMemcpyAsync(r->out_subpix, dsp, WH * 4, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (e != hipSuccess) rc = fail(c, SISTER_EDEVICE, hipGetErrorString(e));
+    // outputs: multiview, horizontal, vertical, disp, subpix
+    struct Out { void* host; size_t off, bytes; };
+    const size_t o0 = 5 * view_b;
+    const Out all[5] = {{(modes & 1) ? r->out_multiview : nullptr, o0, WH * 2},
+                        {(modes & 2) ? r->out_horizontal : nullptr, o0 + map_b, WH * 2},
+                        {(modes & 4) ? r->out_vertical : nullptr, o0 + 2 * map_b, WH * 2},
+                        {(modes & 1) ? r->out_disp : nullptr, o0 + 3 * map_b, WH * 2},
+                        {(modes & 1) ? r->out_subpix : nullptr, o0 + 4 * map_b, WH * 4}};
+    auto dev = [&](int k) { return all[k].host ? (void*)(io.ptr + all[k].off) : nullptr; };
+    d.out_multiview = (uint16_t*)dev(0);
+    d.out_horizontal = (uint16_t*)dev(1);
+    d.out_vertical = (uint16_t*)dev(2);
+    d.out_disp = (uint16_t*)dev(3);
+    d.out_subpix = (float*)dev(4);
+    if (e == hipSuccess) {
+        std::lock_guard<std::mutex> lk(c->mu);
+        rc = run_batch(c, &d, 1, modes);
+    }
+    if (rc == SISTER_OK && e == hipSuccess) {
+        std::vector<Out> outs;
+        for (const Out& o : all)
+            if (o.host) outs.push_back(o);
+        auto unpack = [&](const Out& o) { std::memcpy(o.host, hs + o.off, o.bytes); };
+        if (!hs) {
+            for (size_t k = 0; k < outs.size() && e == hipSuccess; k++)
+                e = hipMemcpyAsync(outs[k].host, io.ptr + outs[k].off, outs[k].bytes, hipMemcpyDeviceToHost, c->stream);
+            if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        } else if (WH < kStageSplit) {
+            // one copy over the requested outputs (and whatever lies between)
+            const size_t a = outs.front().off, b = outs.back().off + outs.back().bytes;
+            e = hipMemcpyAsync(hs + a, io.ptr + a, b - a, hipMemcpyDeviceToHost, c->stream);
+            if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+            for (size_t k = 0; k < outs.size() && e == hipSuccess; k++) unpack(outs[k]);
+        } else {
+            hipEvent_t ev[2] = {c->ev_fork, c->ev_stage[0]};
+            for (size_t k = 0; k <= outs.size() && e == hipSuccess; k++) {
+                if (k < outs.size()) {
+                    e = hipMemcpyAsync(hs + outs[k].off, io.ptr + outs[k].off, outs[k].bytes, hipMemcpyDeviceToHost, c->stream);
+                    if (e == hipSuccess) e = hipEventRecord(ev[k & 1], c->stream);
+                }
+                if (k > 0 && e == hipSuccess) e = hipEventSynchronize(ev[(k - 1) & 1]);
+                if (k > 0 && e == hipSuccess) unpack(outs[k - 1]);
+            }
+        }
         if (c->profiling) c->timer.collect();
     }
-    {
-        std::lock_guard<std::mutex> lk(c->mu);
-        c->pool.put(io);
+    if (e != hipSuccess) rc = fail(c, SISTER_EDEVICE, hipGetErrorString(e));
+    // nothing on the stream may use the staging once it is given back
+    if (rc != SISTER_OK) (void)hipStreamSynchronize(c->stream);
+    if (c->stage_bytes > sister_ctx::kStageKeep) {
+        (void)hipHostFree(c->stage);
+        c->stage = nullptr;
+        c->stage_bytes = 0;
     }
+    std::lock_guard<std::mutex> lk(c->mu);
+    c->pool.put(io);
     return rc;
 }
 

@@ -282,3 +282,38 @@ def test_mode_subsets(gpu_ctx, oracle_mod, modes):
     assert sorted(k for k in got if k in ("multiview", "horizontal", "vertical")) == sorted(names)
     for k in names + (["disp"] if modes & 1 else []):
         assert np.array_equal(got[k], ref[k]), (k, int((got[k] != ref[k]).sum()))
+
+
+# The host form packs views into pinned staging: one copy for all five below
+# 256 KiB a view, a copy per view from there on.  Sizes on both sides of that
+# line and a small one after a large one (the staging is kept), views inside
+# wider rows, and every subset of the outputs' places.
+@pytest.mark.parametrize("W,H,modes,seed", [(512, 508, 7, 94), (512, 512, 7, 95), (516, 512, 5, 96), (16, 12, 6, 97)])
+def test_host_form_staging(gpu_ctx, oracle_mod, W, H, modes, seed):
+    import ctypes as C
+
+    import sister_amd
+    D, pitch = 8, W + 20
+    rig = synth.rig_small(W, H, D, seed)
+    ref = oracle_mod.compute(rig["views"], D, modes=modes)
+    print(f"[parity staging] W={W} H={H} D={D} modes={modes}", flush=True)
+    bufs = []
+    r = sister_amd.RigStruct()
+    r.width, r.height, r.stride, r.disp_count = W, H, pitch, D
+    for i, v in enumerate(rig["views"]):
+        b = np.full((H, pitch), 77, np.uint8)
+        b[:, :W] = v
+        bufs.append(b)
+        r.view[i] = b.ctypes.data
+    outs = {}
+    for bit, name, field in ((1, "multiview", "out_multiview"), (2, "horizontal", "out_horizontal"),
+                             (4, "vertical", "out_vertical"), (1, "disp", "out_disp")):
+        if modes & bit:
+            outs[name] = np.zeros((H, W), np.uint16)
+            setattr(r, field, outs[name].ctypes.data)
+    for _ in range(2):
+        for o in outs.values():
+            o[:] = 9
+        gpu_ctx._check(sister_amd.lib().sister_compute_rig(gpu_ctx._h, C.byref(r), modes))
+        for name, o in outs.items():
+            assert np.array_equal(o, ref[name]), name
