@@ -11,12 +11,13 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsister_hip.so")
-SOURCES = ["kernels.hip", "runtime.hip"]
+SOURCES = ["kernels.hip", "paths.hip", "runtime.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("SISTER_ARCH", "gfx950")
 
@@ -28,9 +29,9 @@ FLAGS = [
 
 
 def build(verbose=False):
-    objs = []
     os.makedirs(os.path.join(HERE, "_build"), exist_ok=True)
-    for src in SOURCES:
+
+    def compile_one(src):
         obj = os.path.join(HERE, "_build", src.replace(".hip", ".o"))
         cmd = [HIPCC, *FLAGS, "-I", os.path.join(ROOT, "include"), "-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
@@ -42,7 +43,10 @@ def build(verbose=False):
             raise RuntimeError(f"hipcc failed on {src}")
         if verbose and msgs:
             print("\n".join(msgs))
-        objs.append(obj)
+        return obj
+
+    with ThreadPoolExecutor(len(SOURCES)) as pool:
+        objs = list(pool.map(compile_one, SOURCES))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
     subprocess.run(cmd, check=True)

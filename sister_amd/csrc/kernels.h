@@ -15,10 +15,11 @@ enum Stage {
     kNumStages
 };
 
-// Launches whose code depends on the disparity count (cost sum, SGM
-// families) run per group of rigs with the same D.
+// Launches whose code depends on the disparity count (cost sum, SGM) run per
+// group of rigs with the same D.
 enum GroupKernel {
-    kGRows = 0, kGCols, kGDiag, kGAnti,   // SGM families
+    kGPaths = 0,                          // SGM chains (ahead of the fused sweep: the rows family's)
+    kGWinner,                             // S and the winner from the chains' bytes
     kGMsumRows, kGMsumCols,               // cost sum: frames 0/180 (row runs), 90/270 (column runs)
     kGMsumTile,                           // cost sum: all frames, per 16x16 tile
     kGVSweep,                             // fused vertical SGM families, per column block
@@ -30,7 +31,6 @@ struct DGroup {
     int D, Dp;
     const int* bs[kNumGroupKernels];   // block starts per kernel, nrig+1 entries each
     int blocks[kNumGroupKernels];
-    int CH[4], KL[4];        // SGM: chunks of 16 disparities per lane, lanes per chain, per family
     int vcols;               // fused vertical sweep: owned columns per block (0: separate families)
     int maxHp;               // tallest padded rig of the group
     int msum_split;          // 1: the two-launch cost sum even where the tiled one fits
@@ -55,7 +55,7 @@ struct LaunchSet {
 // individual kernels, for per-kernel event timing
 enum KernelId {
     kKCensus = 0, kKWta, kKMedianPrep, kKMedianSerial, kKMask, kKMsum,
-    kKRows, kKCols, kKDiag, kKAnti, kKVSweep, kNumKernels
+    kKRows, kKPaths, kKWinner, kKVSweep, kNumKernels
 };
 extern const char* const kKernelNames[kNumKernels];
 
@@ -69,9 +69,10 @@ struct KernelTimer {
 
 bool wta_rows_ok(int maxCols, int maxD);
 void stage_blocks(const RigDesc& g, int maxD, bool wta_rows, int out[kNumStages]);
-int sgm_pick_kl(long cols_chains, int fam, int D);
-int sgm_pick_ch(int D, int KL);
-int sgm_family_blocks(const RigDesc& g, int KL, int fam);
+// paths.hip: blocks of the chains of a rig's first nfam families (whole: over
+// the padded frame, debug sums) and of the winner
+int path_blocks(const RigDesc& g, int nfam, bool whole);
+int winner_blocks(const RigDesc& g, bool whole);
 int msum_blocks(const RigDesc& g, int side);   // side 0 row runs, 1 column runs, 2 tiles
 // fused vertical sweep: owned columns per block for a group whose rigs have
 // `cols` padded columns in all and disparity count D (0: not used)
@@ -86,14 +87,9 @@ void launch_wta(const LaunchSet& ls, hipStream_t st, KernelTimer* t);
 void launch_median(const LaunchSet& ls, hipStream_t st, KernelTimer* t);
 void launch_mask(const LaunchSet& ls, int fmask, hipStream_t st, KernelTimer* t);
 void launch_msum(const LaunchSet& ls, int fuse, hipStream_t st, KernelTimer* t);
-// Streams that let the rows, columns and diagonals families run concurrently
-// (they are independent; the anti-diagonal family, last, reads all three).
-struct FamStreams {
-    hipStream_t side[2];
-    hipEvent_t fork, join[2];
-};
-// keep_sum: also store the final S of cells inside the crop (debug).
-// fs == nullptr runs the four families in sequence on st.
-void launch_sgm(const LaunchSet& ls, int mode, int keep_sum, hipStream_t st, const FamStreams* fs, KernelTimer* t);
+void launch_paths(const DGroup& G, int keep_sum, hipStream_t st);
+void launch_winner(const DGroup& G, int mode, int keep_sum, hipStream_t st);
+// keep_sum: also store the final S of every cell (debug)
+void launch_sgm(const LaunchSet& ls, int mode, int keep_sum, hipStream_t st, KernelTimer* t);
 
 }  // namespace sister

@@ -8,9 +8,9 @@
 //   doLRCheck + mask loops postprocess.cpp:318-341,     k_mask
 //                          hpp:201-251
 //   realign + weighted sum hpp:255-277                  k_msum
-//   accumulateCostsSSE     sgm.cpp:26-455               k_fam<.., 0..3> (rows, columns,
-//                                                       diagonals, anti-diagonals)
-//   WTALeft on S, convert  hpp:283,111-118              fused into k_fam<.., 3>
+//   accumulateCostsSSE     sgm.cpp:26-455               k_paths (paths.hip); batches: rows
+//                                                       in k_paths, the rest in k_vsweep
+//   WTALeft on S, convert  hpp:283,111-118              k_winner (paths.hip), or in k_vsweep
 //
 // Every kernel takes the rig table plus a block-start table so one launch can
 // cover many rigs of different sizes: block b belongs to rig i when
@@ -20,45 +20,9 @@
 #include <cstdlib>
 #include "rig.h"
 #include "kernels.h"
+#include "lanes.h"
 
 namespace sister {
-
-// Device buffers reached through the rig table are generic pointers; casting
-// them to the global address space lets the compiler use global_load/store
-// with a scalar base (flat accesses need 64-bit per-lane addresses and also
-// hold the LDS counter).
-template <typename T> using gptr = __attribute__((address_space(1))) T*;
-template <typename T> __device__ __forceinline__ gptr<T> G(T* p) { return (gptr<T>)p; }
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint4 LD16(const void* p)
-{
-    const u32x4 v = *(gptr<const u32x4>)p;
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ void ST16(void* p, uint4 v) { *(gptr<u32x4>)p = u32x4{v.x, v.y, v.z, v.w}; }
-
-// ---------------------------------------------------------------------------
-// helpers
-// ---------------------------------------------------------------------------
-// Block index b of an n-block grid taken in XCD-contiguous order: with
-// round-robin dispatch block b runs on XCD b % 8, so the XCD gets the
-// consecutive logical blocks [start(b % 8), start(b % 8 + 1)) (the first
-// n % 8 XCDs one more than the others).  A bijection of [0, n).
-__device__ __forceinline__ int xcd_order(int b, int n)
-{
-    const int x = b & 7, k = b >> 3, q = n >> 3, r = n & 7;
-    return x < r ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
-}
-
-__device__ __forceinline__ int find_rig(const int* __restrict__ bs, int n, int b)
-{
-    int lo = 0, hi = n;
-    while (hi - lo > 1) {
-        int mid = (lo + hi) >> 1;
-        if (bs[mid] <= b) lo = mid; else hi = mid;
-    }
-    return lo;
-}
 
 // Popcounts accumulate in place: v_bcnt_u32_b32 adds its second operand, one
 // instruction per 32-bit half (written out, since the compiler reassociates
@@ -497,18 +461,6 @@ __global__ __launch_bounds__(256) void k_wta_fill(const RigDesc* __restrict__ ri
     uint16_t* const map = g.wta[m];
     const uint2 v = *(const uint2*)(map + (size_t)lo * C + c);
     for (int r = lo + 1; r <= hi; r++) *(uint2*)(map + (size_t)r * C + c) = v;
-}
-
-// compile-time loop: f(integral_constant<int, I>) for I in [B, E), so register
-// arrays indexed by I are never indexed at run time
-template <int I> struct IC { static constexpr int value = I; };
-template <int B, int E, class F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    if constexpr (B < E) {
-        f(IC<B>{});
-        static_for<B + 1, E>(f);
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1218,93 +1170,6 @@ __global__ __launch_bounds__(1024) void k_msum_tile(const RigDesc* __restrict__ 
     }
 }
 
-// ---------------------------------------------------------------------------
-// K6 SGM (sgm.cpp:26-455).  S is the sum of eight path costs; each path is a
-// family of independent chains (rows, columns, diagonals, anti-diagonals), each
-// swept in both directions.  One lane owns one chain and keeps all D
-// disparities of its path state in registers as packed u16 pairs, so d-1 / d+1
-// are a byte-permute of neighbouring registers, the minimum over d is a
-// running packed min, and no lane talks to another.
-//
-// Standard step (rows >= 1 of a pass, all paths; sgm.cpp:278-383):
-//   L(d) = M(d) + min(L'(d), min(L'(d-1), L'(d+1)) + P1, minL' + P2) - minL'
-// with L'(-1) = L'(D) = guard.  (L - M) is in [0, P2] and M <= 252, so the
-// reference's saturating u16 arithmetic never saturates and u16 lanes hold it.
-// Pass structure reproduced exactly (sgm.cpp:89-207):
-//   - on the first line of each pass (row 0 down, row H'-1 up) paths r1, r2,
-//     r3 only take the state c~ = (M == 255 ? 0 : M) and add nothing to S; the
-//     horizontal path r0 runs on c~ truncated to 8 bits (uint8 saturate_cast)
-//     and is the only contribution of that pass on that row;
-//   - r0 restarts every other row from L' = 0, minL' = 0 (L = M);
-//   - r1 / r3 entering from beyond the left/right border see L' = guard and
-//     minL' = 0, so L = M + P2 (the standard step from a guard state).
-// Each family stores, for rows 1..H'-2, (L_fwd - M) + (L_bwd - M) in [0, 200]
-// as a byte (part[f]; the rows family its two directions as separate bytes,
-// part[0] and rowsb, so they run independently), and for rows 0 and H'-1 its
-// exact contribution as u16 (edge[f]).  The anti-diagonal family runs last:
-// its upward sweep forms
-//   S = 8 M + part[0] + rowsb + part[1] + part[2] + its own (L - M) sum
-// (rows 1..H'-2) and takes the winner (hpp:283) for cells inside the crop.
-// ---------------------------------------------------------------------------
-typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-constexpr uint32_t kGuard2 = 0x3FFF3FFFu;
-
-__device__ __forceinline__ us2 U2(uint32_t v) { return __builtin_bit_cast(us2, v); }
-__device__ __forceinline__ uint32_t W2(us2 v) { return __builtin_bit_cast(uint32_t, v); }
-__device__ __forceinline__ us2 umin2(us2 a, us2 b) { return __builtin_elementwise_min(a, b); }
-// bytes b0,b1 of w -> pair (b0, b1); bytes b2,b3 -> pair (b2, b3)
-__device__ __forceinline__ uint32_t bytes01(uint32_t w) { return __builtin_amdgcn_perm(w, w, 0x0c010c00u); }
-__device__ __forceinline__ uint32_t bytes23(uint32_t w) { return __builtin_amdgcn_perm(w, w, 0x0c030c02u); }
-// low bytes of pairs a, b -> one word (a.lo, a.hi, b.lo, b.hi)
-__device__ __forceinline__ uint32_t pack4(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x06040200u); }
-__device__ __forceinline__ uint32_t dup16(uint32_t v) { return v | (v << 16); }
-// 255 -> 0 in both halves (paramInvalidDispCost, sgm.cpp:109-110,146-147)
-__device__ __forceinline__ uint32_t tilde2(uint32_t p)
-{
-    uint32_t lo = (p & 0xFFFFu) == 255u ? 0u : (p & 0xFFFFu);
-    uint32_t hi = (p >> 16) == 255u ? 0u : (p >> 16);
-    return lo | (hi << 16);
-}
-
-// unpack one 16-byte chunk of a u8 volume into 8 pairs, and back
-__device__ __forceinline__ void unpack16(const uint4& v, uint32_t (&p)[8])
-{
-    p[0] = bytes01(v.x); p[1] = bytes23(v.x);
-    p[2] = bytes01(v.y); p[3] = bytes23(v.y);
-    p[4] = bytes01(v.z); p[5] = bytes23(v.z);
-    p[6] = bytes01(v.w); p[7] = bytes23(v.w);
-}
-__device__ __forceinline__ uint4 pack16(const uint32_t (&p)[8])
-{
-    return make_uint4(pack4(p[0], p[1]), pack4(p[2], p[3]), pack4(p[4], p[5]), pack4(p[6], p[7]));
-}
-
-// DPP within a 16-lane row: lane i gets lane i-1 (shr) / i+1 (shl); 0 where
-// the source is outside the row (one DPP move, no fill value to materialise)
-__device__ __forceinline__ uint32_t row_shr1(uint32_t v)
-{
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true);
-}
-__device__ __forceinline__ uint32_t row_shl1(uint32_t v)
-{
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x101, 0xF, 0xF, true);
-}
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp_min(uint32_t v)
-{
-    return min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, CTRL, 0xF, 0xF, false));
-}
-// minimum over each aligned group of KL lanes (KL in 1,2,4,8,16), in every lane
-template <int KL>
-__device__ __forceinline__ uint32_t group_min(uint32_t v)
-{
-    if (KL >= 2) v = dpp_min<0xB1>(v);    // quad_perm [1,0,3,2]
-    if (KL >= 4) v = dpp_min<0x4E>(v);    // quad_perm [2,3,0,1]
-    if (KL >= 8) v = dpp_min<0x141>(v);   // row_half_mirror
-    if (KL >= 16) v = dpp_min<0x140>(v);  // row_mirror
-    return v;
-}
-
 // One chain is held by KL consecutive lanes; lane `lid` of the group owns
 // chunks [lid*CH, lid*CH + CH) of the chain's Dp/16 chunks (16 disparities,
 // 8 packed pairs each).  Chunks at or beyond nq are padding and stay guards.
@@ -1314,51 +1179,18 @@ struct LaneState {
     uint32_t mp;
 };
 
-// loads of one visited cell, issued a row ahead of their use
-template <int CH, int NO>
-struct RowBuf {
-    uint4 m[CH];      // cost M
-    uint4 p[CH];      // this family's forward (L - M), backward sweeps
-    uint4 o[NO * CH]; // the other families' parts (final sweep)
-};
-
 struct ChainGeo {
     int lid;        // lane within the chain group
     int nq;         // valid chunks of the chain
     bool half_tail; // D % 16 == 8: the last valid chunk holds 4 real pairs
 };
 
-// one standard step over the lane's chunks.  m = cost pairs per chunk;
-// returns (L - M) pairs in tp (ACC: adds them to tp).  trunc: 8-bit
-// first-line truncation.
-template <int CH, int KL, bool ACC, class MF, bool DEFER = false>
-__device__ __forceinline__ void lane_step_f(LaneState<CH>& st, const ChainGeo& cg, MF&& mpair,
-                                            uint32_t (&tp)[CH][8], bool trunc);
-
-template <int CH, int KL, bool ACC = false>
-__device__ __forceinline__ void lane_step(LaneState<CH>& st, const ChainGeo& cg, const uint32_t (&m)[CH][8],
-                                          uint32_t (&tp)[CH][8], bool trunc)
-{
-    lane_step_f<CH, KL, ACC>(st, cg, [&](int q, int i) __attribute__((always_inline)) { return m[q][i]; }, tp, trunc);
-}
-
-// the same step with the cost pairs taken from packed bytes (4 per word, 16 per chunk).
-// DEFER: the state is kept raw (minL' not subtracted): the new raw values are
-// the normalized ones plus the previous raw minimum, which the caller tracks.
-template <int CH, int KL, bool ACC = false, bool DEFER = false>
-__device__ __forceinline__ void lane_step_pk(LaneState<CH>& st, const ChainGeo& cg, const uint4 (&mb)[CH],
-                                             uint32_t (&tp)[CH][8])
-{
-    auto mf = [&](int q, int i) __attribute__((always_inline)) {
-        const uint32_t w = i < 2 ? mb[q].x : i < 4 ? mb[q].y : i < 6 ? mb[q].z : mb[q].w;
-        return (i & 1) ? bytes23(w) : bytes01(w);
-    };
-    lane_step_f<CH, KL, ACC, decltype(mf)&, DEFER>(st, cg, mf, tp, false);
-}
-
-template <int CH, int KL, bool ACC, class MF, bool DEFER>
-__device__ __forceinline__ void lane_step_f(LaneState<CH>& st, const ChainGeo& cg, MF&& mpair,
-                                            uint32_t (&tp)[CH][8], bool trunc)
+// One standard step (paths.hip) over the lane's chunks, the cost pairs taken
+// from packed bytes (4 per word, 16 per chunk).  DEFER: the state is kept raw
+// (minL' not subtracted): the new raw values are the normalized ones plus the
+// previous raw minimum, which the caller tracks.
+template <int CH, int KL, bool DEFER>
+__device__ __forceinline__ void lane_step(LaneState<CH>& st, const ChainGeo& cg, const uint4 (&mb)[CH])
 {
     // left lane's last pair and right lane's first pair (old); KL divides the
     // 16-lane DPP row, so the lanes at a row's ends are group ends, which take
@@ -1369,21 +1201,22 @@ __device__ __forceinline__ void lane_step_f(LaneState<CH>& st, const ChainGeo& c
     const uint32_t rfill = (cg.lid == KL - 1) ? kGuard2 : nbr;
     const uint32_t mpp = dup16(st.mp);
     const us2 p2t = U2(mpp) + (us2){(unsigned short)kP2, (unsigned short)kP2};
-    // truncation and padding as one and-or per pair: every new value is below
-    // 0x4000 (at most P2 + 255 normalised, raw values stay below the guard), so
-    // or-ing the guard 0x3FFF into a padding pair yields the guard itself
-    const uint32_t tmask = trunc ? 0x00FF00FFu : 0xFFFFFFFFu;
     us2 rmin = U2(0xFFFFFFFFu);
     static_for<0, CH>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         const int qg = cg.lid * CH + q;
         const bool valid = qg < cg.nq;
         const bool ht = cg.half_tail && qg == cg.nq - 1;
+        // every new value is below 0x4000 (at most P2 + 255 normalised, raw
+        // values stay below the guard), so or-ing the guard 0x3FFF into a
+        // padding pair yields the guard itself
         const uint32_t pad_lo = valid ? 0u : kGuard2;           // pairs 0..3 of the chunk
         const uint32_t pad_hi = valid && !ht ? 0u : kGuard2;    // pairs 4..7
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int j = 8 * q + i;
+            const uint32_t w = i < 2 ? mb[q].x : i < 4 ? mb[q].y : i < 6 ? mb[q].z : mb[q].w;
+            const uint32_t m = (i & 1) ? bytes23(w) : bytes01(w);
             const uint32_t cur = st.L[j];
             const uint32_t nxt = (j + 1 < 8 * CH) ? st.L[j + 1] : rfill;
             const us2 left = U2(__builtin_amdgcn_alignbit(cur, prv, 16));
@@ -1391,8 +1224,7 @@ __device__ __forceinline__ void lane_step_f(LaneState<CH>& st, const ChainGeo& c
             const us2 nb = umin2(left, right) + (us2){(unsigned short)kP1, (unsigned short)kP1};
             const us2 t = umin2(umin2(nb, U2(cur)), p2t);
             const us2 d = DEFER ? t : t - U2(mpp);
-            const us2 l = U2((W2(d + U2(mpair(q, i))) & tmask) | (i < 4 ? pad_lo : pad_hi));
-            tp[q][i] = ACC ? W2(U2(tp[q][i]) + d) : W2(d);
+            const us2 l = U2(W2(d + U2(m)) | (i < 4 ? pad_lo : pad_hi));
             st.L[j] = W2(l);
             prv = cur;
             rmin = umin2(rmin, l);
@@ -1437,359 +1269,10 @@ __device__ __forceinline__ uint4 add_u16x8(uint4 a, uint4 b)
     return make_uint4(W2(U2(a.x) + U2(b.x)), W2(U2(a.y) + U2(b.y)), W2(U2(a.z) + U2(b.z)), W2(U2(a.w) + U2(b.w)));
 }
 
-// prefetch depth of the family kernels (cells whose loads are in flight per
-// chain); overridable at build time for tuning.  At 16 lanes per chain the
-// rows, columns and diagonals take 8 (a single rig has under one wave per
-// SIMD, so the bytes in flight per wave set its bandwidth); the
-// anti-diagonal family, whose cells also carry three other families' bytes,
-// keeps 4 (8 would double its registers and halve its occupancy).
-#ifndef SISTER_PF16
-#define SISTER_PF16 8
-#endif
-#ifndef SISTER_PF16A
-#define SISTER_PF16A 4
-#endif
-#ifndef SISTER_PF8
-#define SISTER_PF8 2
-#endif
-#ifndef SISTER_PF4
-#define SISTER_PF4 2
-#endif
-template <int CH, int KL, int FAM>
-struct FamTune {
-    static constexpr int PF = KL == 16 ? (FAM == 3 ? SISTER_PF16A : SISTER_PF16) : (KL == 8 ? SISTER_PF8 : SISTER_PF4);
-};
-
-// Family kernel: FAM 0 rows (lanes over rows, steps along x), 1 columns,
-// 2 diagonals (k = x - y), 3 anti-diagonals (s = x + y, last, with the final
-// winner); each chain swept forward (pass 0 direction) then backward.
-template <int CH, int KL, int FAM>
-__global__ __launch_bounds__(64) void k_fam(const RigDesc* __restrict__ rigs, int nrig, const int* __restrict__ bs,
-                                            int mode, int keep_sum, int rsplit)
-{
-    // The rows family stores its two directions' (L - M) separately (forward
-    // in part[0], backward in rowsb), so neither reads the other.  rsplit: the
-    // two directions run as separate waves, the grid doubled and its second
-    // half sweeping backward; a wave holding the top or bottom row's chain,
-    // whose exact edge values add both directions, sweeps both in its
-    // first-half block.  For the anti-diagonal family rsplit 1 / 2 runs only
-    // the forward / backward (final) sweep: the forward one needs M alone, so
-    // it can run beside the other families.
-    extern __shared__ uint32_t lds_s[];   // final sweep: S pairs of the wave's chains
-    constexpr int CPW = 64 / KL;          // chains per wave
-    constexpr int NO = (FAM == 3) ? 4 : 1;
-    int bid = blockIdx.x, dsel = -1;      // dsel: the one direction of this block, -1 both
-    if (FAM == 0 && rsplit) {
-        const int half = bs[nrig];
-        dsel = bid >= half ? 1 : 0;
-        bid -= dsel * half;
-    }
-    const int ri = find_rig(bs, nrig, bid);
-    const RigDesc& g = rigs[ri];
-    const int lane = threadIdx.x;
-    const int grp = lane / KL;
-    ChainGeo cg;
-    cg.lid = lane % KL;
-    cg.nq = g.Dp >> 4;
-    cg.half_tail = (g.D & 15) != 0;
-    const int Wp = g.Wp, Hp = g.Hp, Dp = g.Dp, D = g.D;
-    const int c = (bid - bs[ri]) * CPW + grp;     // chain index
-    const int nchain = FAM == 0 ? Hp : (FAM == 1 ? Wp : Wp + Hp - 1);
-    const bool valid = c < nchain;
-    const int cw0 = (bid - bs[ri]) * CPW;
-    const int cw1 = min(cw0 + CPW - 1, nchain - 1);
-    uint8_t* part = g.part[FAM];
-    uint16_t* edge = g.edge + (size_t)FAM * 2 * (size_t)Wp * Dp;
-    const int boff = cg.lid * CH * 16;     // byte offset of the lane's chunks in a cell
-    const bool final_pass = FAM == 3;
-    // rows family: byte offset of the lane's chunks in column 0 of its row
-    const size_t row_off = FAM == 0 ? (size_t)(valid ? c : 0) * Wp * Dp + boff : 0;
-    // other families: the chain's cell at row y lies at y (W' + s) Dp + lane_off,
-    // the row term uniform over the wave (s = 0 columns, +1 diagonals, -1
-    // anti-diagonals; lane_off may be negative where the chain starts left of
-    // column 0, and is used only at active cells)
-    const long ystride = (long)(Wp + (FAM == 2 ? 1 : FAM == 3 ? -1 : 0)) * Dp;
-    const long lane_off = (long)(FAM == 2 ? c - (Hp - 1) : c) * Dp + boff;
-
-    // ---- chain geometry --------------------------------------------------
-    // steps 0..n-1 of the wave; cell of chain c at step t, per direction
-    int nsteps;
-    int ylo = 0, yhi = 0, ent_dn = 0, ent_up = 0;
-    if (FAM == 0) {
-        nsteps = Wp;
-    } else if (FAM == 1) {
-        ylo = 0; yhi = Hp - 1; ent_dn = 0; ent_up = Hp - 1;
-        nsteps = Hp;
-    } else if (FAM == 2) {
-        const int klo = cw0 - (Hp - 1), khi = cw1 - (Hp - 1);
-        ylo = max(0, -khi); yhi = min(Hp - 1, Wp - 1 - klo);
-        ent_dn = max(0, -klo); ent_up = min(Hp - 1, Wp - 1 - khi);
-        nsteps = yhi - ylo + 1;
-    } else {
-        ylo = max(0, cw0 - (Wp - 1)); yhi = min(Hp - 1, cw1);
-        ent_dn = max(0, cw1 - (Wp - 1)); ent_up = min(Hp - 1, cw0);
-        nsteps = yhi - ylo + 1;
-    }
-    auto cell_of = [&](int dir, int t, int& y, int& x) {
-        if (FAM == 0) { y = c; x = dir == 0 ? t : Wp - 1 - t; return; }
-        y = dir == 0 ? ylo + t : yhi - t;
-        if (FAM == 1) x = c;
-        else if (FAM == 2) x = y + (c - (Hp - 1));
-        else x = c - y;
-    };
-    auto is_active = [&](int y, int x) { return valid && x >= 0 && x < Wp && y >= 0 && y < Hp; };
-
-    const bool top = FAM == 0 && c == 0, bot = FAM == 0 && c == Hp - 1;
-    const bool want_sub = final_pass && mode == 0 && g.subpix != nullptr;
-    uint16_t* outm = g.out[mode];
-
-    int dlo = 0, dhi = 1;
-    if (FAM == 3 && rsplit) dlo = dhi = rsplit - 1;
-    if (dsel >= 0) {
-        const bool edge_wave = cw0 == 0 || cw1 >= Hp - 1;
-        if (edge_wave) {
-            if (dsel == 1) return;
-        } else {
-            dlo = dhi = dsel;
-        }
-    }
-    LaneState<CH> st;
-    for (int dir = dlo; dir <= dhi; dir++) {
-        lane_guard<CH>(st, false);
-        const bool need_p = dir == 1 && FAM != 0;
-        const bool need_o = final_pass && dir == 1;
-        auto fetch = [&](int t, RowBuf<CH, NO>& b) __attribute__((always_inline)) {
-            if constexpr (FAM == 0) {
-                // rows: the lane's row offset is fixed, the column uniform
-                const int x = dir == 0 ? t : Wp - 1 - t;
-                const uint8_t* src = g.msum + row_off + (size_t)x * Dp;
-                static_for<0, CH>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-                    const bool ok = t < nsteps && valid && cg.lid * CH + q < cg.nq;
-                    // not loaded: a padding chunk (its pairs take the guard whatever
-                    // bytes they hold), a chain past the rig (never stored) or a
-                    // step past the row (never processed): no zero fill
-                    if (ok) b.m[q] = LD16(src + 16 * q);
-                });
-                return;
-            }
-            int y, x;
-            cell_of(dir, t, y, x);
-            const bool act = t < nsteps && is_active(y, x);
-            const size_t off = (size_t)((long)y * ystride + lane_off);
-            static_for<0, CH>([&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                const bool ok = act && cg.lid * CH + q < cg.nq;
-                b.m[q] = ok ? LD16(g.msum + off + 16 * q) : make_uint4(0, 0, 0, 0);
-                if (need_p) b.p[q] = ok ? LD16(part + off + 16 * q) : make_uint4(0, 0, 0, 0);
-                if (need_o) {
-                    b.o[q] = ok ? LD16(g.part[0] + off + 16 * q) : make_uint4(0, 0, 0, 0);
-                    if constexpr (NO == 4) {
-                        b.o[CH + q] = ok ? LD16(g.part[1] + off + 16 * q) : make_uint4(0, 0, 0, 0);
-                        b.o[2 * CH + q] = ok ? LD16(g.part[2] + off + 16 * q) : make_uint4(0, 0, 0, 0);
-                        b.o[3 * CH + q] = ok ? LD16(g.rowsb + off + 16 * q) : make_uint4(0, 0, 0, 0);
-                    }
-                }
-            });
-        };
-        auto process = [&](int t, RowBuf<CH, NO>& b) __attribute__((always_inline)) {
-            int y, x;
-            cell_of(dir, t, y, x);
-            const bool act = is_active(y, x);
-            const size_t off = (size_t)((long)y * ystride + lane_off);   // used at active cells
-            uint32_t m[CH][8], tp[CH][8];
-            static_for<0, CH>([&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                unpack16(b.m[q], m[q]);
-            });
-            // ---------------- rows family ----------------
-            if (FAM == 0) {
-                const bool first_line = dir == 0 ? top : bot;   // 255 -> 0, 8-bit truncation
-                if (first_line) {
-                    static_for<0, CH>([&](auto qc) {
-                        constexpr int q = decltype(qc)::value;
-#pragma unroll
-                        for (int i = 0; i < 8; i++) m[q][i] = tilde2(m[q][i]);
-                    });
-                }
-                if (t == 0) {
-                    lane_set<CH, KL>(st, cg, m, true);      // L = M (c~ on a first line), contributes
-                    static_for<0, CH>([&](auto qc) {
-                        constexpr int q = decltype(qc)::value;
-#pragma unroll
-                        for (int i = 0; i < 8; i++) tp[q][i] = 0;
-                    });
-                } else {
-                    lane_step<CH, KL>(st, cg, m, tp, first_line);
-                }
-                if (!act) return;
-                const bool edge_row = top || bot;
-                // its bytes are read only where S is: at the crop, or everywhere
-                // with the debug sums
-                const bool crop = keep_sum || (y >= D && y < D + g.H && x >= D && x < D + g.W);
-                static_for<0, CH>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-                    if (cg.lid * CH + q >= cg.nq) return;
-                    if (edge_row) {
-                        uint16_t* e = edge + ((size_t)(top ? 0 : 1) * Wp + x) * Dp + (cg.lid * CH + q) * 16;
-                        uint4 a = make_uint4(st.L[8 * q + 0], st.L[8 * q + 1], st.L[8 * q + 2], st.L[8 * q + 3]);
-                        uint4 bb = make_uint4(st.L[8 * q + 4], st.L[8 * q + 5], st.L[8 * q + 6], st.L[8 * q + 7]);
-                        if (cg.half_tail && cg.lid * CH + q == cg.nq - 1) bb = make_uint4(0, 0, 0, 0);
-                        if (dir == 1) {
-                            a = add_u16x8(a, LD16(e));
-                            bb = add_u16x8(bb, LD16(e + 8));
-                        }
-                        ST16(e, a);
-                        ST16(e + 8, bb);
-                    } else if (crop) {
-                        ST16((dir == 1 ? g.rowsb : part) + row_off + (size_t)x * Dp + 16 * q, pack16(tp[q]));
-                    }
-                });
-                return;
-            }
-            // ---------------- vertical families ----------------
-            const int first_row = dir == 0 ? 0 : Hp - 1;
-            if (y == first_row) {
-                // first line of the pass: state c~, no contribution (sgm.cpp:103-207)
-                static_for<0, CH>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-#pragma unroll
-                    for (int i = 0; i < 8; i++) m[q][i] = tilde2(m[q][i]);
-                });
-                lane_set<CH, KL>(st, cg, m, act);
-                if (final_pass && keep_sum && g.sum && act) {
-                    // S of row H'-1 = the four families' exact edge rows
-                    static_for<0, CH>([&](auto qc) {
-                        constexpr int q = decltype(qc)::value;
-                        if (cg.lid * CH + q >= cg.nq) return;
-                        const size_t eo = (size_t)x * Dp + cg.lid * CH * 16 + 16 * q;
-#pragma unroll
-                        for (int h = 0; h < 2; h++) {
-                            uint4 acc = make_uint4(0, 0, 0, 0);
-#pragma unroll
-                            for (int fm = 0; fm < 4; fm++)
-                                acc = add_u16x8(acc, LD16(g.edge + (size_t)(fm * 2 + 1) * Wp * Dp + eo + 8 * h));
-                            ST16(g.sum + ((size_t)y * Wp) * Dp + eo + 8 * h, acc);
-                        }
-                    });
-                }
-                return;
-            }
-            lane_step<CH, KL>(st, cg, m, tp, false);
-            const bool entering = dir == 0 ? (y <= ent_dn) : (y >= ent_up);
-            if (entering) lane_guard<CH>(st, act);
-            const bool edge_row = (y == 0 || y == Hp - 1);
-            const int oy = y - D, ox = x - D;
-            const bool crop = final_pass && act && oy >= 0 && oy < g.H && ox >= 0 && ox < g.W;
-            uint32_t key = 0xFFFFFFFFu;
-            static_for<0, CH>([&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                const int qg = cg.lid * CH + q;
-                if (!act || qg >= cg.nq) return;
-                if (edge_row) {
-                    uint16_t* e = edge + ((size_t)(y == 0 ? 0 : 1) * Wp + x) * Dp + qg * 16;
-                    uint4 a = make_uint4(st.L[8 * q + 0], st.L[8 * q + 1], st.L[8 * q + 2], st.L[8 * q + 3]);
-                    uint4 bb = make_uint4(st.L[8 * q + 4], st.L[8 * q + 5], st.L[8 * q + 6], st.L[8 * q + 7]);
-                    if (cg.half_tail && qg == cg.nq - 1) bb = make_uint4(0, 0, 0, 0);
-                    ST16(e, a);
-                    ST16(e + 8, bb);
-                    if (final_pass && keep_sum && g.sum && y == 0) {
-                        // S of row 0: the other families' edge rows + this sweep
-                        const size_t eo = (size_t)x * Dp + qg * 16;
-                        uint4 s0 = a, s1 = bb;
-#pragma unroll
-                        for (int fm = 0; fm < 3; fm++) {
-                            s0 = add_u16x8(s0, LD16(g.edge + (size_t)(fm * 2) * Wp * Dp + eo));
-                            s1 = add_u16x8(s1, LD16(g.edge + (size_t)(fm * 2) * Wp * Dp + eo + 8));
-                        }
-                        ST16(g.sum + eo, s0);
-                        ST16(g.sum + eo + 8, s1);
-                    }
-                    return;
-                }
-                if (dir == 0) {
-                    ST16(part + off + 16 * q, pack16(tp[q]));
-                    return;
-                }
-                uint32_t pf[8];
-                unpack16(b.p[q], pf);
-#pragma unroll
-                for (int i = 0; i < 8; i++) tp[q][i] = W2(U2(tp[q][i]) + U2(pf[i]));
-                if (!final_pass) {
-                    ST16(part + off + 16 * q, pack16(tp[q]));
-                    return;
-                }
-                if (!(crop || keep_sum)) return;
-                // S = 8 M + part[rows] + part[cols] + part[diag] + this family
-                uint32_t pr[8], pc[8], pd[8], S[8];
-                const uint4 rf = b.o[q], rb = b.o[NO == 4 ? 3 * CH + q : q];
-                unpack16(make_uint4(rf.x + rb.x, rf.y + rb.y, rf.z + rb.z, rf.w + rb.w), pr);   // bytes <= 200
-                unpack16(b.o[NO == 4 ? CH + q : q], pc);
-                unpack16(b.o[NO == 4 ? 2 * CH + q : q], pd);
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const us2 s8 = U2(m[q][i]) << (us2){3, 3};
-                    S[i] = W2(s8 + U2(pr[i]) + U2(pc[i]) + U2(pd[i]) + U2(tp[q][i]));
-                }
-                if (keep_sum && g.sum) {
-                    uint16_t* sc = g.sum + (off - boff) + qg * 16;
-                    ST16(sc, make_uint4(S[0], S[1], S[2], S[3]));
-                    ST16(sc + 8, make_uint4(S[4], S[5], S[6], S[7]));
-                }
-                if (!crop) return;
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const uint32_t d0 = (uint32_t)(qg * 16 + 2 * i);
-                    const uint32_t k0 = ((S[i] & 0xFFFFu) << 9) | d0;
-                    const uint32_t k1 = ((S[i] >> 16) << 9) | (d0 + 1);
-                    key = min(key, d0 < (uint32_t)D ? k0 : 0xFFFFFFFFu);
-                    key = min(key, d0 + 1 < (uint32_t)D ? k1 : 0xFFFFFFFFu);
-                    if (want_sub) lds_s[(grp * cg.nq * 8) + qg * 8 + i] = S[i];
-                }
-            });
-            if (final_pass && dir == 1) {
-                // the winner of each chain's cell: minimum key over the group
-                key = group_min<KL>(key);
-                if (want_sub) __syncthreads();
-                if (crop && cg.lid == 0) {
-                    const uint32_t best = key & 511u;
-                    const size_t o = (size_t)oy * g.W + ox;
-                    if (outm) G(outm)[o] = (uint16_t)min(best * 255u, 65535u);
-                    if (mode == 0 && g.disp) G(g.disp)[o] = (uint16_t)best;
-                    if (want_sub) {
-                        float delta = 0.0f;
-                        if (best > 0 && (int)best < D - 1) {
-                            const uint16_t* sv = (const uint16_t*)(lds_s + grp * cg.nq * 8);
-                            const int sm = sv[best - 1], s0 = (int)(key >> 9), sp = sv[best + 1];
-                            const int den = sm - 2 * s0 + sp;
-                            if (den > 0) delta = (float)(sm - sp) / (2.0f * (float)den);
-                        }
-                        G(g.subpix)[o] = (float)best + delta;
-                    }
-                }
-                if (want_sub) __syncthreads();
-            }
-        };
-        // software pipeline: a ring of PF cell buffers, the loads of the next
-        // PF - 1 cells in flight while the current one is computed
-        constexpr int PF = FamTune<CH, KL, FAM>::PF;
-        RowBuf<CH, NO> ring[PF];
-        static_for<0, PF - 1>([&](auto ic) __attribute__((always_inline)) {
-            fetch(decltype(ic)::value, ring[decltype(ic)::value]);
-        });
-        for (int t = 0; t < nsteps; t += PF) {
-            static_for<0, PF>([&](auto ic) __attribute__((always_inline)) {
-                constexpr int i = decltype(ic)::value;
-                fetch(t + i + PF - 1, ring[(i + PF - 1) % PF]);
-                if (t + i < nsteps) process(t + i, ring[i]);
-            });
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------
 // K6b fused vertical families: the column, diagonal and anti-diagonal chains
-// of a pass in one sweep (same recurrence and pass rules as k_fam).  Lanes own
+// of a pass in one sweep (same recurrence and pass rules as
+// k_paths).  Lanes own
 // columns (kVKL = 4 lanes per column, CH chunks of 16 disparities each), so
 // every cell of a row sees its three vertical paths in one lane group:
 //   downward pass:  P = rows_fwd + rows_bwd + sum_f (L_f,down - M)  (u16, rows 1..H'-2)
@@ -1808,8 +1291,8 @@ __global__ __launch_bounds__(64) void k_fam(const RigDesc* __restrict__ rigs, in
 // one segment of kVGhost rows, and the states cross segments through memory
 // (owned columns stored at the end, owned + ghost columns loaded at the start).
 // No block ever waits for another.
-// Buffers: the rows family's two directions in part[0] and rowsb (bytes,
-// added as words: each sum is at most 200), P (u16) in part[1..2], or over
+// Buffers: the rows family's two directions in part[0] and part[1] (bytes,
+// added as words: each sum is at most 200), P (u16) in psum, or over
 // the rows bytes once the down pass has read them in plans short of memory
 // (pd_at below), the segment states in vstate
 // ([parity][cols, diag, anti][W'][Dp + 16] bytes: the normalised (L - M)
@@ -1947,27 +1430,27 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
     // column's states are reset to guards and nothing of it is stored
     const int xc = min(max(x, 0), Wp - 1);
     // P is this kernel's own intermediate (rows 1..H'-2).  When the plan gives
-    // it volumes of its own (part[1..2]): FULL, planes per (row, chunk slot
+    // it volumes of its own (psum): FULL, planes per (row, chunk slot
     // q, half h) in which lane (x, lid) holds 8 u16 at byte (x KL + lid) * 16,
     // so a wave's 64 lanes move 1 KB contiguous per access (3 ms faster than
     // the cell layout at 16 rigs); otherwise cell layout (chunk qg of cell
     // (y, x) at (y W' + x) Dp + 16 qg).
-    // Plans short of memory give it none (part[1] null, FULL only): P then
+    // Plans short of memory give it none (psum null, FULL only): P then
     // takes the place of the rows family's bytes of the same row and columns,
     // which the down pass reads just before it stores P.  The 2 Dp bytes of
-    // column x occupy its Dp part[0] bytes and its Dp rowsb bytes, and only
+    // column x occupy its Dp part[0] bytes and its Dp part[1] bytes, and only
     // the wave that owns column x reads or writes them; its loads of the row's
     // bytes complete before its P stores (P depends on them).  A lane's
-    // 16-byte piece k = 2 q + h lies in part[0] for k < CH, in rowsb above.
+    // 16-byte piece k = 2 q + h lies in part[0] for k < CH, in part[1] above.
     // Waves whose columns all lie inside the row keep whole-wave planes:
     // plane k of the wave's 64 / KL columns is 1 KB with wave lane l at byte
     // 16 l, planes 0..CH-1 over the wave's part[0] bytes of the row and
-    // CH..2CH-1 over its rowsb bytes.  The others (the last wave of a row)
+    // CH..2CH-1 over its part[1] bytes.  The others (the last wave of a row)
     // keep a column's pieces together: piece k of lane lid at 16 (lid CH +
     // k mod CH) in the column's bytes of its half.  (1.3 ms slower per
     // 64-rig step than volumes of its own.)  Either way the address is a
     // uniform base plus a loop-invariant lane offset.
-    uint16_t* const Pd = (uint16_t*)g.part[1];
+    uint16_t* const Pd = g.psum;
     const bool p_own = Pd != nullptr;
     constexpr int CPW = 64 / KL;                       // columns per wave
     const int lw = tid & 63;
@@ -1988,7 +1471,7 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
             }
             const int k = 2 * q + h, r = k >= CH ? 1 : 0, kk = k - r * CH;
             const size_t s = (size_t)y * Wp * Dp + (wave_planes ? (size_t)x0w * Dp + kk * 1024 : (size_t)kk * 16);
-            return (uint16_t*)((r ? g.rowsb : g.part[0]) + s + pd_lane);
+            return (uint16_t*)(g.part[r] + s + pd_lane);
         }
         return Pd + ((size_t)y * Wp + x) * Dp + boff + 16 * q + 8 * h;
     };
@@ -2064,13 +1547,13 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
             b[q] = FULL ? LD16(msum + cell + 16 * q) : ok ? LD16(msum + cell + 16 * q) : make_uint4(0, 0, 0, 0);
         });
     };
-    // exact L of a family on an edge row (debug sums only), as k_fam stores it
+    // exact L of a family on an edge row (debug sums only)
     auto edge_out = [&](int f, int y, const LaneState<CH>& st) __attribute__((always_inline)) {
         static_for<0, CH>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             const int qg = cg.lid * CH + q;
             if (qg >= cg.nq) return;
-            uint16_t* e = g.edge + ((size_t)(f * 2 + (y == 0 ? 0 : 1)) * Wp + x) * Dp + qg * 16;
+            uint16_t* e = g.edge + ((size_t)((f - 1) * 2 + (y == 0 ? 0 : 1)) * Wp + x) * Dp + qg * 16;
             const uint4 a = make_uint4(st.L[8 * q + 0], st.L[8 * q + 1], st.L[8 * q + 2], st.L[8 * q + 3]);
             uint4 bb = make_uint4(st.L[8 * q + 4], st.L[8 * q + 5], st.L[8 * q + 6], st.L[8 * q + 7]);
             if (cg.half_tail && qg == cg.nq - 1) bb = make_uint4(0, 0, 0, 0);
@@ -2078,7 +1561,9 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
             ST16(e + 8, bb);
         });
     };
-    // S of an edge row (debug): the four families' exact rows summed
+    // S of an edge row (debug): the three vertical families' exact rows and the
+    // rows family's two directions, of which the one of this line's own pass is
+    // the 8-bit first-line path
     auto edge_sum = [&](int y) __attribute__((always_inline)) {
         const int e = y == 0 ? 0 : 1;
         static_for<0, CH>([&](auto qc) {
@@ -2086,11 +1571,19 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
             const int qg = cg.lid * CH + q;
             if (qg >= cg.nq) return;
             const size_t eo = (size_t)x * Dp + qg * 16;
+            const size_t ro = ((size_t)y * Wp + x) * Dp + qg * 16;
+            uint32_t m[8], b8[8], bs8[8];
+            unpack16(LD16(g.msum + ro), m);
+            unpack16(LD16(g.part[e] + ro), b8);
+            unpack16(LD16(g.part[e ^ 1] + ro), bs8);
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                m[i] = (W2(U2(m[i]) + U2(b8[i])) & 0x00FF00FFu) + W2(U2(m[i]) + U2(bs8[i]));
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                uint4 acc = make_uint4(0, 0, 0, 0);
+                uint4 acc = make_uint4(m[4 * h], m[4 * h + 1], m[4 * h + 2], m[4 * h + 3]);
 #pragma unroll
-                for (int fm = 0; fm < 4; fm++)
+                for (int fm = 0; fm < 3; fm++)
                     acc = add_u16x8(acc, LD16(g.edge + (size_t)(fm * 2 + e) * Wp * Dp + eo + 8 * h));
                 ST16(g.sum + (size_t)y * Wp * Dp + eo + 8 * h, acc);
             }
@@ -2163,7 +1656,7 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
                 if (!FULL && cg.lid * CH + q >= cg.nq) return;
                 if (DIR == 0) {
                     ob[q] = LD16(g.part[0] + cell + 16 * q);
-                    ob[CH + q] = LD16(g.rowsb + cell + 16 * q);
+                    ob[CH + q] = LD16(g.part[1] + cell + 16 * q);
                 } else {
                     ob[2 * q] = LD16(pd_at(y, q, 0));
                     ob[2 * q + 1] = LD16(pd_at(y, q, 1));
@@ -2178,13 +1671,12 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
         // the second.  The next row's FL reads follow this row's second
         // barrier, its FR reads its own first one, which orders them after
         // this row's writes.
-        uint32_t dead[CH][8];
         slot_read(XL, c - 1, sx);
         __syncthreads();
         uint32_t off;   // DEFER: sum of the three pre-step minima
         {
             off = sx.mp;
-            lane_step_pk<CH, KL, false, DEFER>(sx, cg, mc, dead);
+            lane_step<CH, KL, DEFER>(sx, cg, mc);
             if (!wave_act) lane_guard<CH>(sx, act);
             slot_write(XL, sx);
             if (own && edge_row && keep_sum && g.sum && act) edge_out(famL, y, sx);
@@ -2192,7 +1684,7 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
         __builtin_amdgcn_sched_barrier(0);
         {
             off += sc.mp;
-            lane_step_pk<CH, KL, false, DEFER>(sc, cg, mc, dead);
+            lane_step<CH, KL, DEFER>(sc, cg, mc);
             if (own && edge_row && keep_sum && g.sum && act) edge_out(1, y, sc);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -2200,7 +1692,7 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
         __syncthreads();
         {
             off += sx.mp;
-            lane_step_pk<CH, KL, false, DEFER>(sx, cg, mc, dead);
+            lane_step<CH, KL, DEFER>(sx, cg, mc);
             if (!wave_act) lane_guard<CH>(sx, act);
             slot_write(XR, sx);
             if (own && edge_row && keep_sum && g.sum && act) edge_out(famR, y, sx);
@@ -2258,7 +1750,7 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
             });
             continue;
         }
-        // upward pass: S and the winner (hpp:283), as k_fam's final sweep
+        // upward pass: S and the winner (hpp:283)
         const int oy = y - D, ox = x - D;
         const bool crop = oy >= 0 && oy < g.H && ox >= 0 && ox < g.W;
         if (!(crop || keep_sum)) continue;
@@ -2336,76 +1828,13 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
 // ---------------------------------------------------------------------------
 // host-side launchers
 // ---------------------------------------------------------------------------
-// SGM launches: (CH chunks per lane, KL lanes per chain) instantiations
-#define SISTER_FAM_LAUNCH(CHV, KLV, FAM, ...) hipLaunchKernelGGL((k_fam<CHV, KLV, FAM>), __VA_ARGS__)
-#define SISTER_FAM_KL4(CHV, FAM, ...)                                                            \
-    switch (CHV) {                                                                               \
-    case 1: SISTER_FAM_LAUNCH(1, 4, FAM, __VA_ARGS__); break;                                    \
-    case 2: SISTER_FAM_LAUNCH(2, 4, FAM, __VA_ARGS__); break;                                    \
-    case 3: SISTER_FAM_LAUNCH(3, 4, FAM, __VA_ARGS__); break;                                    \
-    default: SISTER_FAM_LAUNCH(4, 4, FAM, __VA_ARGS__); break;                                   \
-    }
-#define SISTER_FAM_KL8(CHV, FAM, ...)                                                            \
-    switch (CHV) {                                                                               \
-    case 1: SISTER_FAM_LAUNCH(1, 8, FAM, __VA_ARGS__); break;                                    \
-    case 2: SISTER_FAM_LAUNCH(2, 8, FAM, __VA_ARGS__); break;                                    \
-    case 3: SISTER_FAM_LAUNCH(3, 8, FAM, __VA_ARGS__); break;                                    \
-    default: SISTER_FAM_LAUNCH(4, 8, FAM, __VA_ARGS__); break;                                   \
-    }
-#define SISTER_FAM_KL16(CHV, FAM, ...)                                                           \
-    switch (CHV) {                                                                               \
-    case 1: SISTER_FAM_LAUNCH(1, 16, FAM, __VA_ARGS__); break;                                   \
-    default: SISTER_FAM_LAUNCH(2, 16, FAM, __VA_ARGS__); break;                                  \
-    }
-#define SISTER_FAM(G, FAM, ...)                                                                  \
-    do {                                                                                         \
-        if ((G).KL[FAM] == 16) { SISTER_FAM_KL16((G).CH[FAM], FAM, __VA_ARGS__); }               \
-        else if ((G).KL[FAM] == 8) { SISTER_FAM_KL8((G).CH[FAM], FAM, __VA_ARGS__); }            \
-        else { SISTER_FAM_KL4((G).CH[FAM], FAM, __VA_ARGS__); }                                  \
-    } while (0)
-
-int sgm_pick_kl(long cols_chains, int fam, int D)
-{
-    // SISTER_SGM_LANES (4, 8 or 16) overrides the choice, for tuning; 4 lanes
-    // hold at most 256 disparities (beyond that the state would spill)
-    static const int forced = [] {
-        const char* e = getenv("SISTER_SGM_LANES");
-        const int v = e ? atoi(e) : 0;
-        return (v == 4 || v == 8 || v == 16) ? v : 0;
-    }();
-    if (forced) return (forced == 4 && D > 256) ? 8 : forced;
-    // A single rig has few chains: 16 lanes per chain keep the most waves in
-    // flight.  In a batch (measured on 16 rigs of 2304x1464x192 cells) rows
-    // and columns are still fastest with 16 lanes per chain, the diagonal
-    // families, whose final sweep carries the most registers, with 8.
-    if (cols_chains * 4 / 64 < 1024) return 16;
-    return fam >= 2 ? 8 : 16;
-}
-
-int sgm_pick_ch(int D, int KL)
-{
-    const int k16 = ((D + 15) / 16);
-    int ch = (k16 + KL - 1) / KL;
-    if (KL == 16) return ch <= 1 ? 1 : 2;
-    return ch <= 3 ? ch : 4;   // KL 8 (D <= 512) and KL 4 (D <= 256)
-}
-
-int sgm_family_blocks(const RigDesc& g, int KL, int fam)
-{
-    const int cpw = 64 / KL;
-    const int chains = fam == 0 ? g.Hp : (fam == 1 ? g.Wp : g.Wp + g.Hp - 1);
-    return (chains + cpw - 1) / cpw;
-}
-
 const char* const kKernelNames[kNumKernels] = {
     "census", "wta", "median_prep", "median_serial", "mask", "msum",
-    "sgm_rows", "sgm_cols", "sgm_diag", "sgm_anti", "sgm_vsweep",
+    "sgm_rows", "sgm_paths", "winner", "sgm_vsweep",
 };
 
 #define TB(id) do { if (t) t->begin(id, st); } while (0)
 #define TE(id) do { if (t) t->end(id, st); } while (0)
-#define TB_S(id, s) do { if (t) t->begin(id, s); } while (0)
-#define TE_S(id, s) do { if (t) t->end(id, s); } while (0)
 #define TD(id, n) do { if (t) t->dispatched[id] += (n); } while (0)
 
 void launch_census(const LaunchSet& ls, hipStream_t st, KernelTimer* t)
@@ -2694,84 +2123,24 @@ static int launch_vsweep(const DGroup& G, int mode, int keep_sum, hipStream_t st
     return 2 * nseg;
 }
 
-void launch_sgm(const LaunchSet& ls, int mode, int keep_sum, hipStream_t st, const FamStreams* fs, KernelTimer* t)
+void launch_sgm(const LaunchSet& ls, int mode, int keep_sum, hipStream_t st, KernelTimer* t)
 {
-    bool all_fused = true;
-    for (int gi = 0; gi < ls.ngroups; gi++) all_fused = all_fused && ls.groups[gi].vcols > 0;
-    if (all_fused) {
-        // rows family (its two directions as separate waves: 29.7-30.1 ms per
-        // 64-rig step against 31.3-35.3 with both in one wave), then the fused
-        // vertical sweep (which reads part[rows])
-        for (int gi = 0; gi < ls.ngroups; gi++) {
-            const DGroup& G = ls.groups[gi];
-            TB_S(kKRows, st);
-            SISTER_FAM(G, 0, dim3(2 * G.blocks[0]), dim3(64), 0, st, G.rigs, G.nrig, G.bs[0], mode, keep_sum, 1);
-            TD(kKRows, 1);
-            TE_S(kKRows, st);
-            TB_S(kKVSweep, st);
-            const int nl = launch_vsweep(G, mode, keep_sum, st);
-            TD(kKVSweep, nl);
-            TE_S(kKVSweep, st);
-        }
-        return;
-    }
-    // rows on st, columns and diagonals (then the anti-diagonal family's
-    // forward sweep) on the side streams, joined before the anti-diagonal
-    // family's final sweep
-    hipStream_t sc = st, sd = st;
-    if (fs) {
-        (void)hipEventRecord(fs->fork, st);
-        (void)hipStreamWaitEvent(fs->side[0], fs->fork, 0);
-        (void)hipStreamWaitEvent(fs->side[1], fs->fork, 0);
-        sc = fs->side[0];
-        sd = fs->side[1];
-    }
     for (int gi = 0; gi < ls.ngroups; gi++) {
         const DGroup& G = ls.groups[gi];
-        if (G.vcols > 0) continue;
-        TB_S(kKRows, st);
-        SISTER_FAM(G, 0, dim3(2 * G.blocks[0]), dim3(64), 0, st, G.rigs, G.nrig, G.bs[0], mode, keep_sum, 1);
-        TD(kKRows, 1);
-        TE_S(kKRows, st);
-        TB_S(kKCols, sc);
-        SISTER_FAM(G, 1, dim3(G.blocks[1]), dim3(64), 0, sc, G.rigs, G.nrig, G.bs[1], mode, keep_sum, 0);
-        TD(kKCols, 1);
-        TE_S(kKCols, sc);
-        TB_S(kKDiag, sd);
-        SISTER_FAM(G, 2, dim3(G.blocks[2]), dim3(64), 0, sd, G.rigs, G.nrig, G.bs[2], mode, keep_sum, 0);
-        TD(kKDiag, 1);
-        TE_S(kKDiag, sd);
-        // the anti-diagonal family's forward sweep needs M alone: it follows
-        // the diagonals on their stream, beside the rows
-        TB_S(kKAnti, sd);
-        SISTER_FAM(G, 3, dim3(G.blocks[3]), dim3(64), 0, sd, G.rigs, G.nrig, G.bs[3], mode, keep_sum, 1);
-        TD(kKAnti, 1);
-        TE_S(kKAnti, sd);
-    }
-    if (fs) {
-        (void)hipEventRecord(fs->join[0], sc);
-        (void)hipEventRecord(fs->join[1], sd);
-        (void)hipStreamWaitEvent(st, fs->join[0], 0);
-        (void)hipStreamWaitEvent(st, fs->join[1], 0);
-    }
-    for (int gi = 0; gi < ls.ngroups; gi++) {
-        const DGroup& G = ls.groups[gi];
-        if (G.vcols > 0) {
-            TB_S(kKRows, st);
-            SISTER_FAM(G, 0, dim3(2 * G.blocks[0]), dim3(64), 0, st, G.rigs, G.nrig, G.bs[0], mode, keep_sum, 1);
-            TD(kKRows, 1);
-            TE_S(kKRows, st);
-            TB_S(kKVSweep, st);
-            const int nl = launch_vsweep(G, mode, keep_sum, st);
-            TD(kKVSweep, nl);
-            TE_S(kKVSweep, st);
-            continue;
-        }
-        const size_t lds = (size_t)64 * G.CH[3] * 32;
-        TB_S(kKAnti, st);
-        SISTER_FAM(G, 3, dim3(G.blocks[3]), dim3(64), lds, st, G.rigs, G.nrig, G.bs[3], mode, keep_sum, 2);
-        TD(kKAnti, 1);
-        TE_S(kKAnti, st);
+        const bool fused = G.vcols > 0;
+        // every path and then the winner, or the rows family and then the
+        // fused vertical sweep (which reads its bytes)
+        const int k1 = fused ? kKRows : kKPaths, k2 = fused ? kKVSweep : kKWinner;
+        TB(k1);
+        launch_paths(G, keep_sum, st);
+        TD(k1, 1);
+        TE(k1);
+        TB(k2);
+        int nl = 1;
+        if (fused) nl = launch_vsweep(G, mode, keep_sum, st);
+        else launch_winner(G, mode, keep_sum, st);
+        TD(k2, nl);
+        TE(k2);
     }
 }
 

@@ -33,17 +33,18 @@ struct RigDesc {
     uint16_t* med[8];         // in-place-median results of wta[]
     uint8_t* mask[4];         // confidence mask of frame F, padded original coords H' x W'
     uint8_t* msum;            // mask-weighted cost sum M, H' x W' x Dp (u8: M <= 4*63)
-    uint8_t* part[4];         // per chain family (rows, cols, diag, anti): for rows
-                              // 1..H'-2 the two directions' (L - M) summed, in [0,200];
-                              // the rows family keeps its forward (L - M) here and its
-                              // backward one in rowsb.  Ahead of the fused vertical sweep
-                              // only part[0] and rowsb exist (part[1..3] null), and the
-                              // sweep's u16 partial sums P replace their bytes row by row
-    uint8_t* rowsb;           // rows family's backward (L - M), rows 1..H'-2
+    uint8_t* part[8];         // (L - M) bytes, each in [0, 100], of the eight SGM paths:
+                              // [2f] going right or down, [2f+1] left or up, f = rows,
+                              // columns, diagonals, anti-diagonals.  A null [2f+1]: both
+                              // directions summed in [2f].  Cells of the crop, W x H x Dp;
+                              // of the padded frame ahead of the fused vertical sweep
+                              // (which has [0] and [1] alone) and with the debug sums
+    uint16_t* psum;           // fused vertical sweep: partial sums P (null: they replace
+                              // the bytes of part[0] and part[1] row by row)
     uint32_t* vstate;         // fused vertical sweep: segment-end states, normalised
                               // (L - M) bytes and minL': [2][3][W'][Dp + 16] bytes
-    uint16_t* edge;           // exact family contributions on rows 0 and H'-1:
-                              // [family][2][W'][Dp]
+    uint16_t* edge;           // fused vertical sweep, debug sums: exact contributions of
+                              // its three families on rows 0 and H'-1: [3][2][W'][Dp]
     uint16_t* sum;            // SGM aggregate S, H' x W' x Dp (debug only, may be null)
     uint16_t* out[3];         // API maps W x H, min(255*d, 65535) (hpp:111-118); nullable
     uint16_t* disp;           // integer multiview disparity W x H; nullable

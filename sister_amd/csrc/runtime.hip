@@ -41,15 +41,19 @@ struct WsLayout {
 
 inline int padded_depth(int D) { return (D + 15) & ~15; }
 
-// keep_sum adds the debug copy of S.  separate: the per-chain SGM families,
-// five volumes of Dp bytes per pixel (rows forward, columns, diagonals,
-// anti-diagonals forward, rows backward); otherwise the fused vertical sweep,
-// four (the rows family's forward bytes, its partial sums P in two, the rows
-// family's backward bytes) or, in_place (plans short of memory; only for
-// D = 16 KL CH and not in the debug sweep), two: P then replaces the rows
-// bytes row by row.  The serial median's order statistics (prepass form)
-// alias the volumes, which nothing writes before the SGM.  Footprints for
-// admission and sister_workspace_bytes take the default, the largest form.
+// keep_sum adds the debug copy of S.  separate: the SGM paths as separate
+// chains.  Their bytes take the room of five volumes of Dp bytes per padded
+// pixel and of what only the fused sweep needs (edge rows, segment states):
+// as many of the eight paths' volumes over the crop as fit are kept apart
+// (all eight where the crop is at most 5/8 of the frame), and the two
+// directions of the other families share one.  With the debug sums five
+// volumes over the frame.  Otherwise the fused vertical sweep: four (the rows
+// family's two, its partial sums P in two) or, in_place (plans short of
+// memory; only for D = 16 KL CH and not in the debug sweep), two: P then
+// replaces the rows bytes row by row.  The serial median's order statistics
+// (prepass form) alias the volumes, which nothing writes before the SGM.
+// Footprints for admission and sister_workspace_bytes take the default, the
+// largest form.
 WsLayout ws_layout(int W, int H, int D, bool keep_sum = false, bool separate = true, bool in_place = false)
 {
     const size_t Wp = (size_t)W + 2 * D, Hp = (size_t)H + 2 * D;
@@ -67,6 +71,10 @@ WsLayout ws_layout(int W, int H, int D, bool keep_sum = false, bool separate = t
     l.scratch = l.part;
     l.edge = o;    o += align_up(4 * 2 * Wp * padded_depth(D) * sizeof(uint16_t));
     l.vstate = o;  o += align_up(2 * 3 * Wp * (padded_depth(D) + 16));
+    if (separate && !keep_sum) {
+        l.vol = align_up((size_t)W * H * padded_depth(D));
+        l.nvol = std::min<size_t>(8, (o - l.part) / l.vol);
+    }
     l.sum = o;     if (keep_sum) o += align_up(ncell * sizeof(uint16_t));
     l.total = o;
     return l;
@@ -210,8 +218,8 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 // gives the same outputs; only the time differs.
 // ---------------------------------------------------------------------------
 struct GroupForm {
-    int fused = -1;           // -1 automatic, 0 separate chain families, 1 fused vertical sweep
-    int kl[4] = {0, 0, 0, 0}; // lanes per chain of the separate families (0: automatic)
+    int fused = -1;           // -1 automatic, 0 separate chains, 1 fused vertical sweep
+    int kl[4] = {0, 0, 0, 0}; // a field of the forms file; chains always take 16 lanes
     int msum_split = 0;       // 1: the two-launch cost sum
     bool operator==(const GroupForm& o) const
     {
@@ -283,10 +291,12 @@ struct sister_ctx {
     // (parallel branches of the graph): one part's latency-bound stages (the
     // serial median, launch tails) overlap another part's work
     static constexpr int kMaxParts = 8;
+    // a part per disparity count, up to one per hardware queue of the process:
+    // more branches would only share queues
+    static constexpr int kMaxDParts = 4;
     Plan graph_plan[kMaxParts];
     hipStream_t side[kMaxParts] = {};
     hipEvent_t ev_fork = nullptr, ev_join[kMaxParts] = {}, ev_stage[kMaxParts] = {};
-    FamStreams fam[kMaxParts] = {};   // per part: streams for concurrent SGM families
     std::mutex mu;             // guards pool / plans between the serving thread and callers
 
     // serving
@@ -440,24 +450,18 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         p.host_rigs.push_back(g);
     }
     // SGM groups: runs of equal D
-    struct GroupHost { int i0, i1, KL[4], CH[4], vcols, maxHp, msum_split; };
+    struct GroupHost { int i0, i1, vcols, maxHp, msum_split; };
     std::vector<GroupHost> groups;
     for (int k = 0; k < n;) {
         int e = k;
         long chains = 0;
         while (e < n && p.host_rigs[e].D == p.host_rigs[k].D) chains += p.host_rigs[e++].Wp;
-        GroupHost G{k, e, {}, {}, 0, 0, 0};
+        GroupHost G{k, e, 0, 0, 0};
         for (int j = k; j < e; j++) G.maxHp = std::max(G.maxHp, p.host_rigs[j].Hp);
         const int D = p.host_rigs[k].D;
         GroupForm form;
         const auto it = c->gforms.find(GroupKey{D, octave((double)chains), octave((double)G.maxHp)});
         if (it != c->gforms.end()) form = it->second;
-        for (int f = 0; f < 4; f++) {
-            const int kl = form.kl[f];
-            const bool ok = (kl == 8 || kl == 16 || (kl == 4 && D <= 256));
-            G.KL[f] = ok ? kl : sgm_pick_kl(chains, f, D);
-            G.CH[f] = sgm_pick_ch(D, G.KL[f]);
-        }
         // the debug switch wins over a tuned form
         G.vcols = vsweep_pick_cols(chains, D, c->vsweep >= 0 ? c->vsweep : form.fused);
         G.msum_split = form.msum_split;
@@ -484,8 +488,23 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
             for (int q = 0; q < 4; q++) g.mask[q] = (uint8_t*)(b.ptr + l.mask) + q * npx;
             g.msum = (uint8_t*)(b.ptr + l.msum);
             uint8_t* const vols = (uint8_t*)(b.ptr + l.part);
-            for (int q = 0; q < 4; q++) g.part[q] = q < (int)l.nvol - 1 ? vols + q * l.vol : nullptr;
-            g.rowsb = vols + (l.nvol - 1) * l.vol;
+            for (int q = 0; q < 8; q++) g.part[q] = nullptr;
+            g.psum = nullptr;
+            if (G.vcols > 0) {
+                g.part[0] = vols;
+                g.part[1] = vols + l.vol;
+                if (l.nvol == 4) g.psum = (uint16_t*)(vols + 2 * l.vol);
+            } else {
+                // the rows' directions always have a volume each; with fewer
+                // than eight, columns, diagonals and anti-diagonals join theirs
+                // in this order
+                const int joined = 8 - (int)l.nvol;
+                size_t v = 0;
+                for (int f = 0; f < 4; f++) {
+                    g.part[2 * f] = vols + l.vol * v++;
+                    if (f == 0 || f > joined) g.part[2 * f + 1] = vols + l.vol * v++;
+                }
+            }
             g.edge = (uint16_t*)(b.ptr + l.edge);
             g.vstate = (uint32_t*)(b.ptr + l.vstate);
             g.sum = c->keep_sum ? (uint16_t*)(b.ptr + l.sum) : nullptr;
@@ -528,7 +547,8 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
             const RigDesc& g = p.host_rigs[G.i0 + k];
             for (int f = 0; f < kNumGroupKernels; f++) {
                 gbs[gpos + f * (ng + 1) + k] = tot[f];
-                tot[f] += f < 4 ? sgm_family_blocks(g, G.KL[f], f)
+                tot[f] += f == kGPaths ? path_blocks(g, G.vcols > 0 ? 1 : 4, c->keep_sum)
+                        : f == kGWinner ? winner_blocks(g, c->keep_sum)
                         : f == kGVSweep ? vsweep_blocks(g, G.vcols) : msum_blocks(g, f - kGMsumRows);
             }
         }
@@ -564,10 +584,6 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         for (int f = 0; f < kNumGroupKernels; f++) {
             sg.bs[f] = dg + gofs[gi] + f * (ng + 1);
             sg.blocks[f] = gbs[gofs[gi] + f * (ng + 1) + ng];
-        }
-        for (int f = 0; f < 4; f++) {
-            sg.KL[f] = G.KL[f];
-            sg.CH[f] = G.CH[f];
         }
         sg.vcols = G.vcols;
         sg.maxHp = G.maxHp;
@@ -611,8 +627,7 @@ static void free_plan(sister_ctx* c, Plan& p)
 constexpr int kNumPlanStages = 10;
 
 // enqueue stages [from, to) of a plan on `st`
-static void enqueue_range(sister_ctx* c, const Plan& p, int modes, hipStream_t st, const FamStreams* fs,
-                          KernelTimer* t, int from, int to)
+static void enqueue_range(sister_ctx* c, const Plan& p, int modes, hipStream_t st, KernelTimer* t, int from, int to)
 {
     const LaunchSet& ls = p.ls;
     auto in = [&](int k) { return k >= from && k < to; };
@@ -628,14 +643,14 @@ static void enqueue_range(sister_ctx* c, const Plan& p, int modes, hipStream_t s
     for (int m = 0; m < 3; m++) {
         if (!(modes & (1 << m))) continue;
         if (in(4 + 2 * m)) launch_msum(ls, fuse[m], st, t);
-        if (in(5 + 2 * m)) launch_sgm(ls, m, c->keep_sum ? 1 : 0, st, fs, t);
+        if (in(5 + 2 * m)) launch_sgm(ls, m, c->keep_sum ? 1 : 0, st, t);
     }
 }
 
 // enqueue every stage of a plan on `st`
-static void enqueue(sister_ctx* c, const Plan& p, int modes, hipStream_t st, const FamStreams* fs, KernelTimer* t)
+static void enqueue(sister_ctx* c, const Plan& p, int modes, hipStream_t st, KernelTimer* t)
 {
-    enqueue_range(c, p, modes, st, fs, t, 0, kNumPlanStages);
+    enqueue_range(c, p, modes, st, t, 0, kNumPlanStages);
 }
 
 static int check_modes(sister_ctx* c, const sister_rig* rigs, int n, int modes)
@@ -678,13 +693,6 @@ int sister_create(const sister_config* cfg, sister_ctx** out)
              hipEventCreateWithFlags(&c->ev_join[k], hipEventDisableTiming) == hipSuccess;
     for (int k = 0; ok && k < sister_ctx::kMaxParts; k++)
         ok = hipEventCreateWithFlags(&c->ev_stage[k], hipEventDisableTiming) == hipSuccess;
-    for (int k = 0; ok && k < sister_ctx::kMaxParts; k++) {
-        FamStreams& f = c->fam[k];
-        ok = hipEventCreateWithFlags(&f.fork, hipEventDisableTiming) == hipSuccess;
-        for (int j = 0; ok && j < 2; j++)
-            ok = hipStreamCreateWithFlags(&f.side[j], hipStreamNonBlocking) == hipSuccess &&
-                 hipEventCreateWithFlags(&f.join[j], hipEventDisableTiming) == hipSuccess;
-    }
     ok = ok && kernels_setup(c->device) == 0;
     // a failed look-up leaves the allocation-free entry point reporting it
     if (ok) c->scratch = scratch_address(c->device);
@@ -724,13 +732,6 @@ void sister_destroy(sister_ctx* c)
         if (c->ev_join[k]) (void)hipEventDestroy(c->ev_join[k]);
         if (c->side[k]) (void)hipStreamDestroy(c->side[k]);
     }
-    for (auto& f : c->fam) {
-        (void)hipEventDestroy(f.fork);
-        for (int j = 0; j < 2; j++) {
-            (void)hipEventDestroy(f.join[j]);
-            (void)hipStreamDestroy(f.side[j]);
-        }
-    }
     (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -765,8 +766,7 @@ static int run_batch(sister_ctx* c, const sister_rig* rigs, int n, int modes)
     free_plan(c, c->last);
     const int rc = build_plan_compact(c, rigs, n, c->last);
     if (rc) return rc;
-    // profiling times every kernel on its own: the SGM families then run in sequence
-    enqueue(c, c->last, modes, c->stream, c->profiling ? nullptr : &c->fam[0], c->profiling ? &c->timer : nullptr);
+    enqueue(c, c->last, modes, c->stream, c->profiling ? &c->timer : nullptr);
     HIPCHK(c, hipGetLastError());
     return SISTER_OK;
 }
@@ -800,7 +800,7 @@ int sister_run_device_noalloc(sister_ctx* c, const sister_rig* rigs, int n, int 
         rc = build_plan(c, rigs, n, c->noalloc, &carve, true);
     }
     if (rc) return rc;
-    enqueue(c, c->noalloc, modes, c->stream, c->profiling ? nullptr : &c->fam[0], c->profiling ? &c->timer : nullptr);
+    enqueue(c, c->noalloc, modes, c->stream, c->profiling ? &c->timer : nullptr);
     HIPCHK(c, hipGetLastError());
     return SISTER_OK;
 }
@@ -982,7 +982,7 @@ static int partition_batch(sister_ctx* c, const sister_rig* rigs, int n, int mod
         for (int i = 0; i < n; i++) ds.push_back(rigs[i].disp_count);
         std::sort(ds.begin(), ds.end());
         ds.erase(std::unique(ds.begin(), ds.end()), ds.end());
-        if ((int)ds.size() <= sister_ctx::kMaxParts) {
+        if ((int)ds.size() <= sister_ctx::kMaxDParts) {
             for (int i = 0; i < n; i++)
                 part[std::lower_bound(ds.begin(), ds.end(), rigs[i].disp_count) - ds.begin()].push_back(rigs[i]);
             return (int)ds.size();
@@ -1045,22 +1045,19 @@ int sister_graph_capture(sister_ctx* c, const sister_rig* rigs, int n, int modes
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     (void)hipEventRecord(c->ev_fork, c->stream);
     for (int h = 1; h < nparts; h++) (void)hipStreamWaitEvent(c->side[h], c->ev_fork, 0);
-    // the SGM families of a part run in sequence inside a captured graph
-    // (concurrent families are used by eager runs only: a capture that forked
-    // them from the part streams ended in a host-side crash in the runtime)
     auto part_stream = [&](int h) { return h ? c->side[h] : c->stream; };
     if (stagger > 0 && nparts > 1) {
         // part h + 1's first stages wait for part h's: one part's SGM then
         // runs beside the next part's census, WTA and cost sum
         for (int h = 0; h < nparts; h++) {
             if (h) (void)hipStreamWaitEvent(part_stream(h), c->ev_stage[h - 1], 0);
-            enqueue_range(c, c->graph_plan[h], modes, part_stream(h), nullptr, nullptr, 0, stagger);
+            enqueue_range(c, c->graph_plan[h], modes, part_stream(h), nullptr, 0, stagger);
             (void)hipEventRecord(c->ev_stage[h], part_stream(h));
         }
         for (int h = 0; h < nparts; h++)
-            enqueue_range(c, c->graph_plan[h], modes, part_stream(h), nullptr, nullptr, stagger, kNumPlanStages);
+            enqueue_range(c, c->graph_plan[h], modes, part_stream(h), nullptr, stagger, kNumPlanStages);
     } else {
-        for (int h = 0; h < nparts; h++) enqueue(c, c->graph_plan[h], modes, part_stream(h), nullptr, nullptr);
+        for (int h = 0; h < nparts; h++) enqueue(c, c->graph_plan[h], modes, part_stream(h), nullptr);
     }
     for (int h = 1; h < nparts; h++) {
         (void)hipEventRecord(c->ev_join[h], c->side[h]);
@@ -1199,7 +1196,7 @@ int sister_autotune(sister_ctx* c, const sister_rig* rigs, int n, int modes, con
     if (!tuned_batch) {
         std::vector<BatchForm> cand;
         for (int p = 1; p <= std::min(4, n); p++) cand.push_back(BatchForm{p, 0});
-        if (bk.nd >= 2 && bk.nd <= sister_ctx::kMaxParts) cand.push_back(BatchForm{0, 1});
+        if (bk.nd >= 2 && bk.nd <= sister_ctx::kMaxDParts) cand.push_back(BatchForm{0, 1});
         double best = 1e30;
         BatchForm bestf;
         for (const BatchForm& f : cand) {
@@ -1230,7 +1227,7 @@ int sister_autotune(sister_ctx* c, const sister_rig* rigs, int n, int modes, con
         c->bforms[bk] = bestf;
     }
     // 2. each disparity group of those parts: vertical families fused or
-    // separate, lanes per chain, cost-sum form (the other groups keep theirs)
+    // separate, cost-sum form (the other groups keep theirs)
     std::vector<GroupKey> keys;
     {
         std::lock_guard<std::mutex> lk(c->mu);
@@ -1244,15 +1241,11 @@ int sister_autotune(sister_ctx* c, const sister_rig* rigs, int n, int modes, con
         std::vector<GroupForm> cand;
         GroupForm f;
         cand.push_back(f);                                       // automatic
-        f.fused = 0; cand.push_back(f);                          // separate families, automatic lanes
+        f.fused = 0; cand.push_back(f);                          // separate chains
         if (vsweep_pick_cols(1, k.D, 1) > 0) {                   // fused vertical sweep, where it reaches
             f.fused = 1;
             cand.push_back(f);
         }
-        f = GroupForm(); f.fused = 0;
-        for (int q = 0; q < 4; q++) f.kl[q] = 16;
-        cand.push_back(f);                                       // separate, 16 lanes everywhere
-        f.kl[2] = f.kl[3] = 8; cand.push_back(f);                // separate, diagonals on 8
         f = GroupForm(); f.msum_split = 1; cand.push_back(f);    // two-launch cost sum
         double best = 1e30;
         GroupForm bestf;
@@ -1548,7 +1541,7 @@ static void serve_loop(sister_ctx* c)
             } else {
                 fail_reason = "staging allocation failed";
             }
-            if (ok) enqueue(c, f->plan, modes, f->stream, nullptr, nullptr);
+            if (ok) enqueue(c, f->plan, modes, f->stream, nullptr);
         }
         // outputs of host requests back into their pinned staging (copied to
         // the caller's buffers when the batch retires)

@@ -317,3 +317,25 @@ def test_host_form_staging(gpu_ctx, oracle_mod, W, H, modes, seed):
         gpu_ctx._check(sister_amd.lib().sister_compute_rig(gpu_ctx._h, C.byref(r), modes))
         for name, o in outs.items():
             assert np.array_equal(o, ref[name]), name
+
+
+# The path kernel (vertical sweep off): each number of pairs per lane, full
+# and partly filled, cells ending inside and at a lane's end (D = 8 .. 448),
+# and workspaces that hold eight, seven, six and five volumes (joined
+# directions), every map against the oracle.
+@pytest.mark.parametrize("W,H,D,seed", [
+    (300, 200, 8, 101), (420, 300, 24, 102), (400, 300, 40, 103), (72, 56, 64, 104), (36, 28, 104, 105),
+    (100, 60, 128, 106), (128, 40, 144, 107), (40, 24, 152, 108), (32, 24, 192, 109), (24, 20, 208, 110),
+    (20, 16, 272, 111), (24, 16, 288, 112), (16, 12, 336, 113), (16, 8, 448, 114)])
+def test_path_chains_outputs(gpu_ctx, oracle_mod, W, H, D, seed):
+    rig = synth.rig_small(W, H, D, seed)
+    print(f"[parity chains] W={W} H={H} D={D} seed={seed}", flush=True)
+    gpu_ctx.vsweep(0)
+    try:
+        got = gpu_ctx.compute_rig(rig["views"], D, modes=7)
+    finally:
+        gpu_ctx.vsweep(-1)
+    ref = oracle_mod.compute(rig["views"], D, modes=7)
+    for k in ("multiview", "horizontal", "vertical", "disp"):
+        assert np.array_equal(got[k], ref[k]), k
+    assert float(np.abs(got["subpix"] - ref["subpix"]).max()) <= 1e-3
