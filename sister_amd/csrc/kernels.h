@@ -45,7 +45,8 @@ struct LaunchSet {
     int blocks[kNumStages];         // total blocks per stage
     uint64_t* const* scratch;       // per rig: 8 median order-statistic maps
     int maxD;
-    int maxCols;                    // max frame width over the rigs (median LDS)
+    int maxCols;                    // max frame width over the rigs
+    int med_waves;                  // waves per block of k_median
     int maxWp, maxHp;               // max padded width / height over the rigs
     bool wta_rows;                  // WTA by frame rows from shared costs (k_wta_row)
     int ngroups;
@@ -84,6 +85,9 @@ int vsweep_blocks(const RigDesc& g, int vcols);
 int kernels_setup(int device);
 void launch_census(const LaunchSet& ls, hipStream_t st, KernelTimer* t);
 void launch_wta(const LaunchSet& ls, hipStream_t st, KernelTimer* t);
+int median_setup(int lds_limit);
+int median_waves(const RigDesc& g);
+extern int g_num_cu;    // compute units of the device (kernels_setup)
 void launch_median(const LaunchSet& ls, hipStream_t st, KernelTimer* t);
 void launch_mask(const LaunchSet& ls, int fmask, hipStream_t st, KernelTimer* t);
 void launch_msum(const LaunchSet& ls, int fuse, hipStream_t st, KernelTimer* t);

@@ -4,7 +4,7 @@
 //   censusTransform        census.cpp:38-51             k_census
 //   WTALeft/WTARight on    postprocess.cpp:74-315       k_wta   (cost recomputed from
 //     the raw frame DSIs     (hpp:196-197,...)                   census, never stored)
-//   median3x3_SSE in place postprocess.cpp:15-71        k_median_prep + k_median_serial
+//   median3x3_SSE in place postprocess.cpp:15-71        k_median (median.hip)
 //   doLRCheck + mask loops postprocess.cpp:318-341,     k_mask
 //                          hpp:201-251
 //   realign + weighted sum hpp:255-277                  k_msum
@@ -461,296 +461,6 @@ __global__ __launch_bounds__(256) void k_wta_fill(const RigDesc* __restrict__ ri
     uint16_t* const map = g.wta[m];
     const uint2 v = *(const uint2*)(map + (size_t)lo * C + c);
     for (int r = lo + 1; r <= hi; r++) *(uint2*)(map + (size_t)r * C + c) = v;
-}
-
-// ---------------------------------------------------------------------------
-// K3 in-place 3x3 median (postprocess.cpp:15-71 called with source == dest).
-// Over flat index q of a R x C map, processed in increasing q:
-//   out[q] = in[q]                       q < C  or  q >= RC-C-4
-//   out[C] = 0                           (first store is the zero lastMedian)
-//   out[q] = med9(out[q-C-1], out[q-C], out[q-C+1],
-//                 in[q-1],  in[q],  in[q+1],  in[q+C-1], in[q+C], in[q+C+1])
-//                                        C+1 <= q <= RC-C-5
-// The six `in` values of each q are fixed, so a parallel prepass sorts them
-// (s0 <= ... <= s5) and keeps s1..s4.  With the three recursive values sorted
-// (u0 <= u1 <= u2), the 5th smallest of the nine is
-//   min(s4, max(s3, u0), max(s2, u1), max(s1, u2))
-// (k-th smallest of the union of two sorted lists; s0 and s5 can never be the
-// median).  The serial pass is then a few min/max per pixel.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void cswap(unsigned& a, unsigned& b)
-{
-    unsigned lo = min(a, b), hi = max(a, b);
-    a = lo;
-    b = hi;
-}
-
-__global__ __launch_bounds__(256) void k_median_prep(const RigDesc* __restrict__ rigs, int nrig,
-                                                     const int* __restrict__ bs, uint64_t* const* __restrict__ scratch)
-{
-    const int ri = find_rig(bs, nrig, blockIdx.x);
-    const RigDesc& g = rigs[ri];
-    const long npx = (long)g.Wp * g.Hp;
-    const long perMap = (npx + 255) / 256;
-    const long lb = blockIdx.x - bs[ri];
-    const int m = (int)(lb / perMap);
-    const long q = (lb % perMap) * 256 + threadIdx.x;
-    const int F = m >> 1;
-    const long C = frame_cols(g, F);
-    if (q >= npx) return;
-    const uint16_t* in = g.wta[m];
-    uint64_t* out = scratch[ri] + (size_t)m * npx;
-    if (q < C + 1 || q > npx - C - 5) { out[q] = 0; return; }
-    unsigned v0 = in[q - 1], v1 = in[q], v2 = in[q + 1];
-    unsigned v3 = in[q + C - 1], v4 = in[q + C], v5 = in[q + C + 1];
-    // 12-comparator sorting network for six inputs
-    cswap(v0, v5); cswap(v1, v3); cswap(v2, v4);
-    cswap(v1, v2); cswap(v3, v4);
-    cswap(v0, v3); cswap(v2, v5);
-    cswap(v0, v1); cswap(v2, v3); cswap(v4, v5);
-    cswap(v1, v2); cswap(v3, v4);
-    out[q] = (uint64_t)v1 | ((uint64_t)v2 << 16) | ((uint64_t)v3 << 32) | ((uint64_t)v4 << 48);
-}
-
-__device__ __forceinline__ unsigned med9_4(unsigned s1, unsigned s2, unsigned s3, unsigned s4, unsigned a,
-                                           unsigned b, unsigned c)
-{
-    cswap(a, b); cswap(b, c); cswap(a, b);
-    return min(min(s4, max(s3, a)), min(max(s2, b), max(s1, c)));
-}
-
-__device__ __forceinline__ unsigned med9_pre(uint64_t s, unsigned a, unsigned b, unsigned c)
-{
-    return med9_4((unsigned)(s & 0xFFFF), (unsigned)((s >> 16) & 0xFFFF), (unsigned)((s >> 32) & 0xFFFF),
-                  (unsigned)(s >> 48), a, b, c);
-}
-
-// the same from the six fixed values themselves (12-comparator network)
-__device__ __forceinline__ unsigned med9_raw(const uint32_t (&w)[6], unsigned a, unsigned b, unsigned c)
-{
-    unsigned v0 = w[0], v1 = w[1], v2 = w[2], v3 = w[3], v4 = w[4], v5 = w[5];
-    cswap(v0, v5); cswap(v1, v3); cswap(v2, v4);
-    cswap(v1, v2); cswap(v3, v4);
-    cswap(v0, v3); cswap(v2, v5);
-    cswap(v0, v1); cswap(v2, v3); cswap(v4, v5);
-    cswap(v1, v2); cswap(v3, v4);
-    return med9_4(v1, v2, v3, v4, a, b, c);
-}
-
-template <int K, bool RAW> struct MedBuf;
-template <int K> struct MedBuf<K, true> { uint32_t v[K][6]; uint32_t l[6]; };   // six fixed values
-template <int K> struct MedBuf<K, false> { uint64_t v[K]; uint64_t l; };        // their s1..s4
-
-// One block per (rig, map), 1024 threads; rows in sequence, columns in
-// parallel: thread t owns columns t + 1024 k for k < K = ceil(C / 1024), and
-// frame rows are at most kMedMaxK * 1024 wide.  The order statistics of row
-// r + 1 are loaded while row r is computed (two register buffers,
-// alternating), and each result is stored from the register that holds it.
-// LDS keeps two rows of results, each with one slot in front (index -1)
-// holding out(r - 2, C - 1), the raster-order predecessor of column 0 in the
-// window of row r; so every column reads its three upper neighbours alike.
-// The last column reads column 0 of the same row, which thread 0 computes
-// itself, so one barrier per row suffices.  Rows 2 .. R - 3 have none of the
-// special cases (out(1, 0) = 0 and the copied tail from index R*C - C - 4 on)
-// and run without checks.  EXACT: K is the frame's exact slot count, so only
-// slot K - 1 can reach past column C - 2.  PF: load row r + 1 during row r
-// (frames up to 8192 wide); without it the loads of a row precede its
-// compute, which keeps the 16-slot buffer of the widest frames in registers.
-// RAW (frames up to 4096 wide): the six fixed values of each position are
-// loaded a row ahead and sorted in the row's step, so no prepass runs; wider
-// frames read the prepass's order statistics (fewer registers per slot).
-constexpr int kMedMaxK = 16;
-constexpr int kMedRawK = 4;
-// row buffers of the serial median's prefetch ring: the sorting form holds six
-// values per slot (three buffers fit its register budget, four spill), the
-// prepass form one (four fit); frames wider than the sorting form's keep two
-#ifndef SISTER_MED_RING_RAW
-#define SISTER_MED_RING_RAW 3
-#endif
-#ifndef SISTER_MED_RING_PRE
-#define SISTER_MED_RING_PRE 4
-#endif
-template <int K, bool RAW>
-constexpr int med_ring() { return RAW ? SISTER_MED_RING_RAW : K <= kMedRawK ? SISTER_MED_RING_PRE : 2; }
-
-template <int K, bool EXACT, bool PF, bool RAW>
-__device__ __forceinline__ void median_serial_body(int R, int C, const uint16_t* __restrict__ in,
-                                                   uint16_t* __restrict__ out,
-                                                   const uint64_t* __restrict__ pre, uint16_t* lds)
-{
-    const int tid = threadIdx.x;
-    const bool wave0 = __builtin_amdgcn_readfirstlane(tid) < 64;
-    const int qhi = R * C - C - 5;
-    const int kact = (C + 1023) >> 10;
-    uint16_t* prev = lds + 1;
-    uint16_t* cur = lds + C + 2;
-    for (int c = tid; c < C; c += 1024) {
-        const uint16_t v = G(in)[c];
-        prev[c] = v;
-        G(out)[c] = v;
-    }
-    if (tid == 0) prev[-1] = 0;
-    // slot k may hold a column below C - 1 (one that this thread computes)
-    auto live = [&](int k) __attribute__((always_inline)) {
-        return (EXACT && k < K - 1) || tid + 1024 * k < C - 1;
-    };
-    auto col = [&](int k) __attribute__((always_inline)) {
-        return (EXACT && k < K - 1) ? tid + 1024 * k : min(tid + 1024 * k, C - 2);
-    };
-    // Order statistics of row r (1 <= r < R).  Indices past qhi (the copied
-    // tail) are clamped; their statistics are loaded but never used.  Byte
-    // offsets fit 32 bits (R * C * 8 <= 2^31).  The last column's statistics
-    // are needed by thread 0 alone; wave 0 loads them with a lane-dependent
-    // index (lane 0's is the one used) so that the load stays a vector load:
-    // a scalar load would make every LDS wait of the row wait for it too.
-    auto at = [&](int i) __attribute__((always_inline)) {
-        return G((const uint64_t*)((const char*)pre + (uint32_t)i * 8u));
-    };
-    // RAW: in[q-1..q+1] and in[q+C-1..q+C+1] at q clamped to qhi (C <= q:
-    // every index in bounds; the clamped positions' values go unused)
-    auto six = [&](int q, uint32_t (&o)[6]) __attribute__((always_inline)) {
-        const int qq = min(q, qhi);
-        o[0] = G(in)[qq - 1]; o[1] = G(in)[qq]; o[2] = G(in)[qq + 1];
-        o[3] = G(in)[qq + C - 1]; o[4] = G(in)[qq + C]; o[5] = G(in)[qq + C + 1];
-    };
-    auto fetch = [&](int r, MedBuf<K, RAW>& b) __attribute__((always_inline)) {
-        const int base = r * C;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            if (!EXACT && k >= kact) break;
-            if constexpr (RAW) six(base + col(k), b.v[k]);
-            else b.v[k] = *at(min(base + col(k), qhi));
-        }
-        if constexpr (RAW) {
-            if (wave0) six(base + C - 1 + tid, b.l);
-        } else {
-            if (wave0) b.l = *at(min(base + C - 1 + tid, qhi));
-        }
-    };
-    auto med = [&](const MedBuf<K, RAW>& b, int k, unsigned a, unsigned bb, unsigned c) __attribute__((always_inline)) {
-        if constexpr (RAW) return k < 0 ? med9_raw(b.l, a, bb, c) : med9_raw(b.v[k], a, bb, c);
-        else return k < 0 ? med9_pre(b.l, a, bb, c) : med9_pre(b.v[k], a, bb, c);
-    };
-    // In rows 2 .. R - 3 nothing is read from `in`; the other rows wait for
-    // their `in` loads inside their own branch (vmcnt(0), expcnt and lgkmcnt
-    // left free: 0x0F70), so that the plain rows' stores do not wait for the
-    // next row's statistics still in flight.
-    auto row = [&](int r, const MedBuf<K, RAW>& pb) __attribute__((always_inline)) {
-        const int base = r * C;
-        const bool plain = r >= 2 && r <= R - 3;
-        unsigned v[K];
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            if (!EXACT && k >= kact) break;
-            const int c = col(k);
-            v[k] = med(pb, k, prev[c - 1], prev[c], prev[c + 1]);
-        }
-        if (!plain) {
-            // out(1, 0) = 0; from index qhi + 1 on the input is copied
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                if (!EXACT && k >= kact) break;
-                const int q = base + tid + 1024 * k;
-                if (q == C) v[k] = 0;
-                else if (q > qhi && live(k)) v[k] = G(in)[q];
-            }
-            __builtin_amdgcn_s_waitcnt(0x0F70);
-        }
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            if (!EXACT && k >= kact) break;
-            if (live(k)) {
-                const int c = tid + 1024 * k;
-                cur[c] = (uint16_t)v[k];
-                G(out)[base + c] = (uint16_t)v[k];
-            }
-        }
-        if (tid == 0) {
-            // column C - 1 reads column 0 of this row, v[0] of this thread
-            const int q = base + C - 1;
-            unsigned w = med(pb, -1, prev[C - 2], prev[C - 1], v[0]);
-            if (!plain) {
-                if (q > qhi) w = G(in)[q];
-                __builtin_amdgcn_s_waitcnt(0x0F70);
-            }
-            cur[C - 1] = (uint16_t)w;
-            cur[-1] = prev[C - 1];
-            G(out)[q] = (uint16_t)w;
-        }
-        __syncthreads();
-        uint16_t* t = prev; prev = cur; cur = t;
-    };
-    if constexpr (PF) {
-        // a ring of kMedRing buffers: row r's statistics are requested
-        // kMedRing - 1 rows ahead of their use, so that the row chain waits
-        // on load latency only when a row computes faster than that
-        constexpr int NB = med_ring<K, RAW>();
-        MedBuf<K, RAW> buf[NB];
-        static_for<0, NB - 1>([&](auto ic) { fetch(min(1 + decltype(ic)::value, R - 1), buf[decltype(ic)::value]); });
-        __syncthreads();
-        int r = 1;
-        for (; r + NB - 1 < R; r += NB) {
-            static_for<0, NB>([&](auto ic) __attribute__((always_inline)) {
-                constexpr int i = decltype(ic)::value;
-                fetch(min(r + i + NB - 1, R - 1), buf[(i + NB - 1) % NB]);
-                row(r + i, buf[i]);
-            });
-        }
-        // fewer than NB rows remain; all of them are fetched already
-        static_for<0, NB - 1>([&](auto ic) __attribute__((always_inline)) {
-            constexpr int i = decltype(ic)::value;
-            if (r + i < R) row(r + i, buf[i]);
-        });
-    } else {
-        MedBuf<K, RAW> buf;
-        __syncthreads();
-        for (int r = 1; r < R; r++) {
-            fetch(r, buf);
-            row(r, buf);
-        }
-    }
-}
-
-// MODE 0: frames up to kMedRawK * 1024 wide, sorting the six fixed values
-// itself (its blocks of wider frames return at once); MODE 1: the same frames
-// from the prepass; MODE 2: every frame from the prepass, for plans with
-// frames wider than that (all maps at once: a rig's wide and narrow frames
-// take the same time, so they run side by side).
-// Blocks are dispatched long maps first: block b takes map slot b / nrig of rig
-// b % nrig, slots 0-3 being the rig's four maps of the frames with more rows
-// (the serial chain is one row per step) and slots 4-7 the other four.  When
-// the blocks take more than one round of the CUs, the short maps then fill
-// the CUs the long ones leave, instead of long maps starting last.
-template <int MODE>
-__global__ __launch_bounds__(1024) void k_median_serial(const RigDesc* __restrict__ rigs, int nrig,
-                                                        uint64_t* const* __restrict__ scratch)
-{
-    extern __shared__ uint16_t lds16[];
-    const int ri = blockIdx.x % nrig, slot = blockIdx.x / nrig;
-    const RigDesc& g = rigs[ri];
-    // frames 1/3 have W' rows, frames 0/2 H' rows; map m = 2 F + side
-    const int long_odd = g.Wp > g.Hp ? 1 : 0;
-    const int fr = (slot >> 1) & 1, side = slot & 1;             // frame pair index, side
-    const int F = ((slot < 4) == (long_odd == 1)) ? 2 * fr + 1 : 2 * fr;
-    const int m = 2 * F + side;
-    const int R = frame_rows(g, F), C = frame_cols(g, F);
-    const uint16_t* in = g.wta[m];
-    uint16_t* out = g.med[m];
-    const uint64_t* pre = scratch[ri] + (size_t)m * R * C;
-    const int k = (C + 1023) >> 10;
-    if (MODE < 2 && k > kMedRawK) return;
-    constexpr bool RAW = MODE == 0;
-    if (k <= kMedRawK) {
-        switch (k) {
-        case 1: median_serial_body<1, true, true, RAW>(R, C, in, out, pre, lds16); break;
-        case 2: median_serial_body<2, true, true, RAW>(R, C, in, out, pre, lds16); break;
-        case 3: median_serial_body<3, true, true, RAW>(R, C, in, out, pre, lds16); break;
-        default: median_serial_body<4, true, true, RAW>(R, C, in, out, pre, lds16); break;
-        }
-    } else if constexpr (MODE == 2) {
-        if (k <= 8) median_serial_body<8, false, true, false>(R, C, in, out, pre, lds16);
-        else median_serial_body<kMedMaxK, false, false, false>(R, C, in, out, pre, lds16);
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1870,32 +1580,7 @@ void launch_wta(const LaunchSet& ls, hipStream_t st, KernelTimer* t)
 }
 
 static size_t g_lds_per_block = 0;   // set by kernels_setup
-static int g_num_cu = 0;
-
-void launch_median(const LaunchSet& ls, hipStream_t st, KernelTimer* t)
-{
-    // With enough (rig, map) blocks to spread over the chip the serial kernel
-    // sorts each position's six fixed values itself (no prepass pass over
-    // memory); with few, each block's row chain is the critical path and the
-    // parallel prepass takes the sorting off it.  Plans with frames wider
-    // than the raw form takes run every map from the prepass in one launch.
-    const size_t lds = (size_t)2 * (ls.maxCols + 1) * sizeof(uint16_t);
-    const bool wide = ls.maxCols > 1024 * kMedRawK;
-    const bool raw = !wide && ls.nrig * 8 >= std::max(g_num_cu / 4, 1);
-    if (!raw) {
-        TB(kKMedianPrep);
-        hipLaunchKernelGGL(k_median_prep, dim3(ls.blocks[kStageMedianPrep]), dim3(256), 0, st, ls.rigs, ls.nrig,
-                           ls.bs[kStageMedianPrep], ls.scratch);
-        TD(kKMedianPrep, 1);
-        TE(kKMedianPrep);
-    }
-    TB(kKMedianSerial);
-    if (raw) hipLaunchKernelGGL(k_median_serial<0>, dim3(ls.nrig * 8), dim3(1024), lds, st, ls.rigs, ls.nrig, ls.scratch);
-    else if (wide) hipLaunchKernelGGL(k_median_serial<2>, dim3(ls.nrig * 8), dim3(1024), lds, st, ls.rigs, ls.nrig, ls.scratch);
-    else hipLaunchKernelGGL(k_median_serial<1>, dim3(ls.nrig * 8), dim3(1024), lds, st, ls.rigs, ls.nrig, ls.scratch);
-    TD(kKMedianSerial, 1);
-    TE(kKMedianSerial);
-}
+int g_num_cu = 0;
 
 void launch_mask(const LaunchSet& ls, int fmask, hipStream_t st, KernelTimer* t)
 {
@@ -1935,6 +1620,10 @@ int kernels_setup(int device)
             return 0;
         }
     g_lds_per_block = (size_t)lim;
+    if (median_setup(lim) != 0) {
+        (void)hipGetLastError();
+        return -1;
+    }
 #define SISTER_VS_FNS(K, F)                                                         \
     (const void*)k_vsweep<1, 0, K, F, 4>, (const void*)k_vsweep<2, 0, K, F, 4>,     \
         (const void*)k_vsweep<3, 0, K, F, 4>, (const void*)k_vsweep<1, 1, K, F, 4>, \
@@ -2169,7 +1858,7 @@ void stage_blocks(const RigDesc& g, int maxD, bool wta_rows, int out[kNumStages]
         out[kStageWtaV] = 0;
     }
     out[kStageWtaFill] = 8 * 2 * ((std::max(g.Wp, g.Hp) + kWtaFillCols - 1) / kWtaFillCols);
-    out[kStageMedianPrep] = (int)(8 * ((npx + 255) / 256));
+    out[kStageMedianPrep] = (int)(8 * ((npx / 2 + 255) / 256));
     out[kStageMask] = 4 * ((g.Wp + kMT32 - 1) / kMT32) * ((g.Hp + kMT32 - 1) / kMT32);
 }
 

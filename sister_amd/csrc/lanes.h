@@ -21,6 +21,44 @@ __device__ __forceinline__ uint4 LD16(const void* p)
 }
 __device__ __forceinline__ void ST16(void* p, uint4 v) { *(gptr<u32x4>)p = u32x4{v.x, v.y, v.z, v.w}; }
 
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
+template <int N> struct Vec;
+template <> struct Vec<1> { typedef uint32_t T; };
+template <> struct Vec<2> { typedef u32x2 T; };
+template <> struct Vec<3> { typedef u32x3 T; };
+template <> struct Vec<4> { typedef u32x4 T; };
+
+
+// Raw buffers: a base and a size in bytes; an access of N dwords at a lane
+// offset past the size reads 0 and stores nothing, so a lane that has nothing
+// to move takes kDropped instead of a branch.
+constexpr uint32_t kDropped = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf(uint8_t* base, uint32_t bytes = 0x7FFFFFFFu)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, 0x00020000);
+}
+template <int N> __device__ __forceinline__ void buf_store(const uint32_t* w, __amdgpu_buffer_rsrc_t r, uint32_t off)
+{
+    if constexpr (N == 1) __builtin_amdgcn_raw_buffer_store_b32(w[0], r, off, 0, 0);
+    else if constexpr (N == 2) __builtin_amdgcn_raw_buffer_store_b64(u32x2{w[0], w[1]}, r, off, 0, 0);
+    else if constexpr (N == 3) __builtin_amdgcn_raw_buffer_store_b96(u32x3{w[0], w[1], w[2]}, r, off, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b128(u32x4{w[0], w[1], w[2], w[3]}, r, off, 0, 0);
+}
+template <int N> __device__ __forceinline__ void buf_load(uint32_t* w, __amdgpu_buffer_rsrc_t r, uint32_t off)
+{
+    if constexpr (N == 1) {
+        w[0] = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+    } else {
+        typename Vec<N>::T v;
+        if constexpr (N == 2) v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+        else if constexpr (N == 3) v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
+        else v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+#pragma unroll
+        for (int i = 0; i < N; i++) w[i] = v[i];
+    }
+}
+
 // Block index b of an n-block grid taken in XCD-contiguous order: with
 // round-robin dispatch block b runs on XCD b % 8, so the XCD gets the
 // consecutive logical blocks [start(b % 8), start(b % 8 + 1)) (the first
@@ -59,6 +97,26 @@ constexpr uint32_t kGuard2 = 0x3FFF3FFFu;
 __device__ __forceinline__ us2 U2(uint32_t v) { return __builtin_bit_cast(us2, v); }
 __device__ __forceinline__ uint32_t W2(us2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ us2 umin2(us2 a, us2 b) { return __builtin_elementwise_min(a, b); }
+__device__ __forceinline__ us2 umax2(us2 a, us2 b) { return __builtin_elementwise_max(a, b); }
+// minimum and maximum of three pairs in one instruction.  gfx950 has packed
+// three-input forms for halves only; non-negative halves order like their bit
+// patterns, and finite ones (patterns below 0x7C00) pass through unchanged,
+// denormals included (f16 denormals are on by default): exact for integers
+// below 0x7C00.
+__device__ __forceinline__ us2 umin3(us2 a, us2 b, us2 c)
+{
+    uint32_t r;
+    asm("v_pk_minimum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(__builtin_bit_cast(uint32_t, a)),
+        "v"(__builtin_bit_cast(uint32_t, b)), "v"(__builtin_bit_cast(uint32_t, c)));
+    return __builtin_bit_cast(us2, r);
+}
+__device__ __forceinline__ us2 umax3(us2 a, us2 b, us2 c)
+{
+    uint32_t r;
+    asm("v_pk_maximum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(__builtin_bit_cast(uint32_t, a)),
+        "v"(__builtin_bit_cast(uint32_t, b)), "v"(__builtin_bit_cast(uint32_t, c)));
+    return __builtin_bit_cast(us2, r);
+}
 // bytes b0,b1 of w -> pair (b0, b1); bytes b2,b3 -> pair (b2, b3)
 __device__ __forceinline__ uint32_t bytes01(uint32_t w) { return __builtin_amdgcn_perm(w, w, 0x0c010c00u); }
 __device__ __forceinline__ uint32_t bytes23(uint32_t w) { return __builtin_amdgcn_perm(w, w, 0x0c030c02u); }
@@ -95,6 +153,15 @@ __device__ __forceinline__ uint32_t row_shr1(uint32_t v)
 __device__ __forceinline__ uint32_t row_shl1(uint32_t v)
 {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x101, 0xF, 0xF, true);
+}
+// the same over the wave's 64 lanes
+__device__ __forceinline__ uint32_t wave_from_left(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xF, 0xF, true);
+}
+__device__ __forceinline__ uint32_t wave_from_right(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xF, 0xF, true);
 }
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_min(uint32_t v)

@@ -25,12 +25,8 @@
 
 namespace sister {
 
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
-
 constexpr int kPathLanes = 16;              // lanes per chain: one DPP row
 constexpr int kPathChains = 64 / kPathLanes;   // chains per wave
-constexpr uint32_t kDropped = 0x80000000u;  // buffer offset out of range: loads give 0, stores nothing
 
 // 2 NP bytes of a lane (NP pairs, 2 NP disparities) as one or two vector
 // accesses: NW dwords, the first W0 = min(NW, 4) of them in the first
@@ -38,12 +34,6 @@ template <int NP> struct Span {
     static constexpr int NW = NP / 2, W0 = NW < 4 ? NW : 4, W1 = NW - W0;
     uint32_t w[NW];
 };
-template <int N> struct Vec;
-template <> struct Vec<1> { typedef uint32_t T; };
-template <> struct Vec<2> { typedef u32x2 T; };
-template <> struct Vec<3> { typedef u32x3 T; };
-template <> struct Vec<4> { typedef u32x4 T; };
-
 // N dwords at a uniform base plus a 32-bit lane offset
 template <int N> __device__ __forceinline__ void load_dw(const uint8_t* base, uint32_t off, uint32_t* w)
 {
@@ -55,31 +45,6 @@ template <int N> __device__ __forceinline__ void load_dw(const uint8_t* base, ui
 #pragma unroll
         for (int i = 0; i < N; i++) w[i] = v[i];
 }
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf(uint8_t* base)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7FFFFFFF, 0x00020000);
-}
-template <int N> __device__ __forceinline__ void buf_store(const uint32_t* w, __amdgpu_buffer_rsrc_t r, uint32_t off)
-{
-    if constexpr (N == 1) __builtin_amdgcn_raw_buffer_store_b32(w[0], r, off, 0, 0);
-    else if constexpr (N == 2) __builtin_amdgcn_raw_buffer_store_b64(u32x2{w[0], w[1]}, r, off, 0, 0);
-    else if constexpr (N == 3) __builtin_amdgcn_raw_buffer_store_b96(u32x3{w[0], w[1], w[2]}, r, off, 0, 0);
-    else __builtin_amdgcn_raw_buffer_store_b128(u32x4{w[0], w[1], w[2], w[3]}, r, off, 0, 0);
-}
-template <int N> __device__ __forceinline__ void buf_load(uint32_t* w, __amdgpu_buffer_rsrc_t r, uint32_t off)
-{
-    if constexpr (N == 1) {
-        w[0] = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
-    } else {
-        typename Vec<N>::T v;
-        if constexpr (N == 2) v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
-        else if constexpr (N == 3) v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
-        else v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-#pragma unroll
-        for (int i = 0; i < N; i++) w[i] = v[i];
-    }
-}
-
 // uniform 64-bit value of lane l
 __device__ __forceinline__ long lane64(long v, int l)
 {

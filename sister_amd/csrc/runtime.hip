@@ -567,9 +567,11 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
     p.ls.wta_rows = wta_rows;
     p.ls.maxWp = 8;
     p.ls.maxHp = 8;
+    p.ls.med_waves = 0;
     for (const RigDesc& g : p.host_rigs) {
         p.ls.maxWp = std::max(p.ls.maxWp, g.Wp);
         p.ls.maxHp = std::max(p.ls.maxHp, g.Hp);
+        p.ls.med_waves = std::max(p.ls.med_waves, median_waves(g));
     }
     p.ls.ngroups = (int)groups.size();
     const int* dg = (const int*)(p.table.ptr + rig_bytes + scr_bytes + bs_bytes);

@@ -390,3 +390,26 @@ def test_serving_caller_errors_while_serving():
         ctx.serve_stop()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("W", [208, 212, 880, 884, 1904, 1908, 2864, 2868, 3824, 3828, 5744, 5748, 9904, 9908])
+def test_median_strips_match_oracle(gpu_ctx, oracle_mod, W):
+    """The serial median at both sides of every change of its strips (frames of
+    W + 16 columns and of W + 16 rows: one wave exactly filled, up to four and
+    eight waves of each width, the widest form), from the prepass (one rig) and
+    sorting by itself (eight rigs); 28 rows a frame: a whole segment and rows
+    left over."""
+    import torch
+    H, D = 12, 8
+    rig = synth.rig_scene(W, H, D, 700 + W, n_boxes=2, blur_sigma=0.7, box_side=(4, 10))
+    ref = oracle_mod.compute(rig["views"], D, modes=1, debug=True)
+    shapes = [(H + 16, W + 16), (W + 16, H + 16)] * 2
+    dev = [_device_rig(gpu_ctx, rig, torch) for _ in range(8)]
+    for n in (1, 8):
+        print(f"[median] W={W} rigs={n}", flush=True)
+        gpu_ctx.run_device([d["struct"] for d in dev[:n]], sister_amd.MODE_MULTIVIEW)
+        gpu_ctx.sync()
+        for F in range(4):
+            for side in range(2):
+                g = gpu_ctx.fetch(n - 1, "med", 2 * F + side, shapes[F], np.uint16)
+                assert np.array_equal(g, ref["med_r" if side else "med_l"][F].astype(np.uint16)), (n, F, side)
