@@ -911,7 +911,7 @@ __device__ __forceinline__ void lane_step(LaneState<CH>& st, const ChainGeo& cg,
     const uint32_t rfill = (cg.lid == KL - 1) ? kGuard2 : nbr;
     const uint32_t mpp = dup16(st.mp);
     const us2 p2t = U2(mpp) + (us2){(unsigned short)kP2, (unsigned short)kP2};
-    us2 rmin = U2(0xFFFFFFFFu);
+    us2 rmin;
     static_for<0, CH>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         const int qg = cg.lid * CH + q;
@@ -932,12 +932,12 @@ __device__ __forceinline__ void lane_step(LaneState<CH>& st, const ChainGeo& cg,
             const us2 left = U2(__builtin_amdgcn_alignbit(cur, prv, 16));
             const us2 right = U2(__builtin_amdgcn_alignbit(nxt, cur, 16));
             const us2 nb = umin2(left, right) + (us2){(unsigned short)kP1, (unsigned short)kP1};
-            const us2 t = umin2(umin2(nb, U2(cur)), p2t);
+            const us2 t = umin3(nb, U2(cur), p2t);   // below 0x7C00: at most the guard + 255 + P2
             const us2 d = DEFER ? t : t - U2(mpp);
             const us2 l = U2(W2(d + U2(m)) | (i < 4 ? pad_lo : pad_hi));
+            if (i & 1) rmin = j == 1 ? umin2(U2(st.L[0]), l) : umin3(rmin, U2(st.L[j - 1]), l);
             st.L[j] = W2(l);
             prv = cur;
-            rmin = umin2(rmin, l);
         }
     });
     st.mp = group_min<KL>(min((uint32_t)rmin.x, (uint32_t)rmin.y));

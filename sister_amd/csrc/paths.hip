@@ -151,13 +151,13 @@ __device__ __forceinline__ void path_sweep(PathLane<NP>& st, const uint8_t* mb, 
         a[NP] = __builtin_amdgcn_alignbit(from_right(st.L[0]), st.L[NP - 1], 16);
 #pragma unroll
         for (int j = 1; j < NP; j++) a[j] = __builtin_amdgcn_alignbit(st.L[j], st.L[j - 1], 16);
-        us2 rmin = U2(0xFFFFFFFFu);
+        us2 rmin;
         uint32_t d[NP];
 #pragma unroll
         for (int j = 0; j < NP; j++) {
             const uint32_t m = (j & 1) ? bytes23(b.w[j / 2]) : bytes01(b.w[j / 2]);
             const us2 nb = umin2(U2(a[j]), U2(a[j + 1])) + (us2){(unsigned short)kP1, (unsigned short)kP1};
-            const us2 v = umin2(umin2(nb, U2(st.L[j])), p2t) - U2(mpp);
+            const us2 v = umin3(nb, U2(st.L[j]), p2t) - U2(mpp);
             uint32_t l = W2(v + U2(m));
             if constexpr (KEEP) l &= tmask;          // first line of a pass: 8-bit path
             // every value is below 0x4000 (at most P2 + 255, or the guard), so
@@ -165,7 +165,7 @@ __device__ __forceinline__ void path_sweep(PathLane<NP>& st, const uint8_t* mb, 
             if constexpr (!FULL) l |= st.pad[j];
             d[j] = W2(v);
             st.L[j] = l;
-            rmin = umin2(rmin, U2(l));
+            if (j & 1) rmin = j == 1 ? umin2(U2(st.L[0]), U2(l)) : umin3(rmin, U2(st.L[j - 1]), U2(l));   // NP is even
         }
         st.mp = group_min<kPathLanes>(min((uint32_t)rmin.x, (uint32_t)rmin.y));
         if constexpr (decltype(store)::value) {
