@@ -1093,8 +1093,12 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
     const RigDesc& g = rigs[ri];
     const int Wp = g.Wp, Hp = g.Hp, D = g.D, Dp = g.Dp;
     const int t0 = seg * kVGhost;
-    if (t0 >= Hp) return;                          // the rig has no such segment: whole block
-    const int nrows = min(kVGhost, Hp - t0);
+    // a pass ends with its last crop row: the D rows beyond it reach no S (the
+    // debug sums cover every row).  1920x1080 D=192: 1272 of 1464 rows, 160
+    // launches of 184, 64 rigs 68.3 -> 61.7 ms
+    const int tend = KEEP ? Hp : Hp - D;
+    if (t0 >= tend) return;                        // the rig has no such segment: whole block
+    const int nrows = min(kVGhost, tend - t0);
     (void)ncol;                                    // VC (compile-time LDS strides)
     constexpr int nt = VC + 2 * kVGhost;
     const int tid = threadIdx.x, c = tid / KL;
@@ -1523,7 +1527,7 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
         }
     }
     // states at the end of the segment, for the next launch
-    if (t0 + nrows < Hp && own && act) {
+    if (t0 + nrows < tend && own && act) {
         const int pout = seg & 1;
         uint4 mr[CH];
         load_m(t0 + nrows - 1, mr);
@@ -1765,7 +1769,7 @@ static int launch_vsweep(const DGroup& G, int mode, int keep_sum, hipStream_t st
     const size_t lds = vs_lds(G.D, G.vcols);
     const dim3 grid(G.blocks[kGVSweep]), block(kl * nt);
     const int* bs = G.bs[kGVSweep];
-    const int nseg = (G.maxHp + kVGhost - 1) / kVGhost;
+    const int nseg = (G.maxHp - (keep_sum ? 0 : G.D) + kVGhost - 1) / kVGhost;
     // 1..3 chunks with 4 lanes per column, 2..3 with 8 (vsweep_pick_cols
     // gives no columns beyond)
     const int ch = vs_ch(G.D);
