@@ -538,8 +538,8 @@ __global__ __launch_bounds__(256) void k_mask(const RigDesc* __restrict__ rigs, 
 // block = a run of one column) adds to it.  Each block stages the partner
 // window of its run (kRun + D - 1 codes per frame) in LDS once.  A wave takes
 // one pixel at a time, lane q the disparities q + 64 j: conflict-free 8-byte
-// LDS reads at immediate offsets and coalesced 64-byte stores per group, with
-// no per-disparity branches.  Cell stride Dp, zero past D.
+// LDS reads at immediate offsets, with no per-disparity branches, and stores
+// four pixels together (quad_bytes).  Cell stride Dp, zero past D.
 // ---------------------------------------------------------------------------
 constexpr int kRun = 256;   // pixels per block
 constexpr int kWinPad = 8;  // window entries before each partner window
@@ -561,6 +561,23 @@ __device__ __forceinline__ void msum_add_frame(const uint64_t* L, uint64_t cc, i
         const uint64_t x = cc ^ tv[j];
         acc[j] = bcnt_add((uint32_t)(x >> 32), bcnt_add((uint32_t)x, acc[j]));
     }
+}
+
+// Stores of M.  A wave's lane q holds one disparity of a pixel, so one pixel's
+// bytes would leave as byte stores (16 or more address cycles for 64 bytes).
+// Four pixels go together instead: a lane packs its disparity's four sums and
+// a 4 x 4 byte transpose over each four lanes (two DPP exchanges, two byte
+// permutes) leaves lane l the disparities (l & ~3) .. + 3 of pixel l & 3, one
+// dword store for four pixels.  Two-launch form: pair modes of eight 1000x620
+// D=136 rigs 1.56 -> 1.28 ms, 4096x3000 D=384 6.2 -> 5.7 ms; tiled form
+// 640x480 D=64 53 -> 48 us, 64 rigs 1920x1080 D=192 34.0 -> 33.0 ms.
+__device__ __forceinline__ uint32_t quad_bytes(const unsigned (&a)[4], int lane)
+{
+    const uint32_t own = a[0] | (a[1] << 8) | (a[2] << 16) | (a[3] << 24);
+    const uint32_t n1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)own, 0xB1, 0xF, 0xF, true);   // lane ^ 1
+    const uint32_t h = __builtin_amdgcn_perm(n1, own, (lane & 1) ? 0x03070105u : 0x06020400u);
+    const uint32_t n2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0x4E, 0xF, 0xF, true);     // lane ^ 2
+    return __builtin_amdgcn_perm(n2, h, (lane & 2) ? 0x03020706u : 0x05040100u);
 }
 
 // SIDE = 0: frames 0/180 along row y; SIDE = 1: frames 90/270 along column x.
@@ -629,33 +646,46 @@ __global__ __launch_bounds__(256) void k_msum_run(const RigDesc* __restrict__ ri
         LM[i] = mb;
     }
     __syncthreads();
-    // one wave per pixel; lane q owns d = q + 64 j.  In the last group, lanes
-    // at or past Dp read as lane Dp - 1 - 64 (J - 1) (and store nothing),
-    // lanes at or past D add nothing.
+    // one wave per pixel, four pixels of the run at a time (the line's length is
+    // a multiple of 4); lane q owns d = q + 64 j.  In the last group, lanes at
+    // or past Dp read as lane Dp - 1 - 64 (J - 1) (and store nothing), lanes at
+    // or past D add nothing.
     const int wave = tid >> 6, q = tid & 63;
     const int qlast = min(q, Dp - 1 - 64 * (J - 1));
-    const bool store_last = q + 64 * (J - 1) < Dp;
+    const bool store_last = (q & ~3) + 64 * (J - 1) < Dp;
     const bool live_last = q + 64 * (J - 1) < D;
-    uint8_t* const msum = g.msum;
-    for (int i = wave; i < kRun; i += 4) {
+    const size_t pstep = (size_t)(SIDE == 0 ? 1 : Wp) * Dp;     // to the line's next pixel
+    for (int i = 4 * wave; i < kRun; i += 16) {
         const int pos = p0 + i;
         if (pos >= len) break;
         const int y = SIDE == 0 ? line : pos, x = SIDE == 0 ? pos : line;
-        gptr<uint8_t> o = G(msum) + ((size_t)y * Wp + x) * Dp;
-        unsigned acc[J];
-#pragma unroll
-        for (int j = 0; j < J; j++) acc[j] = 0;
+        gptr<uint32_t> o = (gptr<uint32_t>)(G(g.msum) + ((size_t)y * Wp + x) * Dp + (q & 3) * pstep + (q & ~3));
+        uint32_t old[J];
         if (SIDE == 1 && (fuse & 5)) {
 #pragma unroll
-            for (int j = 0; j < J - 1; j++) acc[j] = o[q + 64 * j];
-            if (store_last) acc[J - 1] = o[q + 64 * (J - 1)];
+            for (int j = 0; j < J; j++)
+                if (j < J - 1 || store_last) old[j] = o[16 * j];
         }
-        const int mb = __builtin_amdgcn_readfirstlane(LM[i]);   // one pixel per wave
-        if (mb & 1) msum_add_frame<J>(LA, LCa[i], (SIDE == 0 ? pos : Hp - 1 - pos) - loA, q, qlast, acc);
-        if (mb & 2) msum_add_frame<J>(LB, LCb[i], (SIDE == 0 ? Wp - 1 - pos : pos) - loB, q, qlast, acc);
+        unsigned acc[J][4];
+        static_for<0, 4>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int k = decltype(kc)::value;
+            unsigned a[J];
 #pragma unroll
-        for (int j = 0; j < J - 1; j++) o[q + 64 * j] = (uint8_t)acc[j];
-        if (store_last) o[q + 64 * (J - 1)] = live_last ? (uint8_t)acc[J - 1] : (uint8_t)0;
+            for (int j = 0; j < J; j++) a[j] = 0;
+            const int mb = __builtin_amdgcn_readfirstlane(LM[i + k]);   // one pixel per wave
+            const int pk = pos + k;
+            if (mb & 1) msum_add_frame<J>(LA, LCa[i + k], (SIDE == 0 ? pk : Hp - 1 - pk) - loA, q, qlast, a);
+            if (mb & 2) msum_add_frame<J>(LB, LCb[i + k], (SIDE == 0 ? Wp - 1 - pk : pk) - loB, q, qlast, a);
+            a[J - 1] = live_last ? a[J - 1] : 0u;
+#pragma unroll
+            for (int j = 0; j < J; j++) acc[j][k] = a[j];
+        });
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            uint32_t w = quad_bytes(acc[j], q);
+            if (SIDE == 1 && (fuse & 5)) w += old[j];   // bytes <= 126 each
+            if (j < J - 1 || store_last) o[16 * j] = w;
+        }
     }
 }
 
@@ -673,9 +703,6 @@ __global__ __launch_bounds__(256) void k_msum_run(const RigDesc* __restrict__ ri
 // Per pixel as above: one wave per pixel, lane q owns d = q + 64 j.
 // ---------------------------------------------------------------------------
 constexpr int kMT = 16;
-#ifndef SISTER_MSUM_HOIST
-#define SISTER_MSUM_HOIST 0
-#endif
 
 // window line stride (entries) for J groups of 64 disparities: holds
 // kWinPad + kMT + D - 1 <= 64 J + 23 entries; a compile-time constant, so a
@@ -785,7 +812,7 @@ __global__ __launch_bounds__(1024) void k_msum_tile(const RigDesc* __restrict__ 
     };
     const int q = lane;
     const int qlast = min(q, Dp - 1 - 64 * (J - 1));
-    const bool store_last = q + 64 * (J - 1) < Dp;
+    const bool store_last = (q & ~3) + 64 * (J - 1) < Dp;
     const bool live_last = q + 64 * (J - 1) < D;
     // wave w walks tile column w, its 16 pixels fully unrolled: every read
     // sits at a compile-time offset from one lane address per frame, so no
@@ -807,58 +834,43 @@ __global__ __launch_bounds__(1024) void k_msum_tile(const RigDesc* __restrict__ 
         const uint64_t* pl[4] = {win(0, 0) + tx + lo - qlast, win(1, tx) + lo - qlast,
                                  win(2, 0) + (kMT - 1 - tx) + lo - qlast, win(3, tx) + lo - qlast};
         const uint64_t* pc0 = CEN + tx;
-        gptr<uint8_t> o = G(g.msum) + ((size_t)gq.y0 * Wp + x) * Dp;
         const size_t rstride = (size_t)Wp * Dp;
-        static_for<0, kMT>([&](auto tyc) __attribute__((always_inline)) {
-            constexpr int ty = decltype(tyc)::value;
-            if (gq.y0 + ty >= Hp) return;
-            unsigned acc[J];
+        gptr<uint8_t> o = G(g.msum) + ((size_t)gq.y0 * Wp + x) * Dp + (q & 3) * rstride + (q & ~3);
+        static_for<0, kMT / 4>([&](auto gc) __attribute__((always_inline)) {
+            constexpr int ty0 = 4 * decltype(gc)::value;
+            if (gq.y0 + ty0 >= Hp) return;                        // H' is a multiple of 4
+            unsigned acc[J][4];
+            static_for<0, 4>([&](auto tyc) __attribute__((always_inline)) {
+                constexpr int k = decltype(tyc)::value, ty = ty0 + k;
+                unsigned a[J];
 #pragma unroll
-            for (int j = 0; j < J; j++) acc[j] = 0;
-            const int mb = __builtin_amdgcn_readlane(mcol, ty);   // one pixel per wave
-#if SISTER_MSUM_HOIST
-            // every frame's window and centre reads are issued before any
-            // frame's (mask-dependent) sum, so one LDS latency covers the
-            // pixel instead of one per frame
-            uint64_t tv[4][J], cc[4];
-            static_for<0, 4>([&](auto kc) __attribute__((always_inline)) {
-                constexpr int F = decltype(kc)::value;
-                constexpr int off = F == 0 || F == 2 ? ty * LSTR : F == 1 ? kMT - 1 - ty : ty;
+                for (int j = 0; j < J; j++) a[j] = 0;
+                const int mb = __builtin_amdgcn_readlane(mcol, ty);   // one pixel per wave
+                static_for<0, 4>([&](auto kc) __attribute__((always_inline)) {
+                    constexpr int F = (0x3120 >> (4 * decltype(kc)::value)) & 15;   // frames 0, 2, 1, 3
+                    constexpr int off = F == 0 || F == 2 ? ty * LSTR : F == 1 ? kMT - 1 - ty : ty;
+                    if (!(mb & (1 << F))) return;
+                    uint64_t tv[J];
 #pragma unroll
-                for (int j = 0; j < J - 1; j++) tv[F][j] = pa[F][off + 64 * (J - 1 - j)];
-                tv[F][J - 1] = pl[F][off];
-                cc[F] = pc0[F * kMT * kMT + ty * kMT];
+                    for (int j = 0; j < J - 1; j++) tv[j] = pa[F][off + 64 * (J - 1 - j)];
+                    tv[J - 1] = pl[F][off];
+                    const uint64_t cc = pc0[F * kMT * kMT + ty * kMT];
+#pragma unroll
+                    for (int j = 0; j < J; j++) {
+                        const uint64_t xv = cc ^ tv[j];
+                        a[j] = bcnt_add((uint32_t)(xv >> 32), bcnt_add((uint32_t)xv, a[j]));
+                    }
+                });
+                a[J - 1] = live_last ? a[J - 1] : 0u;
+#pragma unroll
+                for (int j = 0; j < J; j++) acc[j][k] = a[j];
             });
-            static_for<0, 4>([&](auto kc) __attribute__((always_inline)) {
-                constexpr int F = (0x3120 >> (4 * decltype(kc)::value)) & 15;   // frames 0, 2, 1, 3
-                if (!(mb & (1 << F))) return;
+            gptr<uint32_t> op = (gptr<uint32_t>)(o + ty0 * rstride);
 #pragma unroll
-                for (int j = 0; j < J; j++) {
-                    const uint64_t xv = cc[F] ^ tv[F][j];
-                    acc[j] = bcnt_add((uint32_t)(xv >> 32), bcnt_add((uint32_t)xv, acc[j]));
-                }
-            });
-#else
-            static_for<0, 4>([&](auto kc) __attribute__((always_inline)) {
-                constexpr int F = (0x3120 >> (4 * decltype(kc)::value)) & 15;   // frames 0, 2, 1, 3
-                constexpr int off = F == 0 || F == 2 ? ty * LSTR : F == 1 ? kMT - 1 - ty : ty;
-                if (!(mb & (1 << F))) return;
-                uint64_t tv[J];
-#pragma unroll
-                for (int j = 0; j < J - 1; j++) tv[j] = pa[F][off + 64 * (J - 1 - j)];
-                tv[J - 1] = pl[F][off];
-                const uint64_t cc = pc0[F * kMT * kMT + ty * kMT];
-#pragma unroll
-                for (int j = 0; j < J; j++) {
-                    const uint64_t xv = cc ^ tv[j];
-                    acc[j] = bcnt_add((uint32_t)(xv >> 32), bcnt_add((uint32_t)xv, acc[j]));
-                }
-            });
-#endif
-            gptr<uint8_t> op = o + ty * rstride;
-#pragma unroll
-            for (int j = 0; j < J - 1; j++) op[q + 64 * j] = (uint8_t)acc[j];
-            if (store_last) op[q + 64 * (J - 1)] = live_last ? (uint8_t)acc[J - 1] : (uint8_t)0;
+            for (int j = 0; j < J; j++) {
+                const uint32_t w = quad_bytes(acc[j], q);
+                if (j < J - 1 || store_last) op[16 * j] = w;
+            }
         });
     };
     Geo cur = geo(t);
