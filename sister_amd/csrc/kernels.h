@@ -33,6 +33,7 @@ struct DGroup {
     int blocks[kNumGroupKernels];
     int vcols;               // fused vertical sweep: owned columns per block (0: separate families)
     int maxHp;               // tallest padded rig of the group
+    int joined;              // paths: some family of some rig in the joined form
     int msum_split;          // 1: the two-launch cost sum even where the tiled one fits
 };
 constexpr int kMaxDGroups = 16;
@@ -74,6 +75,8 @@ void stage_blocks(const RigDesc& g, int maxD, bool wta_rows, int out[kNumStages]
 // the padded frame, debug sums) and of the winner
 int path_blocks(const RigDesc& g, int nfam, bool whole);
 int winner_blocks(const RigDesc& g, bool whole);
+size_t path_state_total(int W, int H, int D, int f);
+int path_waves(int W, int H, int f);
 int msum_blocks(const RigDesc& g, int side);   // side 0 row runs, 1 column runs, 2 tiles
 // fused vertical sweep: owned columns per block for a group whose rigs have
 // `cols` padded columns in all and disparity count D (0: not used)

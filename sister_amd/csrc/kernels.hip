@@ -1177,6 +1177,7 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
     // 64-rig step than volumes of its own.)  Either way the address is a
     // uniform base plus a loop-invariant lane offset.
     uint16_t* const Pd = g.psum;
+    const bool rows2 = g.part[1] != nullptr;   // the rows family's directions in volumes of their own
     const bool p_own = Pd != nullptr;
     constexpr int CPW = 64 / KL;                       // columns per wave
     const int lw = tid & 63;
@@ -1382,7 +1383,7 @@ __global__ __launch_bounds__(kVMaxThreads) void k_vsweep(const RigDesc* __restri
                 if (!FULL && cg.lid * CH + q >= cg.nq) return;
                 if (DIR == 0) {
                     ob[q] = LD16(g.part[0] + cell + 16 * q);
-                    ob[CH + q] = LD16(g.part[1] + cell + 16 * q);
+                    if (KEEP || rows2) ob[CH + q] = LD16(g.part[1] + cell + 16 * q);
                 } else {
                     ob[2 * q] = LD16(pd_at(y, q, 0));
                     ob[2 * q + 1] = LD16(pd_at(y, q, 1));

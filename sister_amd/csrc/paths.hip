@@ -72,6 +72,16 @@ __device__ __forceinline__ PathArea path_area(const RigDesc& g)
 }
 __host__ __device__ inline int path_chains(int w, int h, int f) { return f == 0 ? h : f == 1 ? w : w + h - 1; }
 
+// cells of a segment of the joined form
+__host__ __device__ constexpr int path_seg(int np) { return np <= 8 ? 16 : 8; }
+// bytes of a wave's forward states in the joined form: one per segment of the
+// crop part but the last, of at most that family's longest chain and 3 cells
+__host__ __device__ inline size_t path_state_bytes(int w, int h, int f, int np)
+{
+    const int longest = f == 0 ? w : f == 1 ? h : (w < h ? w : h), seg = path_seg(np);
+    return (size_t)((longest + 3 + seg - 1) / seg) * 64 * (np + 1) * 4;
+}
+
 // ---------------------------------------------------------------------------
 // The path kernel.  A wave carries four chains, 16 lanes each; a lane holds
 // 2 NP consecutive disparities as NP packed u16 pairs, so d-1 / d+1 are a byte
@@ -110,6 +120,37 @@ struct PathLane {
     int n, t0, t1;            // the chain's cells, and the range of them stored
 };
 
+// One step of the recurrence on a cell's cost bytes w: the state takes L, d the
+// pairs L - M.  tmask: 8-bit first-line path (KEEP).
+template <int NP, bool FULL, bool KEEP>
+__device__ __forceinline__ void path_step(uint32_t (&L)[NP], uint32_t& mp, const uint32_t (&pad)[NP], const uint32_t* w,
+                                          uint32_t (&d)[NP], uint32_t tmask)
+{
+    const uint32_t mpp = dup16(mp);
+    const us2 p2t = U2(mpp) + (us2){(unsigned short)kP2, (unsigned short)kP2};
+    uint32_t a[NP + 1];      // pair j: entries 2j - 1 and 2j
+    a[0] = __builtin_amdgcn_alignbit(L[0], from_left(L[NP - 1]), 16);
+    a[NP] = __builtin_amdgcn_alignbit(from_right(L[0]), L[NP - 1], 16);
+#pragma unroll
+    for (int j = 1; j < NP; j++) a[j] = __builtin_amdgcn_alignbit(L[j], L[j - 1], 16);
+    us2 rmin;
+#pragma unroll
+    for (int j = 0; j < NP; j++) {
+        const uint32_t m = (j & 1) ? bytes23(w[j / 2]) : bytes01(w[j / 2]);
+        const us2 nb = umin2(U2(a[j]), U2(a[j + 1])) + (us2){(unsigned short)kP1, (unsigned short)kP1};
+        const us2 v = umin3(nb, U2(L[j]), p2t) - U2(mpp);
+        uint32_t l = W2(v + U2(m));
+        if constexpr (KEEP) l &= tmask;
+        // every value is below 0x4000 (at most P2 + 255, or the guard), so
+        // or-ing the guard 0x3FFF into a pair past D yields the guard
+        if constexpr (!FULL) l |= pad[j];
+        d[j] = W2(v);
+        L[j] = l;
+        if (j & 1) rmin = j == 1 ? umin2(U2(L[0]), U2(l)) : umin3(rmin, U2(L[j - 1]), U2(l));   // NP is even
+    }
+    mp = group_min<kPathLanes>(min((uint32_t)rmin.x, (uint32_t)rmin.y));
+}
+
 // one direction of the wave's chains.  mb / pb: address of the wave's first
 // cell in M and in the volume, ms / ps: byte strides per cell
 template <int NP, bool FULL, bool KEEP, bool ADD>
@@ -144,30 +185,8 @@ __device__ __forceinline__ void path_sweep(PathLane<NP>& st, const uint8_t* mb, 
         __builtin_amdgcn_sched_barrier(0);
     };
     auto step = [&](const S& b, const S& o, int t, uint8_t* out, auto store) __attribute__((always_inline)) {
-        const uint32_t mpp = dup16(st.mp);
-        const us2 p2t = U2(mpp) + (us2){(unsigned short)kP2, (unsigned short)kP2};
-        uint32_t a[NP + 1];      // pair j: entries 2j - 1 and 2j
-        a[0] = __builtin_amdgcn_alignbit(st.L[0], from_left(st.L[NP - 1]), 16);
-        a[NP] = __builtin_amdgcn_alignbit(from_right(st.L[0]), st.L[NP - 1], 16);
-#pragma unroll
-        for (int j = 1; j < NP; j++) a[j] = __builtin_amdgcn_alignbit(st.L[j], st.L[j - 1], 16);
-        us2 rmin;
         uint32_t d[NP];
-#pragma unroll
-        for (int j = 0; j < NP; j++) {
-            const uint32_t m = (j & 1) ? bytes23(b.w[j / 2]) : bytes01(b.w[j / 2]);
-            const us2 nb = umin2(U2(a[j]), U2(a[j + 1])) + (us2){(unsigned short)kP1, (unsigned short)kP1};
-            const us2 v = umin3(nb, U2(st.L[j]), p2t) - U2(mpp);
-            uint32_t l = W2(v + U2(m));
-            if constexpr (KEEP) l &= tmask;          // first line of a pass: 8-bit path
-            // every value is below 0x4000 (at most P2 + 255, or the guard), so
-            // or-ing the guard 0x3FFF into a pair past D yields the guard
-            if constexpr (!FULL) l |= st.pad[j];
-            d[j] = W2(v);
-            st.L[j] = l;
-            if (j & 1) rmin = j == 1 ? umin2(U2(st.L[0]), U2(l)) : umin3(rmin, U2(st.L[j - 1]), U2(l));   // NP is even
-        }
-        st.mp = group_min<kPathLanes>(min((uint32_t)rmin.x, (uint32_t)rmin.y));
+        path_step<NP, FULL, KEEP>(st.L, st.mp, st.pad, b.w, d, tmask);
         if constexpr (decltype(store)::value) {
             uint32_t w[S::NW];
 #pragma unroll
@@ -205,7 +224,181 @@ __device__ __forceinline__ void path_sweep(PathLane<NP>& st, const uint8_t* mb, 
         });
 }
 
-template <int NP, bool FULL, bool KEEP>
+// ---------------------------------------------------------------------------
+// Both directions of the wave's chains with one byte per cell and disparity
+// (their (L - M) summed, at most 200) instead of one each.  The crop part of
+// the chains is cut into segments of path_seg cells.
+//   1. forward from the chains' first border: at each segment's start the
+//      state goes to memory (pairs and minimum, 2 bytes per disparity and
+//      segment); nothing else is stored;
+//   2. backward from the last border to the crop;
+//   3. segment by segment, last first: the costs of its cells (requested one
+//      segment ahead) and its forward state are read, the forward steps run
+//      again with their bytes kept in registers, then the backward steps, and
+//      the sums are stored.
+// The costs are read as often as by two separate waves, 1 / 2 of the bytes are
+// written (and read by k_winner or the fused sweep), for half as many steps
+// again: the form for plans bound by memory (4096x3000 D=384 39.5 -> 33.3 ms a
+// call, 1920x1080 D=192 3.84 -> 3.39, pair modes of eight 1000x620 D=136 rigs
+// 11.1 -> 9.3, the rows family ahead of the fused sweep of 64 1920x1080 rigs
+// 21.6 -> 16.7 and the sweep reading one byte less 61.7 -> 59.1).  Chains of a wave run aligned:
+// position s is a chain's own cell, and the crop part of the wave is
+// [aw, bw), the union of its chains' (which differ by at most 3 cells: all
+// inside the frame, which reaches D >= 16 cells beyond the crop).
+// ---------------------------------------------------------------------------
+template <int NP>
+constexpr int join_pf() { return NP <= 8 ? 8 : 4; }
+constexpr int kJoinMinD = 16;   // a segment's cells below the crop stay in the frame
+
+// the wave's chains in the joined form (lane values marked *)
+struct JoinGeo {
+    const uint8_t* mb;    // cost bytes of position 0 of the wave's lowest chain
+    uint8_t* pb;          // its place in the volume
+    uint32_t ms, ps;      // byte strides per position (forward, positive)
+    uint8_t* ck;          // the wave's states, one per segment after the last
+    int len, lmax;        // cells of the chain *, of the wave's longest
+    int a, b, aw, bw;     // crop part of the chain *, of the wave
+    uint32_t mlast;       // offset of the longest chain
+    uint32_t f0, b0;      // the states before the first cell *: 0, or guards (from beyond a side)
+};
+
+template <int NP, bool FULL>
+__device__ __forceinline__ void path_joined(PathLane<NP>& st, const JoinGeo& g, int lane)
+{
+    typedef Span<NP> S;
+    constexpr int PF = join_pf<NP>(), G = path_seg(NP);
+    static_assert(G % PF == 0, "states are stored between rounds of the ring");
+    const int nseg = (g.bw - g.aw + G - 1) / G, s0 = g.bw - nseg * G;   // first segment's start, above aw - G
+    auto load_cell = [&](S& c, const uint8_t* p, uint32_t o, uint32_t o1) __attribute__((always_inline)) {
+        const auto r = buf((uint8_t*)p);
+        buf_load<S::W0>(c.w, r, o);
+        if constexpr (S::W1 > 0) buf_load<S::W1>(c.w + 4, r, o1);
+    };
+    // states: planes of up to 4 dwords per lane, then the minima
+    constexpr uint32_t CK = 64 * (NP + 1) * 4;
+    auto ck_store = [&](int k, const uint32_t (&L)[NP], uint32_t mp) __attribute__((always_inline)) {
+        const auto r = buf(g.ck + (size_t)(k - 1) * CK);
+        static_for<0, NP / 4>([&](auto ic) { buf_store<4>(L + 4 * decltype(ic)::value, r, 1024u * decltype(ic)::value + 16u * lane); });
+        if constexpr (NP % 4 == 2) buf_store<2>(L + NP - 2, r, 256u * (NP - 2) + 8u * lane);
+        buf_store<1>(&mp, r, 256u * NP + 4u * lane);
+    };
+    auto ck_load = [&](int k, uint32_t (&L)[NP], uint32_t& mp) __attribute__((always_inline)) {
+        const auto r = buf(g.ck + (size_t)(k - 1) * CK);
+        static_for<0, NP / 4>([&](auto ic) { buf_load<4>(L + 4 * decltype(ic)::value, r, 1024u * decltype(ic)::value + 16u * lane); });
+        if constexpr (NP % 4 == 2) buf_load<2>(L + NP - 2, r, 256u * (NP - 2) + 8u * lane);
+        buf_load<1>(&mp, r, 256u * NP + 4u * lane);
+    };
+    // `rounds` rounds of PF steps from the wave's position p0 by step dir; the
+    // first `hold` steps stay at p0 (and, lane by lane, a chain's first `wait`
+    // steps change nothing: its state keeps init).  Requests past the last
+    // step repeat its cell.
+    auto lead = [&](uint32_t (&L)[NP], uint32_t& mp, uint32_t init, int p0, int dir, int hold, int wait, int waitmax,
+                    int rounds, auto each) __attribute__((always_inline)) {
+        const int n = rounds * PF;
+        S ring[PF];
+        const uint8_t* fp = g.mb + (long)p0 * g.ms;
+        const long ms = dir > 0 ? (long)g.ms : -(long)g.ms;
+        int fu = 0;
+        auto fetch = [&](S& c) __attribute__((always_inline)) {
+            load_cell(c, fp, fu >= wait ? st.moff : g.mlast, fu >= wait ? st.moff1 : g.mlast);
+            const bool more = fu >= hold && fu < n - 1;
+            fp += more ? ms : 0;
+            fu = min(fu + 1, n - 1);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int j = 0; j < NP; j++) L[j] = FULL ? init : (init | st.pad[j]);
+        mp = 0;
+        if (rounds == 0) return;
+        static_for<0, PF - 1>([&](auto ic) __attribute__((always_inline)) { fetch(ring[decltype(ic)::value]); });
+        int r = 0;
+        for (; r * PF < waitmax; r++) {
+            static_for<0, PF>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value;
+                fetch(ring[(i + PF - 1) % PF]);
+                uint32_t d[NP];
+                path_step<NP, FULL, false>(L, mp, st.pad, ring[i].w, d, 0);
+                const bool live = r * PF + i >= wait;
+#pragma unroll
+                for (int j = 0; j < NP; j++) L[j] = live ? L[j] : FULL ? init : (init | st.pad[j]);
+                mp = live ? mp : 0;
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            each(r + 1);
+        }
+        for (; r < rounds; r++) {
+            static_for<0, PF>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value;
+                fetch(ring[(i + PF - 1) % PF]);
+                uint32_t d[NP];
+                path_step<NP, FULL, false>(L, mp, st.pad, ring[i].w, d, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            each(r + 1);
+        }
+    };
+    uint32_t F[NP], B[NP], fm, bm;
+    // 1. forward to the last segment's start
+    const int r0 = (s0 + PF - 1) / PF, pad0 = r0 * PF - s0;
+    lead(F, fm, g.f0, 0, 1, pad0, pad0, pad0, r0 + (nseg - 1) * (G / PF), [&](int r) __attribute__((always_inline)) {
+        const int k = r - r0;   // rounds past the first segment's start
+        if (k >= 0 && k % (G / PF) == 0 && k / (G / PF) < nseg - 1) ck_store(nseg - 1 - k / (G / PF), F, fm);
+    });
+    // 2. backward to the crop
+    const int n1 = g.lmax - g.bw, r1 = (n1 + PF - 1) / PF, pad1 = r1 * PF - n1;
+    lead(B, bm, g.b0, g.lmax - 1, -1, pad1, pad1 + g.lmax - g.len, pad1 + 3, r1, [](int) {});
+    // 3. the segments (segment k ends at bw - k G)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's states, read back below
+    S cur[G], nxt[G];
+    uint32_t Fn[NP], fmn = 0;
+    auto request = [&](int k, S (&c)[G]) __attribute__((always_inline)) {
+        const uint8_t* p = g.mb + (long)(g.bw - (k + 1) * G) * g.ms;
+        static_for<0, G>([&](auto ic) __attribute__((always_inline)) {
+            load_cell(c[decltype(ic)::value], p, st.moff, st.moff1);
+            p += g.ms;
+        });
+    };
+    request(0, nxt);
+    for (int k = 0; k < nseg; k++) {
+#pragma unroll
+        for (int i = 0; i < G; i++) cur[i] = nxt[i];
+        if (k > 0) {
+#pragma unroll
+            for (int j = 0; j < NP; j++) F[j] = Fn[j];
+            fm = fmn;
+        }
+        const int kn = min(k + 1, nseg - 1);   // past the last segment: requested again
+        request(kn, nxt);
+        ck_load(max(kn, 1), Fn, fmn);
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t fw[G][S::NW];
+        static_for<0, G>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            uint32_t d[NP];
+            path_step<NP, FULL, false>(F, fm, st.pad, cur[i].w, d, 0);
+#pragma unroll
+            for (int q = 0; q < S::NW; q++) fw[i][q] = pack4(d[2 * q], d[2 * q + 1]);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        const int sk = g.bw - (k + 1) * G;
+        uint8_t* out = g.pb + (long)(sk + G - 1) * g.ps;
+        static_for<0, G>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = G - 1 - decltype(ic)::value;
+            uint32_t d[NP], w[S::NW];
+            path_step<NP, FULL, false>(B, bm, st.pad, cur[i].w, d, 0);
+#pragma unroll
+            for (int q = 0; q < S::NW; q++) w[q] = fw[i][q] + pack4(d[2 * q], d[2 * q + 1]);   // bytes <= 100 each
+            const bool in = sk + i >= g.a && sk + i < g.b;
+            const auto r = buf(out);
+            buf_store<S::W0>(w, r, in ? st.poff : kDropped);
+            if constexpr (S::W1 > 0) buf_store<S::W1>(w + 4, r, in ? st.poff1 : kDropped);
+            out -= g.ps;
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    }
+}
+
+template <int NP, bool FULL, bool KEEP, bool JOIN>
 __global__ __launch_bounds__(64) void k_paths(const RigDesc* __restrict__ rigs, int nrig, const int* __restrict__ bs,
                                               int nfam, int frame)
 {
@@ -293,6 +486,61 @@ __global__ __launch_bounds__(64) void k_paths(const RigDesc* __restrict__ rigs, 
             st, g.msum + mlo, (long)(dy * Wp + dx) * Dp, g.part[2 * f + (both ? 0 : dr)] + plo, (long)(dy * pw + dx) * Dp,
             nmax, tmin, (uint32_t)(mlong - mlo), first_line ? 0x00FF00FFu : 0xFFFFFFFFu);
     };
+    if (JOIN && g.ck[f]) {
+        // chain c from its forward border: position 0 .. len - 1, crop part [a, b)
+        JoinGeo J;
+        int x, y, dx = 1, dy = 1, ya = ar.y0, yb = ar.y1, ye = Hp - 1;
+        J.f0 = J.b0 = 0;
+        if (f == 0) {
+            y = ar.y0 + c; x = 0; dy = 0;
+            J.a = ar.x0; J.b = ar.x1 + 1; J.len = Wp;
+        } else {
+            if (f == 1) {
+                x = ar.x0 + c; y = 0; dx = 0;
+            } else if (f == 2) {
+                const int k = c + ar.x0 - ar.y1;   // x - y
+                y = max(0, -k); ye = min(Hp - 1, Wp - 1 - k);
+                x = y + k;
+                ya = max(ya, ar.x0 - k); yb = min(yb, ar.x1 - k);
+            } else {
+                const int s = c + ar.x0 + ar.y0;   // x + y
+                y = max(0, s - (Wp - 1)); ye = min(Hp - 1, s);
+                x = s - y; dx = -1;
+                ya = max(ya, s - ar.x1); yb = min(yb, s - ar.x0);
+            }
+            J.a = ya - y; J.b = yb - y + 1; J.len = ye - y + 1;
+            J.f0 = y > 0 ? kGuard2 : 0u;
+            J.b0 = ye < Hp - 1 ? kGuard2 : 0u;
+        }
+        const long mo = ((long)y * Wp + x) * Dp, po = ((long)(y - poy) * pw + (x - pox)) * Dp;
+        long mlo = lane64(mo, 0), plo = lane64(po, 0), mlong = mlo;
+        J.lmax = __builtin_amdgcn_readlane(J.len, 0);
+        J.aw = __builtin_amdgcn_readlane(J.a, 0);
+        J.bw = __builtin_amdgcn_readlane(J.b, 0);
+#pragma unroll
+        for (int k = 1; k < kPathChains; k++) {
+            const long m1 = lane64(mo, k * kPathLanes);
+            const int n1 = __builtin_amdgcn_readlane(J.len, k * kPathLanes);
+            mlo = min(mlo, m1);
+            plo = min(plo, lane64(po, k * kPathLanes));
+            if (n1 > J.lmax) { J.lmax = n1; mlong = m1; }
+            J.aw = min(J.aw, __builtin_amdgcn_readlane(J.a, k * kPathLanes));
+            J.bw = max(J.bw, __builtin_amdgcn_readlane(J.b, k * kPathLanes));
+        }
+        if (ci >= nch) J.b = J.a;                  // a repeated chain: not stored
+        st.moff = (uint32_t)(mo - mlo) + (has ? b0 : 0);
+        st.moff1 = (uint32_t)(mo - mlo) + (has1 ? b0 + 16 : 0);
+        st.poff = has ? (uint32_t)(po - plo) + b0 : kDropped;
+        st.poff1 = has1 ? (uint32_t)(po - plo) + b0 + 16 : kDropped;
+        J.mlast = (uint32_t)(mlong - mlo);
+        J.mb = g.msum + mlo;
+        J.pb = g.part[2 * f] + plo;
+        J.ms = (uint32_t)((dy * Wp + dx) * Dp);
+        J.ps = (uint32_t)((dy * pw + dx) * Dp);
+        J.ck = g.ck[f] + (size_t)lb * path_state_bytes(aw, ah, f, NP);
+        path_joined<NP, FULL>(st, J, lane);
+        return;
+    }
     sweep(dir, IC<0>{});
     if (both) {
         // the second direction reads the bytes this wave has just stored
@@ -436,32 +684,49 @@ int path_blocks(const RigDesc& g, int nfam, bool whole)
     return n;
 }
 
+int path_waves(int W, int H, int f) { return (path_chains(W, H, f) + kPathChains - 1) / kPathChains; }
+
 int winner_blocks(const RigDesc& g, bool whole)
 {
     const long n = whole ? (long)g.Wp * g.Hp : (long)g.W * g.H;
     return (int)((n + kWinCells - 1) / kWinCells);
 }
 
-#define SISTER_PATHS(NPV, FULLV, KEEPV)                                                                          \
-    hipLaunchKernelGGL((k_paths<NPV, FULLV, KEEPV>), dim3(G.blocks[kGPaths]), dim3(64), 0, st, G.rigs, G.nrig,   \
-                       G.bs[kGPaths], nfam, frame)
-#define SISTER_WINNER(NPV, FULLV, KEEPV)                                                                         \
+#define SISTER_PATHS(NPV, FULLV, KEEPV)                                                                           \
+    do {                                                                                                          \
+        if (!KEEPV && G.joined)                                                                                   \
+            hipLaunchKernelGGL((k_paths<NPV, FULLV, KEEPV, !KEEPV>), dim3(G.blocks[kGPaths]), dim3(64), 0, st,    \
+                               G.rigs, G.nrig, G.bs[kGPaths], nfam, frame);                                       \
+        else                                                                                                      \
+            hipLaunchKernelGGL((k_paths<NPV, FULLV, KEEPV, false>), dim3(G.blocks[kGPaths]), dim3(64), 0, st,     \
+                               G.rigs, G.nrig, G.bs[kGPaths], nfam, frame);                                       \
+    } while (0)
+#define SISTER_WINNER(NPV, FULLV, KEEPV)                                                                          \
     hipLaunchKernelGGL((k_winner<NPV, FULLV, KEEPV>), dim3(G.blocks[kGWinner]), dim3(256), 0, st, G.rigs, G.nrig, \
                        G.bs[kGWinner], mode)
 // FULL where every pair of every lane is a real disparity
-#define SISTER_BY_PAIRS(K)                                                  \
-    do {                                                                    \
-        const int np = path_pairs(G.Dp);                                    \
-        const bool full = G.D == 32 * np && !keep_sum;                      \
-        switch (np) {                                                       \
+#define SISTER_BY_PAIRS(K)                                                                                        \
+    do {                                                                                                          \
+        const int np = path_pairs(G.Dp);                                                                          \
+        const bool full = G.D == 32 * np && !keep_sum;                                                            \
+        switch (np) {                                                                                             \
         case 2: if (keep_sum) K(2, false, true); else if (full) K(2, true, false); else K(2, false, false); break;      \
         case 4: if (keep_sum) K(4, false, true); else if (full) K(4, true, false); else K(4, false, false); break;      \
         case 6: if (keep_sum) K(6, false, true); else if (full) K(6, true, false); else K(6, false, false); break;      \
         case 8: if (keep_sum) K(8, false, true); else if (full) K(8, true, false); else K(8, false, false); break;      \
         case 12: if (keep_sum) K(12, false, true); else if (full) K(12, true, false); else K(12, false, false); break;  \
         default: if (keep_sum) K(16, false, true); else if (full) K(16, true, false); else K(16, false, false); break;  \
-        }                                                                   \
+        }                                                                                                         \
     } while (0)
+
+// bytes of the forward states of family f of a rig in the joined form (0: D
+// too small for it)
+size_t path_state_total(int W, int H, int D, int f)
+{
+    if (D < kJoinMinD) return 0;
+    const size_t waves = (size_t)(path_chains(W, H, f) + kPathChains - 1) / kPathChains;
+    return waves * path_state_bytes(W, H, f, path_pairs((D + 15) & ~15));
+}
 
 // every path of a group (its rows family alone ahead of the fused vertical sweep)
 void launch_paths(const DGroup& G, int keep_sum, hipStream_t st)

@@ -36,9 +36,11 @@ struct RigDesc {
     uint8_t* part[8];         // (L - M) bytes, each in [0, 100], of the eight SGM paths:
                               // [2f] going right or down, [2f+1] left or up, f = rows,
                               // columns, diagonals, anti-diagonals.  A null [2f+1]: both
-                              // directions summed in [2f].  Cells of the crop, W x H x Dp;
+                              // directions summed in [2f], by the joined form where ck[f]
+                              // is set.  Cells of the crop, W x H x Dp;
                               // of the padded frame ahead of the fused vertical sweep
-                              // (which has [0] and [1] alone) and with the debug sums
+                              // (which has the rows' alone) and with the debug sums
+    uint8_t* ck[4];           // joined form: forward states of the family's segments
     uint16_t* psum;           // fused vertical sweep: partial sums P (null: they replace
                               // the bytes of part[0] and part[1] row by row)
     uint32_t* vstate;         // fused vertical sweep: segment-end states, normalised

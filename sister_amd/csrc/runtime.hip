@@ -37,6 +37,8 @@ namespace {
 // workspace layout of one rig (offsets from the workspace base)
 struct WsLayout {
     size_t code, wta, med, mask, msum, part, nvol, vol, edge, scratch, vstate, sum, total;
+    bool join;       // the families in the joined form
+    size_t ck[4];    // their forward states (0: not joined)
 };
 
 inline int padded_depth(int D) { return (D + 15) & ~15; }
@@ -46,15 +48,18 @@ inline int padded_depth(int D) { return (D + 15) & ~15; }
 // pixel and of what only the fused sweep needs (edge rows, segment states):
 // as many of the eight paths' volumes over the crop as fit are kept apart
 // (all eight where the crop is at most 5/8 of the frame), and the two
-// directions of the other families share one.  With the debug sums five
-// volumes over the frame.  Otherwise the fused vertical sweep: four (the rows
-// family's two, its partial sums P in two) or, in_place (plans short of
-// memory; only for D = 16 KL CH and not in the debug sweep), two: P then
+// directions of the other families share one.  join (plans bound by memory):
+// the joined form, four volumes and the forward states.  With the debug sums
+// five volumes over the frame.  Otherwise the fused vertical sweep: four (the
+// rows family's two, its partial sums P in two), three with join (the rows
+// joined) or, in_place (plans short of memory; only for D = 16 KL CH and not in
+// the debug sweep), two: P then
 // replaces the rows bytes row by row.  The serial median's order statistics
 // (prepass form) alias the volumes, which nothing writes before the SGM.
 // Footprints for admission and sister_workspace_bytes take the default, the
 // largest form.
-WsLayout ws_layout(int W, int H, int D, bool keep_sum = false, bool separate = true, bool in_place = false)
+WsLayout ws_layout(int W, int H, int D, bool keep_sum = false, bool separate = true, bool in_place = false,
+                   bool join = false)
 {
     const size_t Wp = (size_t)W + 2 * D, Hp = (size_t)H + 2 * D;
     const size_t npx = Wp * Hp, ncell = npx * padded_depth(D);
@@ -65,15 +70,31 @@ WsLayout ws_layout(int W, int H, int D, bool keep_sum = false, bool separate = t
     l.med = o;     o += align_up(8 * npx * sizeof(uint16_t));
     l.mask = o;    o += align_up(4 * npx);
     l.msum = o;    o += align_up(ncell);
-    l.nvol = separate ? 5 : (in_place && vsweep_in_place(D) && !keep_sum) ? 2 : 4;
+    const bool two = !separate && in_place && vsweep_in_place(D) && !keep_sum;
+    size_t cks[4], ckall = 0;
+    for (int f = 0; f < 4; f++) {
+        cks[f] = f == 0 || separate ? align_up(path_state_total(W, H, D, f)) : 0;
+        ckall += cks[f];
+        l.ck[f] = 0;
+    }
+    l.join = join && !keep_sum && !two && cks[0] > 0;
+    l.nvol = separate ? 5 : two ? 2 : l.join ? 3 : 4;
     l.vol = align_up(ncell);
-    l.part = o;    o += std::max(l.nvol * l.vol, align_up(8 * npx * sizeof(uint64_t)));
+    l.part = o;    o += std::max(l.nvol * l.vol + (!separate && l.join ? ckall : 0), align_up(8 * npx * sizeof(uint64_t)));
+    if (!separate && l.join) l.ck[0] = l.part + l.nvol * l.vol;
     l.scratch = l.part;
     l.edge = o;    o += align_up(4 * 2 * Wp * padded_depth(D) * sizeof(uint16_t));
     l.vstate = o;  o += align_up(2 * 3 * Wp * (padded_depth(D) + 16));
     if (separate && !keep_sum) {
         l.vol = align_up((size_t)W * H * padded_depth(D));
-        l.nvol = std::min<size_t>(8, (o - l.part) / l.vol);
+        const size_t room = o - l.part;
+        l.join = l.join && 4 * l.vol + ckall <= room;   // about 4.6 volumes
+        l.nvol = l.join ? 4 : std::min<size_t>(8, room / l.vol);
+        size_t at = l.part + l.nvol * l.vol;
+        for (int f = 0; l.join && f < 4; f++) {
+            l.ck[f] = at;
+            at += cks[f];
+        }
     }
     l.sum = o;     if (keep_sum) o += align_up(ncell * sizeof(uint16_t));
     l.total = o;
@@ -392,6 +413,16 @@ static void record_latency(sister_ctx* c, double ms)
             return fail(ctx, SISTER_EDEVICE, std::string(#expr ": ") + hipGetErrorString(_e));   \
     } while (0)
 
+// Vertical waves of a group (four chains each) from which its chains run in the
+// joined form: about one per SIMD.  Below, the steps of the longest chains set
+// the time (640x480 D=64, 840 waves: 0.43 ms apart, 0.47 joined); from there on
+// memory does (1244x700 D=200, 1283 waves, three modes: 5.65 apart, 5.46
+// joined; 1920x1080 D=192, 1980 waves: 3.84 and 3.39 ms).
+#ifndef SISTER_JOIN_WAVES
+#define SISTER_JOIN_WAVES 1024
+#endif
+constexpr long kJoinWaves = SISTER_JOIN_WAVES;
+
 // Build the device plan for n rigs whose views/outputs are device pointers.
 // The rig table is ordered by D so that the SGM launches can take each group
 // of equal depth as one contiguous slice.
@@ -450,13 +481,13 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         p.host_rigs.push_back(g);
     }
     // SGM groups: runs of equal D
-    struct GroupHost { int i0, i1, vcols, maxHp, msum_split; };
+    struct GroupHost { int i0, i1, vcols, maxHp, msum_split, join; };
     std::vector<GroupHost> groups;
     for (int k = 0; k < n;) {
         int e = k;
         long chains = 0;
         while (e < n && p.host_rigs[e].D == p.host_rigs[k].D) chains += p.host_rigs[e++].Wp;
-        GroupHost G{k, e, 0, 0, 0};
+        GroupHost G{k, e, 0, 0, 0, 0};
         for (int j = k; j < e; j++) G.maxHp = std::max(G.maxHp, p.host_rigs[j].Hp);
         const int D = p.host_rigs[k].D;
         GroupForm form;
@@ -465,16 +496,22 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         // the debug switch wins over a tuned form
         G.vcols = vsweep_pick_cols(chains, D, c->vsweep >= 0 ? c->vsweep : form.fused);
         G.msum_split = form.msum_split;
+        long waves = 0;
+        for (int j = k; j < e; j++)
+            for (int f = 1; f < 4; f++) waves += path_waves(p.host_rigs[j].W, p.host_rigs[j].H, f);
+        G.join = waves >= kJoinWaves;
         groups.push_back(G);
         k = e;
     }
     // workspaces: a rig of a fused group has four SGM volumes (two in place),
     // the others five
     std::vector<WsLayout> lay(n);
-    for (const GroupHost& G : groups)
+    for (GroupHost& G : groups) {
+        bool lay_join = false;
         for (int k = G.i0; k < G.i1; k++) {
             RigDesc& g = p.host_rigs[k];
-            const WsLayout l = ws_layout(g.W, g.H, g.D, c->keep_sum, G.vcols == 0, p_in_place || c->p_in_place);
+            const WsLayout l = ws_layout(g.W, g.H, g.D, c->keep_sum, G.vcols == 0, p_in_place || c->p_in_place,
+                                         G.vcols > 0 || G.join);
             lay[k] = l;
             Block b;
             if (get(l.total, b) != 0) return no_room("workspace of " + std::to_string(l.total) + " bytes");
@@ -490,25 +527,24 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
             uint8_t* const vols = (uint8_t*)(b.ptr + l.part);
             for (int q = 0; q < 8; q++) g.part[q] = nullptr;
             g.psum = nullptr;
-            if (G.vcols > 0) {
-                g.part[0] = vols;
-                g.part[1] = vols + l.vol;
-                if (l.nvol == 4) g.psum = (uint16_t*)(vols + 2 * l.vol);
-            } else {
-                // the rows' directions always have a volume each; with fewer
-                // than eight, columns, diagonals and anti-diagonals join theirs
-                // in this order
-                const int joined = 8 - (int)l.nvol;
-                size_t v = 0;
-                for (int f = 0; f < 4; f++) {
-                    g.part[2 * f] = vols + l.vol * v++;
-                    if (f == 0 || f > joined) g.part[2 * f + 1] = vols + l.vol * v++;
-                }
+            // a family's second direction has a volume of its own, or shares the
+            // first's: in the joined form, or with fewer than eight volumes
+            // (columns, diagonals and anti-diagonals in this order)
+            const int shared = G.vcols > 0 || l.join ? 0 : 8 - (int)l.nvol;
+            size_t v = 0;
+            for (int f = 0; f < (G.vcols > 0 ? 1 : 4); f++) {
+                g.ck[f] = l.ck[f] ? (uint8_t*)(b.ptr + l.ck[f]) : nullptr;
+                g.part[2 * f] = vols + l.vol * v++;
+                if (!g.ck[f] && (f == 0 || f > shared)) g.part[2 * f + 1] = vols + l.vol * v++;
             }
+            if (G.vcols > 0 && l.nvol > 2) g.psum = (uint16_t*)(vols + l.vol * v);
+            lay_join = lay_join || l.join;
             g.edge = (uint16_t*)(b.ptr + l.edge);
             g.vstate = (uint32_t*)(b.ptr + l.vstate);
             g.sum = c->keep_sum ? (uint16_t*)(b.ptr + l.sum) : nullptr;
         }
+        G.join = lay_join;
+    }
     if ((int)groups.size() > kMaxDGroups) {
         drop();
         return fail(c, SISTER_EINVAL, "too many distinct disparity counts in one batch");
@@ -590,6 +626,7 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         sg.vcols = G.vcols;
         sg.maxHp = G.maxHp;
         sg.msum_split = G.msum_split;
+        sg.joined = G.join;
     }
     return SISTER_OK;
 }

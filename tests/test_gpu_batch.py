@@ -413,3 +413,26 @@ def test_median_strips_match_oracle(gpu_ctx, oracle_mod, W):
             for side in range(2):
                 g = gpu_ctx.fetch(n - 1, "med", 2 * F + side, shapes[F], np.uint16)
                 assert np.array_equal(g, ref["med_r" if side else "med_l"][F].astype(np.uint16)), (n, F, side)
+
+
+@pytest.mark.parametrize("W,H,D", [(64, 48, 16), (28, 36, 24), (52, 40, 64), (36, 28, 72), (20, 36, 128), (40, 24, 144),
+                                   (24, 20, 152), (32, 24, 192), (24, 20, 208), (20, 16, 272), (24, 16, 288),
+                                   (16, 12, 336), (16, 8, 448)])
+def test_joined_chains_match_oracle(gpu_ctx, oracle_mod, W, H, D):
+    """Enough small rigs in one plan that their chains run in the joined form
+    (1024 vertical waves): each number of pairs per lane, crops of less than a
+    segment, whole segments and parts of one, all three modes."""
+    import torch
+    waves = (W + 3) // 4 + 2 * ((W + H + 2) // 4)
+    n = -(-1024 // waves)
+    rigs = [synth.rig_small(W, H, D, 800 + D + k) for k in range(2)]
+    refs = [oracle_mod.compute(r["views"], D, modes=7) for r in rigs]
+    views = [[torch.from_numpy(v).cuda() for v in r["views"]] for r in rigs]
+    names = ("multiview", "horizontal", "vertical", "disp")
+    outs = [{k: torch.zeros((H, W), dtype=torch.uint16, device="cuda") for k in names} for _ in range(n)]
+    print(f"[joined] {n} rigs W={W} H={H} D={D}", flush=True)
+    gpu_ctx.run_device([gpu_ctx.rig_struct(views[i % 2], D, outs[i]) for i in range(n)], sister_amd.MODE_ALL)
+    gpu_ctx.sync()
+    for i in range(n):
+        for k in names:
+            assert np.array_equal(outs[i][k].cpu().numpy(), refs[i % 2][k]), (i, k)
