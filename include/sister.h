@@ -124,9 +124,8 @@ int sister_graph_launch(sister_ctx* ctx);
    balanced by padded cells, or one part per disparity count, so that groups
    of different D run side by side, and the parts started together or each
    after the previous part's first stages), then for each disparity group of those
-   parts the SGM vertical families fused or separate, and the tiled or
-   two-launch cost sum.  The fastest
-   of each is kept in the context's table, which every later plan and capture
+   parts the SGM vertical families fused or separate.  The fastest of
+   each is kept in the context's table, which every later plan and capture
    of a matching shape consults: groups are matched by D and the half-octaves
    of their padded column total and tallest padded rig, batches by rig count,
    distinct D count, half-octave of padded cells and modes.  Shapes already in

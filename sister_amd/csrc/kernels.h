@@ -20,8 +20,8 @@ enum Stage {
 enum GroupKernel {
     kGPaths = 0,                          // SGM chains (ahead of the fused sweep: the rows family's)
     kGWinner,                             // S and the winner from the chains' bytes
-    kGMsumRows, kGMsumCols,               // cost sum: frames 0/180 (row runs), 90/270 (column runs)
-    kGMsumTile,                           // cost sum: all frames, per 16x16 tile
+    kGCost,                               // cost sum, per tile
+    kGMsumRows, kGMsumCols,               // cost sum, D > 256: row runs, column runs
     kGVSweep,                             // fused vertical SGM families, per column block
     kNumGroupKernels
 };
@@ -34,7 +34,6 @@ struct DGroup {
     int vcols;               // fused vertical sweep: owned columns per block (0: separate families)
     int maxHp;               // tallest padded rig of the group
     int joined;              // paths: some family of some rig in the joined form
-    int msum_split;          // 1: the two-launch cost sum even where the tiled one fits
 };
 constexpr int kMaxDGroups = 16;
 
@@ -77,7 +76,9 @@ int path_blocks(const RigDesc& g, int nfam, bool whole);
 int winner_blocks(const RigDesc& g, bool whole);
 size_t path_state_total(int W, int H, int D, int f);
 int path_waves(int W, int H, int f);
-int msum_blocks(const RigDesc& g, int side);   // side 0 row runs, 1 column runs, 2 tiles
+int cost_blocks(const RigDesc& g);
+int msum_blocks(const RigDesc& g, int side);   // side 0 row runs, 1 column runs
+int path_pairs(int Dp);   // pairs of disparities per lane (16 lanes) of the path and cost kernels
 // fused vertical sweep: owned columns per block for a group whose rigs have
 // `cols` padded columns in all and disparity count D (0: not used)
 int vsweep_pick_cols(long cols, int D, int choice);

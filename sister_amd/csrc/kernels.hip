@@ -7,7 +7,7 @@
 //   median3x3_SSE in place postprocess.cpp:15-71        k_median (median.hip)
 //   doLRCheck + mask loops postprocess.cpp:318-341,     k_mask
 //                          hpp:201-251
-//   realign + weighted sum hpp:255-277                  k_msum
+//   realign + weighted sum hpp:255-277                  k_cost, k_msum_run (cost.hip)
 //   accumulateCostsSSE     sgm.cpp:26-455               k_paths (paths.hip); batches: rows
 //                                                       in k_paths, the rest in k_vsweep
 //   WTALeft on S, convert  hpp:283,111-118              k_winner (paths.hip), or in k_vsweep
@@ -523,372 +523,6 @@ __global__ __launch_bounds__(256) void k_mask(const RigDesc* __restrict__ rigs, 
         int y, x;
         frame_to_orig(g, F, r, c, y, x);
         G(mk)[(size_t)y * g.Wp + x] = tile[tc][tr + 8 * k];
-    }
-}
-
-// ---------------------------------------------------------------------------
-// K5 mask-weighted cost sum (hpp:255-277).  M(y,x,d) = sum over used frames F
-// with mask_F(y,x) = 1 of pop(CC_F[r][c] ^ CN_F[r][c-d]), (r,c) the frame
-// pixel of (y,x).  A set mask implies c >= D > d, so every term is a plain
-// popcount (<= 63) and M <= 252 fits a byte.
-// Each frame's partners of a pixel lie along its frame row, which is an
-// image row for frames 0/180 and an image column for frames 90/270, so two
-// launches share the work: k_msum_run<0> (frames 0 and 180, one block = a run
-// of kRun pixels of one row) writes M, k_msum_run<1> (frames 90 and 270, one
-// block = a run of one column) adds to it.  Each block stages the partner
-// window of its run (kRun + D - 1 codes per frame) in LDS once.  A wave takes
-// one pixel at a time, lane q the disparities q + 64 j: conflict-free 8-byte
-// LDS reads at immediate offsets, with no per-disparity branches, and stores
-// four pixels together (quad_bytes).  Cell stride Dp, zero past D.
-// ---------------------------------------------------------------------------
-constexpr int kRun = 256;   // pixels per block
-constexpr int kWinPad = 8;  // window entries before each partner window
-
-// acc[j] += pop(cc ^ window[base - d]) for lane q's disparities d = q + 64 j.
-// In the last group, lanes at or past Dp read as lane qlast = Dp - 1 - 64 (J-1)
-// (their sums are not stored) and lanes at or past D are zeroed by the caller.
-template <int J>
-__device__ __forceinline__ void msum_add_frame(const uint64_t* L, uint64_t cc, int base, int q, int qlast,
-                                               unsigned (&acc)[J])
-{
-    uint64_t tv[J];
-    const uint64_t* w = L + base - q;       // w[-64 j] = window[base - d]
-#pragma unroll
-    for (int j = 0; j < J - 1; j++) tv[j] = w[-64 * j];
-    tv[J - 1] = L[base - qlast - 64 * (J - 1)];
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        const uint64_t x = cc ^ tv[j];
-        acc[j] = bcnt_add((uint32_t)(x >> 32), bcnt_add((uint32_t)x, acc[j]));
-    }
-}
-
-// Stores of M.  A wave's lane q holds one disparity of a pixel, so one pixel's
-// bytes would leave as byte stores (16 or more address cycles for 64 bytes).
-// Four pixels go together instead: a lane packs its disparity's four sums and
-// a 4 x 4 byte transpose over each four lanes (two DPP exchanges, two byte
-// permutes) leaves lane l the disparities (l & ~3) .. + 3 of pixel l & 3, one
-// dword store for four pixels.  Two-launch form: pair modes of eight 1000x620
-// D=136 rigs 1.56 -> 1.28 ms, 4096x3000 D=384 6.2 -> 5.7 ms; tiled form
-// 640x480 D=64 53 -> 48 us, 64 rigs 1920x1080 D=192 34.0 -> 33.0 ms.
-__device__ __forceinline__ uint32_t quad_bytes(const unsigned (&a)[4], int lane)
-{
-    const uint32_t own = a[0] | (a[1] << 8) | (a[2] << 16) | (a[3] << 24);
-    const uint32_t n1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)own, 0xB1, 0xF, 0xF, true);   // lane ^ 1
-    const uint32_t h = __builtin_amdgcn_perm(n1, own, (lane & 1) ? 0x03070105u : 0x06020400u);
-    const uint32_t n2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0x4E, 0xF, 0xF, true);     // lane ^ 2
-    return __builtin_amdgcn_perm(n2, h, (lane & 2) ? 0x03020706u : 0x05040100u);
-}
-
-// SIDE = 0: frames 0/180 along row y; SIDE = 1: frames 90/270 along column x.
-// J = ceil(Dp / 64) groups of 64 disparities; every rig of the launch has this Dp.
-template <int SIDE, int J>
-__global__ __launch_bounds__(256) void k_msum_run(const RigDesc* __restrict__ rigs, int nrig,
-                                                  const int* __restrict__ bs, int fuse)
-{
-    extern __shared__ uint64_t lds64[];
-    const int ri = find_rig(bs, nrig, blockIdx.x);
-    const RigDesc& g = rigs[ri];
-    const int lb = blockIdx.x - bs[ri];
-    const int Wp = g.Wp, Hp = g.Hp, D = g.D, Dp = g.Dp;
-    const int FA = SIDE == 0 ? 0 : 1, FB = SIDE == 0 ? 2 : 3;   // frame pair
-    const bool useA = (fuse >> FA) & 1, useB = (fuse >> FB) & 1;
-    // the run: SIDE 0 -> row y, x in [p0, p0+kRun); SIDE 1 -> column x, y in [p0, p0+kRun)
-    const int runs = SIDE == 0 ? (Wp + kRun - 1) / kRun : (Hp + kRun - 1) / kRun;
-    const int line = lb / runs, p0 = (lb % runs) * kRun;
-    const int len = SIDE == 0 ? Wp : Hp;        // pixels along the line
-    const int SPAN = kRun + D - 1;
-    // lanes of the last group past D read up to Dp - D <= 8 entries before
-    // their window; those terms are masked
-    uint64_t* LA = lds64 + kWinPad;             // partners of frame FA
-    uint64_t* LB = LA + SPAN + kWinPad;         // partners of frame FB
-    uint64_t* LCa = LB + SPAN;                  // centers
-    uint64_t* LCb = LCa + kRun;
-    uint8_t* LM = (uint8_t*)(LCb + kRun);
-    const int tid = threadIdx.x;
-    // frame row holding the line and the frame column of run pixel i:
-    //  SIDE 0: F0 row y col x;  F2 row y col W'-1-x
-    //  SIDE 1: F1 row W'-1-x col H'-1-y;  F3 row W'-1-x col y
-    const int frow = band_row(SIDE == 0 ? line : Wp - 1 - line, SIDE == 0 ? Hp : Wp, D);   // stored row
-    const int fcols = SIDE == 0 ? Wp : Hp;
-    const uint64_t* NA = g.code[2 * FA + 1] + (size_t)frow * fcols;
-    const uint64_t* NB = g.code[2 * FB + 1] + (size_t)frow * fcols;
-    const uint64_t* CA = g.code[2 * FA] + (size_t)frow * fcols;
-    const uint64_t* CB = g.code[2 * FB] + (size_t)frow * fcols;
-    // window of frame X: the frame columns [lo, lo + SPAN) covering every
-    // partner col - d of the run (frame A columns run with the line
-    // coordinate for F0 and F3, against it for F1 and F2)
-    int loA, loB;
-    if (SIDE == 0) { loA = p0 - (D - 1); loB = Wp - p0 - kRun - (D - 1); }
-    else { loA = Hp - p0 - kRun - (D - 1); loB = p0 - (D - 1); }
-    for (int k = tid - kWinPad; k < SPAN; k += 256) {
-        const int ca = loA + k, cb = loB + k;
-        LA[k] = (useA && k >= 0 && ca >= 0 && ca < fcols) ? G(NA)[ca] : 0;
-        LB[k] = (useB && k >= 0 && cb >= 0 && cb < fcols) ? G(NB)[cb] : 0;
-    }
-    for (int i = tid; i < kRun; i += 256) {
-        const int pos = p0 + i;                 // x (SIDE 0) or y (SIDE 1)
-        uint64_t a = 0, b = 0;
-        uint8_t mb = 0;
-        if (pos < len) {
-            const int colA = SIDE == 0 ? pos : Hp - 1 - pos;
-            const int colB = SIDE == 0 ? Wp - 1 - pos : pos;
-            const int y = SIDE == 0 ? line : pos, x = SIDE == 0 ? pos : line;
-            const size_t q = (size_t)y * Wp + x;
-            if (useA) a = G(CA)[colA];
-            if (useB) b = G(CB)[colB];
-            // a set mask implies frame column >= D; the check keeps indices in range
-            if (useA && G(g.mask[FA])[q] && colA >= D) mb |= 1;
-            if (useB && G(g.mask[FB])[q] && colB >= D) mb |= 2;
-        }
-        LCa[i] = a;
-        LCb[i] = b;
-        LM[i] = mb;
-    }
-    __syncthreads();
-    // one wave per pixel, four pixels of the run at a time (the line's length is
-    // a multiple of 4); lane q owns d = q + 64 j.  In the last group, lanes at
-    // or past Dp read as lane Dp - 1 - 64 (J - 1) (and store nothing), lanes at
-    // or past D add nothing.
-    const int wave = tid >> 6, q = tid & 63;
-    const int qlast = min(q, Dp - 1 - 64 * (J - 1));
-    const bool store_last = (q & ~3) + 64 * (J - 1) < Dp;
-    const bool live_last = q + 64 * (J - 1) < D;
-    const size_t pstep = (size_t)(SIDE == 0 ? 1 : Wp) * Dp;     // to the line's next pixel
-    for (int i = 4 * wave; i < kRun; i += 16) {
-        const int pos = p0 + i;
-        if (pos >= len) break;
-        const int y = SIDE == 0 ? line : pos, x = SIDE == 0 ? pos : line;
-        gptr<uint32_t> o = (gptr<uint32_t>)(G(g.msum) + ((size_t)y * Wp + x) * Dp + (q & 3) * pstep + (q & ~3));
-        uint32_t old[J];
-        if (SIDE == 1 && (fuse & 5)) {
-#pragma unroll
-            for (int j = 0; j < J; j++)
-                if (j < J - 1 || store_last) old[j] = o[16 * j];
-        }
-        unsigned acc[J][4];
-        static_for<0, 4>([&](auto kc) __attribute__((always_inline)) {
-            constexpr int k = decltype(kc)::value;
-            unsigned a[J];
-#pragma unroll
-            for (int j = 0; j < J; j++) a[j] = 0;
-            const int mb = __builtin_amdgcn_readfirstlane(LM[i + k]);   // one pixel per wave
-            const int pk = pos + k;
-            if (mb & 1) msum_add_frame<J>(LA, LCa[i + k], (SIDE == 0 ? pk : Hp - 1 - pk) - loA, q, qlast, a);
-            if (mb & 2) msum_add_frame<J>(LB, LCb[i + k], (SIDE == 0 ? Wp - 1 - pk : pk) - loB, q, qlast, a);
-            a[J - 1] = live_last ? a[J - 1] : 0u;
-#pragma unroll
-            for (int j = 0; j < J; j++) acc[j][k] = a[j];
-        });
-#pragma unroll
-        for (int j = 0; j < J; j++) {
-            uint32_t w = quad_bytes(acc[j], q);
-            if (SIDE == 1 && (fuse & 5)) w += old[j];   // bytes <= 126 each
-            if (j < J - 1 || store_last) o[16 * j] = w;
-        }
-    }
-}
-
-// Fused variant for cost sums over all four frames: a kMT x kMT tile of pixels
-// needs the partner windows of every frame line through it (tile rows for
-// frames 0/180, tile columns for frames 90/270: 4 kMT lines of kMT + D - 1
-// codes) and 4 kMT^2 centre codes, staged in LDS, and writes M once -- no
-// read-modify-write of M between two launches.  That is 118.5 KB of LDS at
-// D = 192, so one block per CU: the blocks are persistent and load the next
-// tile's windows into registers while the current tile is summed.  Block b
-// takes tiles s(b), s(b) + n, s(b) + 2n, ... (n blocks); s groups the blocks
-// that share an XCD (b mod 8 under round-robin dispatch) on consecutive
-// tiles, so neighbouring tiles, whose row windows overlap, share an L2.  The
-// two-launch form covers the disparity counts beyond what one block can hold.
-// Per pixel as above: one wave per pixel, lane q owns d = q + 64 j.
-// ---------------------------------------------------------------------------
-constexpr int kMT = 16;
-
-// window line stride (entries) for J groups of 64 disparities: holds
-// kWinPad + kMT + D - 1 <= 64 J + 23 entries; a compile-time constant, so a
-// pixel's reads sit at immediate offsets from per-frame lane addresses
-template <int J>
-constexpr int msum_lstr() { return 64 * J + 24; }
-
-size_t msum_tile_lds(int Dp)
-{
-    const int J = (Dp + 63) / 64;
-    return ((size_t)4 * kMT * (64 * J + 24) + 4 * kMT * kMT) * 8 + kMT * kMT;
-}
-
-template <int J>
-__global__ __launch_bounds__(1024) void k_msum_tile(const RigDesc* __restrict__ rigs, int nrig,
-                                                    const int* __restrict__ bs, int ntiles, int fuse)
-{
-    static_assert(kMT == 16, "one wave per line of each frame, one thread per tile pixel below 256");
-    // a line holds kWinPad + kMT + D - 1 <= 64 J + 23 entries: J + 1 chunks of 64
-    constexpr int NK = J + 1;
-    extern __shared__ uint64_t lds64[];
-    const int D = rigs[0].D, Dp = rigs[0].Dp;   // one disparity count per launch
-    const int SPAN = kMT + D - 1;
-    constexpr int LSTR = msum_lstr<J>();
-    auto win = [&](int F, int l) { return lds64 + (F * kMT + l) * LSTR + kWinPad; };
-    uint64_t* CEN = lds64 + 4 * kMT * LSTR;     // [frame][pixel]
-    uint8_t* MB = (uint8_t*)(CEN + 4 * kMT * kMT);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int nb = gridDim.x, b = blockIdx.x;
-    int t = (nb & 7) == 0 ? (b & 7) * (nb >> 3) + (b >> 3) : b;
-
-    struct Geo { int ri, x0, y0; };
-    auto geo = [&](int tt) __attribute__((always_inline)) {
-        Geo q;
-        q.ri = find_rig(bs, nrig, tt);
-        const int ntx = (rigs[q.ri].Wp + kMT - 1) / kMT, lb = tt - bs[q.ri];
-        q.x0 = (lb % ntx) * kMT;
-        q.y0 = (lb / ntx) * kMT;
-        return q;
-    };
-    // Frame F pixel of image pixel (y, x) and the frame column of window
-    // entry 0 of the line through the tile:
-    //   F0: row y,        col x,         window from x0 - (D-1)
-    //   F2: row y,        col W'-1-x,    window from W' - x0 - kMT - (D-1)
-    //   F1: row W'-1-x,   col H'-1-y,    window from H' - y0 - kMT - (D-1)
-    //   F3: row W'-1-x,   col y,         window from y0 - (D-1)
-    // pc: centre codes; pk: mask bytes, read only at stash time, so that
-    // nothing waits for the loads while the current tile is summed
-    uint64_t pw[4][NK], pc[4];
-    uint32_t pk[4];
-    auto load = [&](const Geo& q) __attribute__((always_inline)) {
-        const RigDesc& g = rigs[q.ri];
-        const int Wp = g.Wp, Hp = g.Hp;
-#pragma unroll
-        for (int F = 0; F < 4; F++) {
-            const int l = wave;
-            const bool rowf = (F & 1) == 0;
-            const bool line_ok = rowf ? q.y0 + l < Hp : q.x0 + l < Wp;
-            const int frow = band_row(rowf ? q.y0 + l : Wp - 1 - (q.x0 + l), rowf ? Hp : Wp, D);   // stored row
-            const int fcols = rowf ? Wp : Hp;
-            const int lo = F == 0 ? q.x0 - (D - 1)
-                         : F == 2 ? Wp - q.x0 - kMT - (D - 1)
-                         : F == 1 ? Hp - q.y0 - kMT - (D - 1) : q.y0 - (D - 1);
-            const bool use = ((fuse >> F) & 1) && line_ok;
-            const uint64_t* N = g.code[2 * F + 1] + (size_t)(use ? frow : 0) * fcols;
-#pragma unroll
-            for (int kk = 0; kk < NK; kk++) {
-                const int k = lane - kWinPad + 64 * kk, col = lo + k;
-                pw[F][kk] = (use && k >= 0 && k < SPAN && col >= 0 && col < fcols) ? G(N)[col] : 0;
-            }
-        }
-        if (tid < kMT * kMT) {
-            const int y = q.y0 + tid / kMT, x = q.x0 + tid % kMT;
-            const bool in = y < Hp && x < Wp;
-#pragma unroll
-            for (int F = 0; F < 4; F++) {
-                const bool rowf = (F & 1) == 0;
-                const int frow = band_row(rowf ? y : Wp - 1 - x, rowf ? Hp : Wp, D);   // stored row
-                const int fcol = F == 0 ? x : F == 2 ? Wp - 1 - x : F == 1 ? Hp - 1 - y : y;
-                const int fcols = rowf ? Wp : Hp;
-                // a set mask implies frame column >= D; the check keeps indices in range
-                const bool use = in && ((fuse >> F) & 1) && fcol >= D;
-                pc[F] = use ? G(g.code[2 * F])[(size_t)frow * fcols + fcol] : 0;
-                pk[F] = use ? G(g.mask[F])[(size_t)y * Wp + x] : 0;
-            }
-        }
-    };
-    auto stash = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int F = 0; F < 4; F++) {
-            uint64_t* W = win(F, wave);
-#pragma unroll
-            for (int kk = 0; kk < NK; kk++) {
-                const int k = lane - kWinPad + 64 * kk;
-                if (k < SPAN) W[k] = pw[F][kk];
-            }
-        }
-        if (tid < kMT * kMT) {
-            uint32_t pm = 0;
-#pragma unroll
-            for (int F = 0; F < 4; F++) {
-                CEN[F * kMT * kMT + tid] = pc[F];
-                pm |= (pk[F] != 0 ? 1u : 0u) << F;
-            }
-            MB[tid] = (uint8_t)pm;
-        }
-    };
-    const int q = lane;
-    const int qlast = min(q, Dp - 1 - 64 * (J - 1));
-    const bool store_last = (q & ~3) + 64 * (J - 1) < Dp;
-    const bool live_last = q + 64 * (J - 1) < D;
-    // wave w walks tile column w, its 16 pixels fully unrolled: every read
-    // sits at a compile-time offset from one lane address per frame, so no
-    // address arithmetic runs per pixel.  Frame line and window index of
-    // pixel (ty, tx) at disparity d:
-    //   F0: line ty, index tx + D - 1 - d;         F2: line ty, index (kMT-1-tx) + D - 1 - d
-    //   F1: line tx, index (kMT-1-ty) + D - 1 - d; F3: line tx, index ty + D - 1 - d
-    auto sum_tile = [&](const Geo& gq) __attribute__((always_inline)) {
-        const RigDesc& g = rigs[gq.ri];
-        const int Wp = g.Wp, Hp = g.Hp;
-        const int tx = wave, x = gq.x0 + tx;
-        if (x >= Wp) return;
-        const uint32_t mcol = lane < kMT ? MB[lane * kMT + tx] : 0u;   // lane ty: mask bits of (ty, tx)
-        // group j of lane q reads entry base - q - 64 j: groups below J - 1 from
-        // pa + 64 (J - 1 - j), the last group (lanes past Dp read as qlast) from pl
-        const int lo = D - 1 - 64 * (J - 1);
-        const uint64_t* pa[4] = {win(0, 0) + tx + lo - q, win(1, tx) + lo - q,
-                                 win(2, 0) + (kMT - 1 - tx) + lo - q, win(3, tx) + lo - q};
-        const uint64_t* pl[4] = {win(0, 0) + tx + lo - qlast, win(1, tx) + lo - qlast,
-                                 win(2, 0) + (kMT - 1 - tx) + lo - qlast, win(3, tx) + lo - qlast};
-        const uint64_t* pc0 = CEN + tx;
-        const size_t rstride = (size_t)Wp * Dp;
-        gptr<uint8_t> o = G(g.msum) + ((size_t)gq.y0 * Wp + x) * Dp + (q & 3) * rstride + (q & ~3);
-        static_for<0, kMT / 4>([&](auto gc) __attribute__((always_inline)) {
-            constexpr int ty0 = 4 * decltype(gc)::value;
-            if (gq.y0 + ty0 >= Hp) return;                        // H' is a multiple of 4
-            unsigned acc[J][4];
-            static_for<0, 4>([&](auto tyc) __attribute__((always_inline)) {
-                constexpr int k = decltype(tyc)::value, ty = ty0 + k;
-                unsigned a[J];
-#pragma unroll
-                for (int j = 0; j < J; j++) a[j] = 0;
-                const int mb = __builtin_amdgcn_readlane(mcol, ty);   // one pixel per wave
-                static_for<0, 4>([&](auto kc) __attribute__((always_inline)) {
-                    constexpr int F = (0x3120 >> (4 * decltype(kc)::value)) & 15;   // frames 0, 2, 1, 3
-                    constexpr int off = F == 0 || F == 2 ? ty * LSTR : F == 1 ? kMT - 1 - ty : ty;
-                    if (!(mb & (1 << F))) return;
-                    uint64_t tv[J];
-#pragma unroll
-                    for (int j = 0; j < J - 1; j++) tv[j] = pa[F][off + 64 * (J - 1 - j)];
-                    tv[J - 1] = pl[F][off];
-                    const uint64_t cc = pc0[F * kMT * kMT + ty * kMT];
-#pragma unroll
-                    for (int j = 0; j < J; j++) {
-                        const uint64_t xv = cc ^ tv[j];
-                        a[j] = bcnt_add((uint32_t)(xv >> 32), bcnt_add((uint32_t)xv, a[j]));
-                    }
-                });
-                a[J - 1] = live_last ? a[J - 1] : 0u;
-#pragma unroll
-                for (int j = 0; j < J; j++) acc[j][k] = a[j];
-            });
-            gptr<uint32_t> op = (gptr<uint32_t>)(o + ty0 * rstride);
-#pragma unroll
-            for (int j = 0; j < J; j++) {
-                const uint32_t w = quad_bytes(acc[j], q);
-                if (j < J - 1 || store_last) op[16 * j] = w;
-            }
-        });
-    };
-    Geo cur = geo(t);
-    load(cur);
-    for (;;) {
-        stash();
-        __syncthreads();
-        const int tn = t + nb;
-        Geo nxt = cur;
-        if (tn < ntiles) {
-            nxt = geo(tn);
-            load(nxt);          // in flight while this tile is summed
-        }
-        sum_tile(cur);
-        if (tn >= ntiles) break;
-        __syncthreads();        // LDS free for the next stash
-        t = tn;
-        cur = nxt;
     }
 }
 
@@ -1607,35 +1241,12 @@ void launch_mask(const LaunchSet& ls, int fmask, hipStream_t st, KernelTimer* t)
     TE(kKMask);
 }
 
-size_t msum_lds(int D)
-{
-    return (size_t)(2 * kWinPad + 2 * (kRun + D - 1) + 2 * kRun) * 8 + kRun;
-}
-
-int msum_blocks(const RigDesc& g, int side)
-{
-    if (side == 2) return ((g.Wp + kMT - 1) / kMT) * ((g.Hp + kMT - 1) / kMT);
-    return side == 0 ? g.Hp * ((g.Wp + kRun - 1) / kRun) : g.Wp * ((g.Hp + kRun - 1) / kRun);
-}
-
-// at 5 groups (D > 256) the tile's windows need 184,576 bytes of LDS, over
-// the 160 KB a block can hold: those disparity counts take the two-launch form
-constexpr int kMsumTileMaxJ = 4;
-
 int kernels_setup(int device)
 {
     int v = 0;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess) return -1;
     const int lim = v;
     if (hipDeviceGetAttribute(&g_num_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return -1;
-    const void* fns[kMsumTileMaxJ] = {(const void*)k_msum_tile<1>, (const void*)k_msum_tile<2>,
-                                      (const void*)k_msum_tile<3>, (const void*)k_msum_tile<4>};
-    for (const void* f : fns)
-        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lim) != hipSuccess) {
-            (void)hipGetLastError();
-            g_lds_per_block = 0;   // fused cost sum off: the two-launch form runs
-            return 0;
-        }
     g_lds_per_block = (size_t)lim;
     if (median_setup(lim) != 0) {
         (void)hipGetLastError();
@@ -1662,70 +1273,6 @@ int kernels_setup(int device)
             return 0;
         }
     return 0;
-}
-
-// SISTER_MSUM_SPLIT=1 keeps the two-launch cost sum everywhere (comparison runs)
-static bool msum_split_forced()
-{
-    static const int v = [] {
-        const char* e = getenv("SISTER_MSUM_SPLIT");
-        return e && atoi(e) != 0 ? 1 : 0;
-    }();
-    return v != 0;
-}
-
-static bool msum_tile_fits(const DGroup& G)
-{
-    return (G.Dp + 63) / 64 <= kMsumTileMaxJ && msum_tile_lds(G.Dp) <= g_lds_per_block;
-}
-
-static void launch_msum_tile(const DGroup& G, int fuse, hipStream_t st)
-{
-    const size_t lds = msum_tile_lds(G.Dp);
-    const int ntiles = G.blocks[kGMsumTile];
-    const dim3 grid(std::min(ntiles, std::max(g_num_cu, 1))), block(1024);   // persistent, one per CU
-    const int* bs = G.bs[kGMsumTile];
-    switch ((G.Dp + 63) / 64) {
-    case 1: hipLaunchKernelGGL(k_msum_tile<1>, grid, block, lds, st, G.rigs, G.nrig, bs, ntiles, fuse); break;
-    case 2: hipLaunchKernelGGL(k_msum_tile<2>, grid, block, lds, st, G.rigs, G.nrig, bs, ntiles, fuse); break;
-    case 3: hipLaunchKernelGGL(k_msum_tile<3>, grid, block, lds, st, G.rigs, G.nrig, bs, ntiles, fuse); break;
-    default: hipLaunchKernelGGL(k_msum_tile<4>, grid, block, lds, st, G.rigs, G.nrig, bs, ntiles, fuse); break;
-    }
-}
-
-template <int SIDE>
-static void launch_msum_side(const DGroup& G, int fuse, hipStream_t st)
-{
-    const size_t lds = msum_lds(G.D);
-    const int k = kGMsumRows + SIDE;
-    const dim3 grid(G.blocks[k]), block(256);
-    switch ((G.Dp + 63) / 64) {
-    case 1: hipLaunchKernelGGL((k_msum_run<SIDE, 1>), grid, block, lds, st, G.rigs, G.nrig, G.bs[k], fuse); break;
-    case 2: hipLaunchKernelGGL((k_msum_run<SIDE, 2>), grid, block, lds, st, G.rigs, G.nrig, G.bs[k], fuse); break;
-    case 3: hipLaunchKernelGGL((k_msum_run<SIDE, 3>), grid, block, lds, st, G.rigs, G.nrig, G.bs[k], fuse); break;
-    case 4: hipLaunchKernelGGL((k_msum_run<SIDE, 4>), grid, block, lds, st, G.rigs, G.nrig, G.bs[k], fuse); break;
-    case 5: hipLaunchKernelGGL((k_msum_run<SIDE, 5>), grid, block, lds, st, G.rigs, G.nrig, G.bs[k], fuse); break;
-    case 6: hipLaunchKernelGGL((k_msum_run<SIDE, 6>), grid, block, lds, st, G.rigs, G.nrig, G.bs[k], fuse); break;
-    case 7: hipLaunchKernelGGL((k_msum_run<SIDE, 7>), grid, block, lds, st, G.rigs, G.nrig, G.bs[k], fuse); break;
-    default: hipLaunchKernelGGL((k_msum_run<SIDE, 8>), grid, block, lds, st, G.rigs, G.nrig, G.bs[k], fuse); break;
-    }
-}
-
-void launch_msum(const LaunchSet& ls, int fuse, hipStream_t st, KernelTimer* t)
-{
-    TB(kKMsum);
-    for (int gi = 0; gi < ls.ngroups; gi++) {
-        const DGroup& G = ls.groups[gi];
-        if ((fuse & 5) && (fuse & 10) && msum_tile_fits(G) && !G.msum_split && !msum_split_forced()) {
-            launch_msum_tile(G, fuse, st);                 // all frames, M written once
-            TD(kKMsum, 1);
-            continue;
-        }
-        if (fuse & 5) launch_msum_side<0>(G, fuse, st);    // frames 0/180 write M (zero when alone)
-        if (fuse & 10) launch_msum_side<1>(G, fuse, st);   // frames 90/270 add (or write when alone)
-        TD(kKMsum, ((fuse & 5) ? 1 : 0) + ((fuse & 10) ? 1 : 0));
-    }
-    TE(kKMsum);
 }
 
 // lanes per column of the fused sweep for D (0: beyond its reach, D > 384)

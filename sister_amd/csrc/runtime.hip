@@ -241,7 +241,7 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 struct GroupForm {
     int fused = -1;           // -1 automatic, 0 separate chains, 1 fused vertical sweep
     int kl[4] = {0, 0, 0, 0}; // a field of the forms file; chains always take 16 lanes
-    int msum_split = 0;       // 1: the two-launch cost sum
+    int msum_split = 0;       // a field of the forms file; the cost sum has one form per disparity count
     bool operator==(const GroupForm& o) const
     {
         return fused == o.fused && msum_split == o.msum_split && kl[0] == o.kl[0] && kl[1] == o.kl[1] &&
@@ -481,13 +481,13 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         p.host_rigs.push_back(g);
     }
     // SGM groups: runs of equal D
-    struct GroupHost { int i0, i1, vcols, maxHp, msum_split, join; };
+    struct GroupHost { int i0, i1, vcols, maxHp, join; };
     std::vector<GroupHost> groups;
     for (int k = 0; k < n;) {
         int e = k;
         long chains = 0;
         while (e < n && p.host_rigs[e].D == p.host_rigs[k].D) chains += p.host_rigs[e++].Wp;
-        GroupHost G{k, e, 0, 0, 0, 0};
+        GroupHost G{k, e, 0, 0, 0};
         for (int j = k; j < e; j++) G.maxHp = std::max(G.maxHp, p.host_rigs[j].Hp);
         const int D = p.host_rigs[k].D;
         GroupForm form;
@@ -495,7 +495,6 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         if (it != c->gforms.end()) form = it->second;
         // the debug switch wins over a tuned form
         G.vcols = vsweep_pick_cols(chains, D, c->vsweep >= 0 ? c->vsweep : form.fused);
-        G.msum_split = form.msum_split;
         long waves = 0;
         for (int j = k; j < e; j++)
             for (int f = 1; f < 4; f++) waves += path_waves(p.host_rigs[j].W, p.host_rigs[j].H, f);
@@ -585,7 +584,8 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
                 gbs[gpos + f * (ng + 1) + k] = tot[f];
                 tot[f] += f == kGPaths ? path_blocks(g, G.vcols > 0 ? 1 : 4, c->keep_sum)
                         : f == kGWinner ? winner_blocks(g, c->keep_sum)
-                        : f == kGVSweep ? vsweep_blocks(g, G.vcols) : msum_blocks(g, f - kGMsumRows);
+                        : f == kGVSweep ? vsweep_blocks(g, G.vcols)
+                        : f == kGCost ? cost_blocks(g) : msum_blocks(g, f - kGMsumRows);
             }
         }
         for (int f = 0; f < kNumGroupKernels; f++) gbs[gpos + f * (ng + 1) + ng] = tot[f];
@@ -625,7 +625,6 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         }
         sg.vcols = G.vcols;
         sg.maxHp = G.maxHp;
-        sg.msum_split = G.msum_split;
         sg.joined = G.join;
     }
     return SISTER_OK;
@@ -1266,7 +1265,7 @@ int sister_autotune(sister_ctx* c, const sister_rig* rigs, int n, int modes, con
         c->bforms[bk] = bestf;
     }
     // 2. each disparity group of those parts: vertical families fused or
-    // separate, cost-sum form (the other groups keep theirs)
+    // separate (the other groups keep theirs)
     std::vector<GroupKey> keys;
     {
         std::lock_guard<std::mutex> lk(c->mu);
@@ -1285,7 +1284,6 @@ int sister_autotune(sister_ctx* c, const sister_rig* rigs, int n, int modes, con
             f.fused = 1;
             cand.push_back(f);
         }
-        f = GroupForm(); f.msum_split = 1; cand.push_back(f);    // two-launch cost sum
         double best = 1e30;
         GroupForm bestf;
         for (const GroupForm& g : cand) {
