@@ -21,7 +21,6 @@ enum GroupKernel {
     kGPaths = 0,                          // SGM chains (ahead of the fused sweep: the rows family's)
     kGWinner,                             // S and the winner from the chains' bytes
     kGCost,                               // cost sum, per tile
-    kGMsumRows, kGMsumCols,               // cost sum, D > 256: row runs, column runs
     kGVSweep,                             // fused vertical SGM families, per column block
     kNumGroupKernels
 };
@@ -77,7 +76,6 @@ int winner_blocks(const RigDesc& g, bool whole);
 size_t path_state_total(int W, int H, int D, int f);
 int path_waves(int W, int H, int f);
 int cost_blocks(const RigDesc& g);
-int msum_blocks(const RigDesc& g, int side);   // side 0 row runs, 1 column runs
 int path_pairs(int Dp);   // pairs of disparities per lane (16 lanes) of the path and cost kernels
 // fused vertical sweep: owned columns per block for a group whose rigs have
 // `cols` padded columns in all and disparity count D (0: not used)

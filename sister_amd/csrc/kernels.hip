@@ -7,7 +7,7 @@
 //   median3x3_SSE in place postprocess.cpp:15-71        k_median (median.hip)
 //   doLRCheck + mask loops postprocess.cpp:318-341,     k_mask
 //                          hpp:201-251
-//   realign + weighted sum hpp:255-277                  k_cost, k_msum_run (cost.hip)
+//   realign + weighted sum hpp:255-277                  k_cost (cost.hip)
 //   accumulateCostsSSE     sgm.cpp:26-455               k_paths (paths.hip); batches: rows
 //                                                       in k_paths, the rest in k_vsweep
 //   WTALeft on S, convert  hpp:283,111-118              k_winner (paths.hip), or in k_vsweep

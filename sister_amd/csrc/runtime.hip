@@ -584,8 +584,7 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
                 gbs[gpos + f * (ng + 1) + k] = tot[f];
                 tot[f] += f == kGPaths ? path_blocks(g, G.vcols > 0 ? 1 : 4, c->keep_sum)
                         : f == kGWinner ? winner_blocks(g, c->keep_sum)
-                        : f == kGVSweep ? vsweep_blocks(g, G.vcols)
-                        : f == kGCost ? cost_blocks(g) : msum_blocks(g, f - kGMsumRows);
+                        : f == kGVSweep ? vsweep_blocks(g, G.vcols) : cost_blocks(g);
             }
         }
         for (int f = 0; f < kNumGroupKernels; f++) gbs[gpos + f * (ng + 1) + ng] = tot[f];

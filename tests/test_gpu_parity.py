@@ -341,13 +341,13 @@ def test_path_chains_outputs(gpu_ctx, oracle_mod, W, H, D, seed):
     assert float(np.abs(got["subpix"] - ref["subpix"]).max()) <= 1e-3
 
 
-# The cost sum: both tile sides (16 to D = 192, 8 to 256) and the runs past 256,
-# every number of pairs per lane, lanes partly and wholly past D, frames of
-# every remainder (0, 4, 8, 12 of 16) in both directions, with both frame pairs
+# The cost sum: every number of pairs per lane and of blocks to a tile, lanes
+# partly and wholly past D, frames of every remainder (0, 4, 8, 12 of 16) in both directions, with both frame pairs
 # (modes 1) and either alone.
 @pytest.mark.parametrize("W,H,D,seed", [
     (16, 8, 8, 121), (20, 4, 56, 122), (24, 28, 64, 123), (28, 20, 72, 124), (4, 12, 128, 125), (12, 16, 136, 126),
-    (20, 8, 192, 127), (8, 20, 200, 128), (12, 8, 256, 129), (8, 4, 264, 130)])
+    (20, 8, 192, 127), (8, 20, 200, 128), (12, 8, 256, 129), (8, 4, 264, 130),
+    (4, 8, 160, 131), (8, 8, 400, 132)])
 def test_cost_sum_tiles_bit_exact(gpu_ctx, oracle_mod, W, H, D, seed):
     for modes in (1, 2, 4):
         print(f"[parity cost] W={W} H={H} D={D} modes={modes} seed={seed}", flush=True)
