@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsister_hip.so")
-SOURCES = ["kernels.hip", "cost.hip", "median.hip", "paths.hip", "runtime.hip"]
+SOURCES = ["kernels.hip", "cost.hip", "median.hip", "paths.hip", "runtime.hip", "wta.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("SISTER_ARCH", "gfx950")
 

@@ -7,8 +7,8 @@ namespace sister {
 
 enum Stage {
     kStageCensus = 0,
-    kStageWta,          // all WTA blocks, or (row form) the rows of frames 0/2
-    kStageWtaV,         // row form: the rows of frames 1/3
+    kStageWta,          // WTA: the rows of frames 0/2
+    kStageWtaV,         // the rows of frames 1/3
     kStageWtaFill,      // the WTA maps' deep padding bands, copied from their first rows
     kStageMedianPrep,
     kStageMask,
@@ -47,7 +47,6 @@ struct LaunchSet {
     int maxCols;                    // max frame width over the rigs
     int med_waves;                  // waves per block of k_median
     int maxWp, maxHp;               // max padded width / height over the rigs
-    bool wta_rows;                  // WTA by frame rows from shared costs (k_wta_row)
     int ngroups;
     DGroup groups[kMaxDGroups];
 };
@@ -67,8 +66,9 @@ struct KernelTimer {
     long dispatched[kNumKernels] = {};   // kernel dispatches issued, per kernel
 };
 
-bool wta_rows_ok(int maxCols, int maxD);
-void stage_blocks(const RigDesc& g, int maxD, bool wta_rows, int out[kNumStages]);
+void stage_blocks(const RigDesc& g, int out[kNumStages]);
+int wta_fill_blocks(const RigDesc& g);
+int wta_setup(int lds_limit);
 // paths.hip: blocks of the chains of a rig's first nfam families (whole: over
 // the padded frame, debug sums) and of the winner
 int path_blocks(const RigDesc& g, int nfam, bool whole);

@@ -2,7 +2,7 @@
 //
 // Stage map (reference file:line -> kernel):
 //   censusTransform        census.cpp:38-51             k_census
-//   WTALeft/WTARight on    postprocess.cpp:74-315       k_wta   (cost recomputed from
+//   WTALeft/WTARight on    postprocess.cpp:74-315       k_wta (wta.hip; cost recomputed from
 //     the raw frame DSIs     (hpp:196-197,...)                   census, never stored)
 //   median3x3_SSE in place postprocess.cpp:15-71        k_median (median.hip)
 //   doLRCheck + mask loops postprocess.cpp:318-341,     k_mask
@@ -23,16 +23,6 @@
 #include "lanes.h"
 
 namespace sister {
-
-// Popcounts accumulate in place: v_bcnt_u32_b32 adds its second operand, one
-// instruction per 32-bit half (written out, since the compiler reassociates
-// pop + pop + acc into two plain popcounts and a three-way add).
-__device__ __forceinline__ unsigned bcnt_add(uint32_t x, unsigned acc)
-{
-    unsigned r;
-    asm("v_bcnt_u32_b32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(acc));
-    return r;
-}
 
 // padded original (y, x) of frame pixel (r, c)
 __device__ __forceinline__ void frame_to_orig(const RigDesc& g, int F, int r, int c, int& y, int& x)
@@ -69,29 +59,6 @@ __device__ __forceinline__ int frame_px(const RigDesc& g, const uint8_t* v, int 
     int y, x;
     frame_to_orig(g, F, r, c, y, x);
     return padded_px(g, v, y, x);
-}
-
-// cross-lane moves (DPP).  shr1: lane i gets lane i-1, lane 0 gets `fill`.
-// shl1: lane i gets lane i+1, lane 63 gets `fill`.
-__device__ __forceinline__ unsigned shr1(unsigned v, unsigned fill)
-{
-    return (unsigned)__builtin_amdgcn_update_dpp((int)fill, (int)v, 0x138, 0xF, 0xF, false);
-}
-__device__ __forceinline__ unsigned shl1(unsigned v, unsigned fill)
-{
-    return (unsigned)__builtin_amdgcn_update_dpp((int)fill, (int)v, 0x130, 0xF, 0xF, false);
-}
-
-// minimum over the 64 lanes, returned wave-uniform
-__device__ __forceinline__ unsigned wave_min(unsigned v)
-{
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x111, 0xF, 0xF, false));  // row_shr:1
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x112, 0xF, 0xF, false));  // row_shr:2
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x114, 0xF, 0xF, false));  // row_shr:4
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x118, 0xF, 0xF, false));  // row_shr:8
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xA, 0xF, false));  // row_bcast:15
-    v = min(v, (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xC, 0xF, false));  // row_bcast:31
-    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
 
 // ---------------------------------------------------------------------------
@@ -235,232 +202,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
         return;   // C is a multiple of 4, so a run is all in or all out
     }
     store_run(r0 + rl, c0 + 4 * run, code);
-}
-
-// ---------------------------------------------------------------------------
-// K2 WTALeft + WTARight of one frame's raw cost volume, costs recomputed from
-// census (census.cpp:81-82: popcount of the XOR; pairs with d > c are the
-// 255 entries and are never the minimum).
-//   L(r,c) = argmin_{d <= min(c,D-1)} pop(CC[r][c] ^ CN[r][c-d])   (postprocess.cpp:74-185)
-//   R(r,c) = argmin_{k <= min(D-1,C-1-c)} pop(CC[r][c+k] ^ CN[r][c]) (postprocess.cpp:187-315)
-// Lowest index wins ties: keys are (cost << 9) | d, reduced with min.
-// One block = one frame row segment of 256 pixels; codes staged in LDS.
-// ---------------------------------------------------------------------------
-// Rows of the deep padding bands other than a band's first row (band_row):
-// the WTA kernels compute the first row of each band and k_wta_fill copies it.
-__device__ __forceinline__ bool wta_band_copy(int r, int R, int D) { return band_row(r, R, D) != r; }
-
-__global__ __launch_bounds__(256) void k_wta(const RigDesc* __restrict__ rigs, int nrig,
-                                             const int* __restrict__ bs)
-{
-    extern __shared__ uint64_t lds64[];
-    const int ri = find_rig(bs, nrig, blockIdx.x);
-    const RigDesc& g = rigs[ri];
-    int lb = blockIdx.x - bs[ri];
-    const int D = g.D;
-    const int n02 = g.Hp * ((g.Wp + 255) / 256), n13 = g.Wp * ((g.Hp + 255) / 256);
-    int F;
-    if (lb < n02) F = 0;
-    else if ((lb -= n02) < n13) F = 1;
-    else if ((lb -= n13) < n02) F = 2;
-    else { lb -= n02; F = 3; }
-    const int R = frame_rows(g, F), C = frame_cols(g, F);
-    const int tilesC = (C + 255) / 256;
-    const int r = lb / tilesC, c0 = (lb % tilesC) * 256;
-    if (wta_band_copy(r, R, D)) return;   // copied from the band's first row
-    const uint64_t* cc = g.code[2 * F] + (size_t)r * C;
-    const uint64_t* cn = g.code[2 * F + 1] + (size_t)r * C;
-    const int n = 256 + D - 1;
-    uint64_t* cnS = lds64;        // cnS[i] = CN[c0 - D + 1 + i]
-    uint64_t* ccS = lds64 + n;    // ccS[i] = CC[c0 + i]
-    for (int i = threadIdx.x; i < n; i += 256) {
-        int a = c0 - D + 1 + i;
-        cnS[i] = (a >= 0 && a < C) ? cn[a] : 0;
-        int b = c0 + i;
-        ccS[i] = (b < C) ? cc[b] : 0;
-    }
-    __syncthreads();
-    const int tid = threadIdx.x;
-    const int c = c0 + tid;
-    if (c >= C) return;
-    const uint64_t myc = ccS[tid];
-    const uint64_t myn = cnS[tid + D - 1];
-    unsigned bestL = 0xFFFFFFFFu, bestR = 0xFFFFFFFFu;
-    const int lastL = min(c, D - 1);
-    for (int d = 0; d <= lastL; d++) {
-        unsigned key = ((unsigned)__popcll(myc ^ cnS[tid + D - 1 - d]) << 9) | (unsigned)d;
-        bestL = min(bestL, key);
-    }
-    const int lastR = min(D - 1, C - 1 - c);
-    for (int k = 0; k <= lastR; k++) {
-        unsigned key = ((unsigned)__popcll(ccS[tid + k] ^ myn) << 9) | (unsigned)k;
-        bestR = min(bestR, key);
-    }
-    g.wta[2 * F][(size_t)r * C + c] = (uint16_t)(bestL & 511u);
-    g.wta[2 * F + 1][(size_t)r * C + c] = (uint16_t)(bestR & 511u);
-}
-
-// WTALeft and WTARight of one frame row from shared costs (same results as
-// k_wta).  The right map's candidates for pixel p are cost(p + k, k), the
-// left map's for pixel c are cost(c, d): one cost serves both.  One block per
-// frame row, the row's codes in LDS; a wave takes 256-pixel segments, lane l
-// the 4 pixels c = x0 + 4l + i, and steps d = 0..D-1:
-//   w[i]  = CN[c_i - d]        partner codes: shift by one pixel per step,
-//                              one new LDS read per step for 4 costs
-//   key   = (pop(CC[c_i] ^ w[i]) << 9) | d        (lowest index wins ties)
-//   L[i]  = min(L[i], key)                         left map of pixel c_i
-//   R[i]  = min(R[i], key)                         right map of pixel c_i - d
-// kept as their complements ~key under max (one v_mad_i32_i24 forms ~key =
-// ~d - 512 pop), so that 0 is the neutral accumulator.
-// R[i] belongs to pixel x0 + 4l + i - d, so the right accumulators move one
-// pixel per step: R[3] of lane l becomes R[0] of lane l + 1 (DPP wave_shr:1,
-// whose zero fill is the fresh accumulator entering lane 0: one move).
-// Accumulators leaving lane 63, and all of them after the last step, are
-// partial results (their pixel's other candidates lie in neighbouring
-// segments): they meet by LDS atomic max, once per pixel and segment.  About
-// 3.6 VALU per evaluation against 6.
-// ---------------------------------------------------------------------------
-constexpr int kWtaRowMaxWaves = 16;
-
-size_t wta_row_lds(int C, int D)
-{
-    return ((size_t)C + (size_t)C + D - 1 + 256) * sizeof(uint64_t) + (size_t)C * sizeof(uint32_t);
-}
-
-// LFIX: a segment with pixels c < D - 1, whose left candidates d > c do not
-// exist: their keys are kept out of the left minima (the same costs feed the
-// right accumulators of pixels c - d < 0, which are dropped).  RFIX: a segment
-// reaching past the row: its pixels c >= C add 128 to their popcounts (the
-// popcount's addend), so their keys exceed every real one in the right minima
-// at no cost per step; their left results are not stored.
-template <bool LFIX, bool RFIX>
-__device__ __forceinline__ void wta_row_segment(const uint64_t* ccS, const uint64_t* cnS, uint32_t* RP,
-                                                uint16_t* outL, int x0, int C, int D, int lane)
-{
-    const int cb = x0 + 4 * lane;
-    uint64_t cci[4], w[4];
-    uint32_t bL[4], bR[4], ba[4];
-    const int32_t m512 = -512;   // a register: the mad's other operand is the scalar ~d
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        cci[i] = (!RFIX || cb + i < C) ? ccS[cb + i] : 0;
-        ba[i] = (RFIX && cb + i >= C) ? 128u : 0u;
-        w[i] = cnS[cb + i + D - 1];
-        bL[i] = 0u;
-        bR[i] = 0u;
-    }
-    auto step = [&](int d) __attribute__((always_inline)) {
-        const uint32_t nd = ~(uint32_t)d;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint64_t x = cci[i] ^ w[i];
-            const uint32_t pop = bcnt_add((uint32_t)(x >> 32), bcnt_add((uint32_t)x, ba[i]));
-            uint32_t nk;   // ~((pop << 9) | d) = ~d - 512 pop (pop <= 192)
-            asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(nk) : "v"(pop), "v"(m512), "s"(nd));
-            bL[i] = max(bL[i], (LFIX && d > cb + i) ? 0u : nk);
-            bR[i] = max(bR[i], nk);
-        }
-    };
-    auto shift = [&](int d) __attribute__((always_inline)) {
-        // to step d + 1: R accumulators move up one pixel (one lane per 4)
-        const uint32_t out = bR[3];
-        const uint32_t in = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)out, 0x138, 0xF, 0xF, true);
-        const int pl = x0 + 255 - d;          // pixel of lane 63's leaving accumulator
-        // interior segments: x0 + 256 <= C and x0 >= D - 1, so 0 <= pl < C; at
-        // the row's start pl < 0 once d > x0 + 255 (D > 256)
-        if (lane == 63 && (!LFIX || pl >= 0) && (!RFIX || pl < C)) atomicMax(&RP[pl], out);
-        bR[3] = bR[2]; bR[2] = bR[1]; bR[1] = bR[0]; bR[0] = in;
-        w[3] = w[2]; w[2] = w[1]; w[1] = w[0];
-        w[0] = cnS[cb + D - 2 - d];           // CN[cb - (d + 1)]
-    };
-    // four steps per iteration (the rotation of w and R repeats every four
-    // shifts, so the registers rename with no moves); D % 8 == 0, and the
-    // last quad, which has no final shift, is peeled
-    int d = 0;
-    for (; d + 4 < D; d += 4) {
-        step(d);     shift(d);
-        step(d + 1); shift(d + 1);
-        step(d + 2); shift(d + 2);
-        step(d + 3); shift(d + 3);
-    }
-    step(d);     shift(d);
-    step(d + 1); shift(d + 1);
-    step(d + 2); shift(d + 2);
-    step(d + 3);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if (!RFIX || cb + i < C) G(outL)[cb + i] = (uint16_t)(~bL[i] & 511u);
-        const int pp = cb + i - (D - 1);      // pixel of R[i] after the last step
-        if (pp >= 0 && pp < C) atomicMax(&RP[pp], bR[i]);
-    }
-}
-
-template <bool V>
-__global__ __launch_bounds__(64 * kWtaRowMaxWaves) void k_wta_row(const RigDesc* __restrict__ rigs, int nrig,
-                                                                 const int* __restrict__ bs)
-{
-    extern __shared__ uint64_t lds64[];
-    const int ri = find_rig(bs, nrig, blockIdx.x);
-    const RigDesc& g = rigs[ri];
-    const int lb = blockIdx.x - bs[ri];
-    const int D = g.D;
-    // V: frames 1 and 3 (W' rows of H' pixels), else frames 0 and 2 (H' rows of W')
-    const int nrow = V ? g.Wp : g.Hp, C = V ? g.Hp : g.Wp;
-    const int F = (V ? 1 : 0) + (lb >= nrow ? 2 : 0);
-    const int r = lb >= nrow ? lb - nrow : lb;
-    if (wta_band_copy(r, nrow, D)) return;   // copied from the band's first row
-    const uint64_t* cc = g.code[2 * F] + (size_t)r * C;
-    const uint64_t* cn = g.code[2 * F + 1] + (size_t)r * C;
-    uint64_t* ccS = lds64;                       // ccS[c] = CC[c]
-    uint64_t* cnS = lds64 + C;                   // cnS[i] = CN[i - (D - 1)], zero outside
-    uint32_t* RP = (uint32_t*)(cnS + C + D - 1 + 256);   // right-map partial keys
-    const int ncn = C + D - 1 + 256;
-    for (int i = threadIdx.x; i < ncn; i += blockDim.x) {
-        const int a = i - (D - 1);
-        cnS[i] = (a >= 0 && a < C) ? G(cn)[a] : 0;
-    }
-    for (int i = threadIdx.x; i < C; i += blockDim.x) {
-        ccS[i] = G(cc)[i];
-        RP[i] = 0u;   // complemented keys under max
-    }
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
-    const int nseg = (C + 255) >> 8;
-    uint16_t* const outL = g.wta[2 * F] + (size_t)r * C;
-    for (int sg = wave; sg < nseg; sg += nwaves) {
-        const int x0 = sg * 256;
-        // segments at the row's ends mask the candidates that do not exist
-        // (fewer than D at the start, pixels past the row at the end)
-        const bool lfix = x0 < D - 1, rfix = x0 + 256 > C;
-        if (lfix && rfix) wta_row_segment<true, true>(ccS, cnS, RP, outL, x0, C, D, lane);
-        else if (lfix) wta_row_segment<true, false>(ccS, cnS, RP, outL, x0, C, D, lane);
-        else if (rfix) wta_row_segment<false, true>(ccS, cnS, RP, outL, x0, C, D, lane);
-        else wta_row_segment<false, false>(ccS, cnS, RP, outL, x0, C, D, lane);
-    }
-    __syncthreads();
-    uint16_t* const outR = g.wta[2 * F + 1] + (size_t)r * C;
-    for (int p = threadIdx.x; p < C; p += blockDim.x) G(outR)[p] = (uint16_t)(~RP[p] & 511u);
-}
-
-// The WTA maps of the deep padding bands' rows from each band's first row:
-// one block per (map, band, 1024 columns), 4 columns per thread.
-constexpr int kWtaFillCols = 1024;
-__global__ __launch_bounds__(256) void k_wta_fill(const RigDesc* __restrict__ rigs, int nrig,
-                                                  const int* __restrict__ bs)
-{
-    const int ri = find_rig(bs, nrig, blockIdx.x);
-    const RigDesc& g = rigs[ri];
-    const int lb = blockIdx.x - bs[ri];
-    const int nch = (max(g.Wp, g.Hp) + kWtaFillCols - 1) / kWtaFillCols;
-    const int m = lb / (2 * nch), band = (lb / nch) & 1;
-    const int F = m >> 1;
-    const int R = frame_rows(g, F), C = frame_cols(g, F), D = g.D;
-    const int c = (lb % nch) * kWtaFillCols + 4 * (int)threadIdx.x;   // C % 4 == 0
-    if (c >= C) return;
-    const int lo = band ? R - D + 3 : 3, hi = band ? R - 4 : D - 4;
-    uint16_t* const map = g.wta[m];
-    const uint2 v = *(const uint2*)(map + (size_t)lo * C + c);
-    for (int r = lo + 1; r <= hi; r++) *(uint2*)(map + (size_t)r * C + c) = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -1206,30 +947,6 @@ void launch_census(const LaunchSet& ls, hipStream_t st, KernelTimer* t)
     TE(kKCensus);
 }
 
-void launch_wta(const LaunchSet& ls, hipStream_t st, KernelTimer* t)
-{
-    TB(kKWta);
-    if (ls.wta_rows) {
-        // frames 0/2 (rows of W' pixels), then frames 1/3 (rows of H')
-        const int waves02 = std::min(kWtaRowMaxWaves, (ls.maxWp + 255) / 256);
-        const int waves13 = std::min(kWtaRowMaxWaves, (ls.maxHp + 255) / 256);
-        hipLaunchKernelGGL(k_wta_row<false>, dim3(ls.blocks[kStageWta]), dim3(64 * waves02),
-                           wta_row_lds(ls.maxWp, ls.maxD), st, ls.rigs, ls.nrig, ls.bs[kStageWta]);
-        hipLaunchKernelGGL(k_wta_row<true>, dim3(ls.blocks[kStageWtaV]), dim3(64 * waves13),
-                           wta_row_lds(ls.maxHp, ls.maxD), st, ls.rigs, ls.nrig, ls.bs[kStageWtaV]);
-        TD(kKWta, 2);
-    } else {
-        size_t lds = (size_t)2 * (256 + ls.maxD - 1) * sizeof(uint64_t);
-        hipLaunchKernelGGL(k_wta, dim3(ls.blocks[kStageWta]), dim3(256), lds, st, ls.rigs, ls.nrig, ls.bs[kStageWta]);
-        TD(kKWta, 1);
-    }
-    // the deep padding bands' rows, copied from each band's first row
-    hipLaunchKernelGGL(k_wta_fill, dim3(ls.blocks[kStageWtaFill]), dim3(256), 0, st, ls.rigs, ls.nrig,
-                       ls.bs[kStageWtaFill]);
-    TD(kKWta, 1);
-    TE(kKWta);
-}
-
 static size_t g_lds_per_block = 0;   // set by kernels_setup
 int g_num_cu = 0;
 
@@ -1248,7 +965,7 @@ int kernels_setup(int device)
     const int lim = v;
     if (hipDeviceGetAttribute(&g_num_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return -1;
     g_lds_per_block = (size_t)lim;
-    if (median_setup(lim) != 0) {
+    if (wta_setup(lim) != 0 || median_setup(lim) != 0) {
         (void)hipGetLastError();
         return -1;
     }
@@ -1258,12 +975,6 @@ int kernels_setup(int device)
         (const void*)k_vsweep<2, 1, K, F, 4>, (const void*)k_vsweep<3, 1, K, F, 4>, \
         (const void*)k_vsweep<2, 0, K, F, 8>, (const void*)k_vsweep<3, 0, K, F, 8>, \
         (const void*)k_vsweep<2, 1, K, F, 8>, (const void*)k_vsweep<3, 1, K, F, 8>
-    for (const void* f : {(const void*)k_wta_row<false>, (const void*)k_wta_row<true>})
-        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lim) != hipSuccess) {
-            (void)hipGetLastError();
-            g_lds_per_block = 0;
-            return 0;
-        }
     const void* vfns[30] = {SISTER_VS_FNS(false, false), SISTER_VS_FNS(false, true), SISTER_VS_FNS(true, false)};
 #undef SISTER_VS_FNS
     for (const void* f : vfns)
@@ -1398,30 +1109,13 @@ void launch_sgm(const LaunchSet& ls, int mode, int keep_sum, hipStream_t st, Ker
 }
 
 // per-rig block counts of each stage (the host builds the block-start tables)
-bool wta_rows_ok(int maxCols, int maxD)
+void stage_blocks(const RigDesc& g, int out[kNumStages])
 {
-    // SISTER_WTA_ROWS=0 keeps the per-segment kernel (comparison runs)
-    static const int env = [] {
-        const char* e = getenv("SISTER_WTA_ROWS");
-        return e ? atoi(e) : -1;
-    }();
-    if (env == 0) return false;
-    return (maxCols + 255) / 256 <= 4 * kWtaRowMaxWaves && wta_row_lds(maxCols, maxD) <= g_lds_per_block;
-}
-
-void stage_blocks(const RigDesc& g, int maxD, bool wta_rows, int out[kNumStages])
-{
-    (void)maxD;
     const long npx = (long)g.Wp * g.Hp;
     out[kStageCensus] = 8 * ((g.Wp + kCT - 1) / kCT) * ((g.Hp + kCT - 1) / kCT);
-    if (wta_rows) {
-        out[kStageWta] = 2 * g.Hp;     // rows of frames 0 and 2
-        out[kStageWtaV] = 2 * g.Wp;    // rows of frames 1 and 3
-    } else {
-        out[kStageWta] = 2 * g.Hp * ((g.Wp + 255) / 256) + 2 * g.Wp * ((g.Hp + 255) / 256);
-        out[kStageWtaV] = 0;
-    }
-    out[kStageWtaFill] = 8 * 2 * ((std::max(g.Wp, g.Hp) + kWtaFillCols - 1) / kWtaFillCols);
+    out[kStageWta] = 2 * g.Hp;     // rows of frames 0 and 2
+    out[kStageWtaV] = 2 * g.Wp;    // rows of frames 1 and 3
+    out[kStageWtaFill] = wta_fill_blocks(g);
     out[kStageMedianPrep] = (int)(8 * ((npx / 2 + 255) / 256));
     out[kStageMask] = 4 * ((g.Wp + kMT32 - 1) / kMT32) * ((g.Hp + kMT32 - 1) / kMT32);
 }

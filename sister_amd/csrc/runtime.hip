@@ -562,10 +562,9 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
     int* gbs = (int*)(host.data() + rig_bytes + scr_bytes + bs_bytes);
     for (int k = 0; k < n; k++) scr[k] = (uint64_t*)(p.workspaces[k].ptr + lay[k].scratch);
     for (int st = 0; st < kNumStages; st++) p.ls.blocks[st] = 0;
-    const bool wta_rows = wta_rows_ok(maxCols, maxD);
     for (int k = 0; k < n; k++) {
         int nb[kNumStages];
-        stage_blocks(p.host_rigs[k], maxD, wta_rows, nb);
+        stage_blocks(p.host_rigs[k], nb);
         for (int st = 0; st < kNumStages; st++) {
             bs[st * (n + 1) + k] = p.ls.blocks[st];
             p.ls.blocks[st] += nb[st];
@@ -599,7 +598,6 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         p.ls.bs[st] = (const int*)(p.table.ptr + rig_bytes + scr_bytes) + st * (n + 1);
     p.ls.maxD = maxD;
     p.ls.maxCols = maxCols;
-    p.ls.wta_rows = wta_rows;
     p.ls.maxWp = 8;
     p.ls.maxHp = 8;
     p.ls.med_waves = 0;

@@ -355,3 +355,15 @@ def test_cost_sum_tiles_bit_exact(gpu_ctx, oracle_mod, W, H, D, seed):
         # frames that a single pair mode does not use are not computed
         bad = [b for b in bad if modes == 1 or b[0] not in ("census", "wta", "med", "mask")]
         assert not bad, (modes, bad)
+
+
+# The WTA maps: frame rows below, at and past one and several blocks' steps (64
+# pixels a wave, 4 or 8 waves), row ends inside a wave's 64 pixels and a 16-pixel
+# tile, D below the four-tile rule, at it, and with its last tile half full.
+@pytest.mark.parametrize("W,H,D,seed", [
+    (48, 4, 8, 141), (28, 100, 56, 142), (128, 64, 64, 143), (132, 60, 64, 144), (184, 4, 72, 145), (384, 8, 64, 146),
+    (260, 12, 200, 147), (20, 256, 192, 148), (4, 8, 384, 149), (136, 4, 440, 150)])
+def test_wta_rows_bit_exact(gpu_ctx, oracle_mod, W, H, D, seed):
+    print(f"[parity wta] W={W} H={H} D={D} seed={seed}", flush=True)
+    bad = _compare_stages(gpu_ctx, oracle_mod, W, H, D, seed, modes=1)
+    assert not bad, bad
