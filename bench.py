@@ -60,34 +60,27 @@ OPS_PER_CELL_PIPELINE = 97        # mode 0: costs 20, LR-check argmins 8, weight
 # kernel: 4 directional costs (xor 2 + popcount 2 + invalid select 1 each = 20)
 # and the 8 LR-check argmins live in `wta`; the mask-weighted sum is 4; each
 # SGM path is 8 (+P1, min d-1, min d+1, min P2 term, -minL, +C, running min,
-# +S) and each chain-family kernel sweeps two paths; the final argmin (1) is
-# fused into sgm_anti.  Total 28 + 4 + 3*16 + 17 = 97.
-OPS_PER_CELL = {"wta": 28, "msum": 4, "sgm_rows": 16, "sgm_cols": 16, "sgm_diag": 16, "sgm_anti": 17,
+# +S); the final argmin is 1.  Total 28 + 4 + 8*8 + 1 = 97.
+OPS_PER_CELL = {"wta": 28, "msum": 4, "sgm_rows": 16, "sgm_paths": 64, "winner": 1,
                 "sgm_vsweep": 49}   # the fused vertical sweep: 3 families x 2 sweeps x 8, + argmin
 
 # Algorithmic HBM bytes per padded cell of the HBM-bound kernels, with
 # `crop` the fraction of padded cells inside the crop (W*H of W'*H'): the
 # intermediates whose only reader is the final aggregate S are moved for those
-# cells alone, since S is read at the crop only.  Each separate SGM chain
-# family reads the u8 cost M in both sweeps (2), writes its forward (L - M)
-# byte (1), reads it back and writes the two-direction sum (2): 5.  The
-# anti-diagonal family, which forms S and the winner, instead reads the three
-# other families' bytes (3) and writes nothing in its backward sweep: 7.  The
-# rows family sweeps its two directions as separate waves, each reading M (2),
-# and stores one byte per direction at crop cells (2 crop).  The fused
-# vertical sweep (columns, diagonals, anti-diagonals together) reads M going
-# down and again going up (2) and, at crop cells, the rows family's two bytes
-# (2), the u16 partial sum P written going down (2) and read going up (2):
-# 2 + 6 crop (against 5 + 5 + 7 for the three separate families).  The cost
-# sum over 16x16 tiles writes M once (1); its two-launch form (frames 0/180,
-# then 90/270 read-modify-write) moves 3.
+# cells alone, since S is read at the crop only.  The rows family ahead of the
+# fused sweep runs joined, reading M forward and again backward (2) and storing
+# one byte at crop cells (crop).  The fused vertical sweep (columns, diagonals,
+# anti-diagonals together) reads M going down and again going up (2) and, at
+# crop cells, the rows family's byte (1), the u16 partial sum P written going
+# down (2) and read going up (2): 2 + 5 crop.  The cost sum writes M once (1).
+# (The chains of smaller batches, sgm_paths, have forms that differ by group
+# and carry no figure here.)
 def bytes_per_cell(kernel, crop):
-    fixed = {"sgm_cols": 5, "sgm_diag": 5, "sgm_anti": 7, "msum": 1}
     if kernel == "sgm_rows":
-        return 2 + 2 * crop
+        return 2 + crop
     if kernel == "sgm_vsweep":
-        return 2 + 6 * crop
-    return fixed.get(kernel)
+        return 2 + 5 * crop
+    return {"msum": 1}.get(kernel)
 
 
 # per-kernel counter totals of one instrumented step (used when their batch
