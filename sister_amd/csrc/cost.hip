@@ -32,11 +32,11 @@ namespace sister {
 // lane's disparities straddle Dp), and past that as many blocks to a tile, of
 // 128 each, as Dp needs.  Wider lanes spend fewer steps on the same cells, but
 // their windows' registers leave fewer waves, and they lose wherever 128 serve
-// (padded 1920x1080, one launch: D=160 1.60 ms against 2.05 with 16 disparities
-// a lane, D=256 1.99 / 2.63, D=264 2.91 / 4.75; D=192 is 1.45 with 12 a lane
-// and would be 1.7 as two blocks).  A block per row or column run with a pixel
-// per wave and its windows in LDS took 3.37 ms at D=264, 4.62 against 3.63 (3.84
-// with 12 a lane) at D=384, 7.06 against 5.85 at D=512.
+// (1920x1080 rigs: D=160 0.53 ms against 0.68 with 16 disparities a lane, D=256
+// 0.66 / 0.88, D=264 0.97 / 1.58; D=192 is 0.48 with 12 a lane and would be
+// 0.57 as two blocks).  A block per row or column run with a pixel per wave and
+// its windows in LDS took 1.12 ms at D=264, 1.54 against 1.21 (1.28 with 12 a
+// lane) at D=384, 2.35 against 1.95 at D=512.
 constexpr int kCostTile = 16;
 static int cost_pairs(int Dp) { return Dp <= 64 ? 2 : Dp > 128 && Dp <= 192 && Dp % 12 == 0 ? 6 : 4; }
 static int cost_parts(int Dp) { return (Dp + 32 * cost_pairs(Dp) - 1) / (32 * cost_pairs(Dp)); }

@@ -76,7 +76,7 @@ int winner_blocks(const RigDesc& g, bool whole);
 size_t path_state_total(int W, int H, int D, int f);
 int path_waves(int W, int H, int f);
 int cost_blocks(const RigDesc& g);
-int path_pairs(int Dp);   // pairs of disparities per lane (16 lanes) of the path and cost kernels
+int path_pairs(int Dp);   // pairs of disparities per lane (16 lanes) of the path kernels
 // fused vertical sweep: owned columns per block for a group whose rigs have
 // `cols` padded columns in all and disparity count D (0: not used)
 int vsweep_pick_cols(long cols, int D, int choice);
