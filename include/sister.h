@@ -12,7 +12,8 @@
  * Plain C: pointers and sizes only.  Every call returns a status code
  * (SISTER_OK = 0); sister_last_error() describes the last failure.  No C++
  * exception crosses this boundary.  A context is not thread safe: use one per
- * host thread, or serialise calls.
+ * host thread, or serialise calls.  sister_compute_rig does so by itself:
+ * threads that share a context (the class's default one) take turns in it.
  *
  * Images are 8-bit gray, W x H with a row stride in bytes.  W and H must be
  * multiples of 4 and D a multiple of 8 with 8 <= D <= 512 (the reference's own

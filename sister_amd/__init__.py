@@ -131,7 +131,8 @@ def bgr_to_gray(img):
 
 
 class Context:
-    """One device context (stream, HBM pool).  Not thread safe."""
+    """One device context (stream, HBM pool).  Not thread safe, apart from
+    compute_rig: threads that share a context take turns in it."""
 
     def __init__(self, device=0, hbm_budget=0):
         cfg = ConfigStruct(device, 0, hbm_budget)

@@ -338,7 +338,13 @@ struct sister_ctx {
         hipEvent_t done;
     };
     PinnedPool pinned;
-    // pinned staging of sister_compute_rig, kept between calls up to kStageKeep
+    // sister_compute_rig: one call at a time on a context (host_mu, taken before
+    // mu), so that threads which share it, as callers of the class do, each have
+    // the staging and its events for the whole of their call.  The stream put
+    // their work in a row anyway.
+    std::mutex host_mu;
+    hipEvent_t ev_host[2] = {};
+    // its pinned staging, kept between calls up to kStageKeep
     char* stage = nullptr;
     size_t stage_bytes = 0;
     static constexpr size_t kStageKeep = (size_t)256 << 20;
@@ -728,6 +734,7 @@ int sister_create(const sister_config* cfg, sister_ctx** out)
              hipEventCreateWithFlags(&c->ev_join[k], hipEventDisableTiming) == hipSuccess;
     for (int k = 0; ok && k < sister_ctx::kMaxParts; k++)
         ok = hipEventCreateWithFlags(&c->ev_stage[k], hipEventDisableTiming) == hipSuccess;
+    for (hipEvent_t& e : c->ev_host) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     ok = ok && kernels_setup(c->device) == 0;
     // a failed look-up leaves the allocation-free entry point reporting it
     if (ok) c->scratch = scratch_address(c->device);
@@ -761,6 +768,7 @@ void sister_destroy(sister_ctx* c)
     c->pinned.release_all();
     if (c->stage) (void)hipHostFree(c->stage);
     (void)hipEventDestroy(c->ev_fork);
+    for (hipEvent_t e : c->ev_host) (void)hipEventDestroy(e);
     for (int k = 0; k < sister_ctx::kMaxParts; k++) {
         if (c->ev_stage[k]) (void)hipEventDestroy(c->ev_stage[k]);
         if (k == 0) continue;   // part 0 runs on the context stream
@@ -879,6 +887,7 @@ int sister_compute_rig(sister_ctx* c, const sister_rig* r, int modes)
         if (!r->view[v]) return fail(c, SISTER_EINVAL, "null view");
     const size_t WH = (size_t)r->width * r->height, view_b = align_up(WH), map_b = align_up(WH * 2);
     const size_t bytes = io_bytes(WH);
+    std::lock_guard<std::mutex> call(c->host_mu);
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipStreamSynchronize(c->stream));   // the previous plan and staging may still be in use
     if (c->stage_bytes < bytes) {
@@ -946,7 +955,7 @@ int sister_compute_rig(sister_ctx* c, const sister_rig* r, int modes)
             if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
             for (size_t k = 0; k < outs.size() && e == hipSuccess; k++) unpack(outs[k]);
         } else {
-            hipEvent_t ev[2] = {c->ev_fork, c->ev_stage[0]};
+            const hipEvent_t* const ev = c->ev_host;
             for (size_t k = 0; k <= outs.size() && e == hipSuccess; k++) {
                 if (k < outs.size()) {
                     e = hipMemcpyAsync(hs + outs[k].off, io.ptr + outs[k].off, outs[k].bytes, hipMemcpyDeviceToHost, c->stream);

@@ -1,0 +1,108 @@
+// Drives the library's host code over the CPU stand-in of host_hip.cpp.
+//   host_calls_check NAME     runs one check; prints "ok"
+#include <cstdio>
+#include <cstring>
+#include <string>
+#include <thread>
+#include <vector>
+
+#include "../../include/sister.h"
+#include "host_hip.h"
+
+#define CHECK(c)                                                   \
+    do {                                                           \
+        if (!(c)) {                                                \
+            std::printf("FAIL %s line %d\n", #c, __LINE__);        \
+            std::fflush(stdout);                                   \
+            std::_Exit(1);                                         \
+        }                                                          \
+    } while (0)
+
+namespace {
+
+// a rig in host memory with views of `seed`, and its outputs
+struct Rig {
+    int W, H, D;
+    std::vector<uint8_t> view[5];
+    std::vector<uint16_t> out[3], disp;
+    std::vector<float> sub;
+    sister_rig r;
+    Rig(int w, int h, int d, unsigned seed) : W(w), H(h), D(d)
+    {
+        std::memset(&r, 0, sizeof r);
+        r.width = W; r.height = H; r.stride = W; r.disp_count = D;
+        for (int i = 0; i < 5; i++) {
+            view[i].resize((size_t)W * H);
+            for (auto& b : view[i]) b = (uint8_t)((seed = seed * 1664525u + 1013904223u) >> 24);
+            r.view[i] = view[i].data();
+        }
+        for (auto& o : out) o.resize((size_t)W * H);
+        disp.resize((size_t)W * H);
+        sub.resize((size_t)W * H);
+        r.out_multiview = out[0].data();
+        r.out_horizontal = out[1].data();
+        r.out_vertical = out[2].data();
+        r.out_disp = disp.data();
+        r.out_subpix = sub.data();
+    }
+    void clear()
+    {
+        for (auto& o : out) std::fill(o.begin(), o.end(), 0xFFFF);
+        std::fill(disp.begin(), disp.end(), 0xFFFF);
+        std::fill(sub.begin(), sub.end(), -1.f);
+    }
+    bool right(int modes) const
+    {
+        for (size_t p = 0; p < disp.size(); p++) {
+            int v = 0;
+            for (int i = 0; i < 5; i++) v += (i + 1) * view[i][p];
+            for (int m = 0; m < 3; m++)
+                if ((modes >> m & 1) && out[m][p] != (uint16_t)host_hip::map_value(v, m)) return false;
+            if ((modes & 1) && (disp[p] != v || sub[p] != (float)v)) return false;
+        }
+        return true;
+    }
+};
+
+sister_ctx* create(size_t budget = 0)
+{
+    sister_config cfg{0, 0, budget};
+    sister_ctx* c = nullptr;
+    CHECK(sister_create(&cfg, &c) == SISTER_OK);
+    return c;
+}
+
+// Threads that compute rigs of different sizes (one copy for all views, a copy
+// per view, a staging that has to grow) on one context, as callers of the class
+// with its shared context do: each gets its own maps.
+void host_form_threads()
+{
+    host_hip::step_us = 100;
+    sister_ctx* c = create();
+    const int dims[3][3] = {{64, 48, 16}, {640, 480, 64}, {320, 240, 32}};
+    std::vector<std::thread> th;
+    for (int k = 0; k < 3; k++)
+        th.emplace_back([=] {
+            Rig r(dims[k][0], dims[k][1], dims[k][2], 10u + k);
+            const int modes = k == 2 ? 1 : 7;
+            for (int i = 0; i < 12; i++) {
+                r.clear();
+                CHECK(sister_compute_rig(c, &r.r, modes) == SISTER_OK);
+                CHECK(r.right(modes));
+            }
+        });
+    for (auto& t : th) t.join();
+    sister_destroy(c);
+    CHECK(host_hip::pinned_bytes == 0);
+}
+
+}  // namespace
+
+int main(int argc, char** argv)
+{
+    const std::string name = argc > 1 ? argv[1] : "";
+    if (name == "host_form_threads") host_form_threads();
+    else return 2;
+    std::printf("ok\n");
+    return 0;
+}
