@@ -302,6 +302,7 @@ struct sister_ctx {
     int vsweep = -1;              // vertical SGM families: -1 automatic, 0 separate, 1 fused
     bool p_in_place = false;      // debug: every plan keeps the fused sweep's P in place
     Plan last;                 // plan of the last sister_run_device (kept for debug fetch)
+    uint64_t issued = 0;       // plans that `last` has held (under mu)
     Plan noalloc;              // plan of the last sister_run_device_noalloc (in the scratch array)
     std::map<GroupKey, GroupForm> gforms;   // autotuned group forms (under mu)
     std::map<BatchKey, BatchForm> bforms;   // autotuned batch forms (under mu)
@@ -807,6 +808,7 @@ int sister_outside_reference_domain(int D) { return D > 256 ? 1 : 0; }
 static int run_batch(sister_ctx* c, const sister_rig* rigs, int n, int modes)
 {
     free_plan(c, c->last);
+    c->issued++;
     const int rc = build_plan_compact(c, rigs, n, c->last);
     if (rc) return rc;
     enqueue(c, c->last, modes, c->stream, c->profiling ? &c->timer : nullptr);
@@ -889,7 +891,6 @@ int sister_compute_rig(sister_ctx* c, const sister_rig* r, int modes)
     const size_t bytes = io_bytes(WH);
     std::lock_guard<std::mutex> call(c->host_mu);
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, hipStreamSynchronize(c->stream));   // the previous plan and staging may still be in use
     if (c->stage_bytes < bytes) {
         if (c->stage) (void)hipHostFree(c->stage);
         c->stage = nullptr;
@@ -903,8 +904,11 @@ int sister_compute_rig(sister_ctx* c, const sister_rig* r, int modes)
     }
     char* const hs = c->stage;   // null: the copies run on the caller's buffers
     Block io;
+    uint64_t seen;
     {
         std::lock_guard<std::mutex> lk(c->mu);
+        HIPCHK(c, hipStreamSynchronize(c->stream));   // the previous plan may still be in use
+        seen = c->issued;
         if (c->pool.get(bytes, io) != 0) return fail(c, SISTER_ENOMEM, "staging allocation failed");
     }
     hipError_t e = hipSuccess;
@@ -937,7 +941,9 @@ int sister_compute_rig(sister_ctx* c, const sister_rig* r, int modes)
     d.out_subpix = (float*)dev(4);
     if (e == hipSuccess) {
         std::lock_guard<std::mutex> lk(c->mu);
-        rc = run_batch(c, &d, 1, modes);
+        // another thread's batch since then: its plan is in use
+        if (c->issued != seen) e = hipStreamSynchronize(c->stream);
+        if (e == hipSuccess) rc = run_batch(c, &d, 1, modes);
     }
     if (rc == SISTER_OK && e == hipSuccess) {
         std::vector<Out> outs;
