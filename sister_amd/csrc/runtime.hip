@@ -891,6 +891,15 @@ int sister_compute_rig(sister_ctx* c, const sister_rig* r, int modes)
     const size_t bytes = io_bytes(WH);
     std::lock_guard<std::mutex> call(c->host_mu);
     HIPCHK(c, hipSetDevice(c->device));
+    Block io;
+    uint64_t seen;
+    {
+        std::lock_guard<std::mutex> lk(c->mu);
+        HIPCHK(c, hipStreamSynchronize(c->stream));   // the previous plan may still be in use
+        seen = c->issued;
+        if (c->pool.get(bytes, io) != 0) return fail(c, SISTER_ENOMEM, "staging allocation failed");
+    }
+    // from here on the call ends below, where a large staging is given back
     if (c->stage_bytes < bytes) {
         if (c->stage) (void)hipHostFree(c->stage);
         c->stage = nullptr;
@@ -903,14 +912,6 @@ int sister_compute_rig(sister_ctx* c, const sister_rig* r, int modes)
         }
     }
     char* const hs = c->stage;   // null: the copies run on the caller's buffers
-    Block io;
-    uint64_t seen;
-    {
-        std::lock_guard<std::mutex> lk(c->mu);
-        HIPCHK(c, hipStreamSynchronize(c->stream));   // the previous plan may still be in use
-        seen = c->issued;
-        if (c->pool.get(bytes, io) != 0) return fail(c, SISTER_ENOMEM, "staging allocation failed");
-    }
     hipError_t e = hipSuccess;
     sister_rig d = *r;
     d.stride = r->width;

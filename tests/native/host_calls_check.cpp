@@ -127,6 +127,20 @@ void host_form_beside_batches()
     sister_destroy(c);
 }
 
+// A rig whose staging is too large to keep and whose device block cannot be
+// had: refused, and nothing pinned stays behind.
+void host_form_refused()
+{
+    sister_ctx* c = create((size_t)64 << 20);
+    Rig r(4096, 4096, 8, 5);
+    CHECK(sister_compute_rig(c, &r.r, 1) == SISTER_ENOMEM);
+    CHECK(host_hip::pinned_bytes == 0);
+    Rig s(64, 48, 16, 6);
+    CHECK(sister_compute_rig(c, &s.r, 7) == SISTER_OK && s.right(7));
+    sister_destroy(c);
+    CHECK(host_hip::pinned_bytes == 0);
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -134,6 +148,7 @@ int main(int argc, char** argv)
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "host_form_threads") host_form_threads();
     else if (name == "host_form_beside_batches") host_form_beside_batches();
+    else if (name == "host_form_refused") host_form_refused();
     else return 2;
     std::printf("ok\n");
     return 0;
