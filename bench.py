@@ -7,7 +7,8 @@ inputs and outputs resident in HBM before the timed region:
 
   plain    one rig per call of the library (sister_run_device with n = 1),
   batched  B rigs in one plan (default 64: 229 GB of workspace), captured
-           once as a hipGraph and replayed.
+           once as a hipGraph in the automatic launch forms (or those of a
+           file, --forms) and replayed.
 
 `value` is the batched throughput in G disparity-evals/s (sum of W*H*D over
 the rigs of a step / step time); the plain figures and the ratio sit beside
@@ -316,6 +317,14 @@ def roofline_entry(kern, launches, cells, step_ms, B, workload, crop, wta_copied
     return roof
 
 
+def capture(ctx, structs, args):
+    """The batch in one graph: in the forms of --forms, or the automatic ones."""
+    if args.forms:
+        ctx.autotune(structs, 1, args.forms)
+    else:
+        ctx.graph_capture(structs, 1)
+
+
 def time_graph(ctx, args, torch):
     """Replays of the context's captured graph: warm-up, then the timed steps."""
     for _ in range(args.warmup):
@@ -363,24 +372,13 @@ def run(args):
     ctx.sync()
 
     # ---- batched: all B rigs in one captured plan ----------------------------
-    # first in the default launch forms, then in the forms the autotuner picks
-    # for this batch (graph parts; per disparity group the SGM and cost-sum
-    # forms), which is what is reported
+    # in the automatic launch forms, or those of --forms
     for d in dev:
         d["outs"]["disp"].zero_()
         d["outs"]["multiview"].zero_()
-    structs = [d["struct"] for d in dev]
-    ctx.graph_capture(structs, 1)
-    default_ms = time_graph(ctx, args, torch)
-    log(f"batched, default forms: {default_ms:.2f} ms per step")
-    t0 = time.perf_counter()
-    ctx.autotune(structs, 1)
-    tune_s = time.perf_counter() - t0
-    for d in dev:
-        d["outs"]["disp"].zero_()
-        d["outs"]["multiview"].zero_()
+    capture(ctx, [d["struct"] for d in dev], args)
     step_ms = time_graph(ctx, args, torch)
-    log(f"batched, tuned forms: {step_ms:.2f} ms per step (tuning {tune_s:.1f} s)")
+    log(f"batched: {step_ms:.2f} ms per step")
     batched_out = [{k: d["outs"][k].clone() for k in ("disp", "multiview")} for d in dev]
 
     # ---- plain: one rig per call, timed right after the batched steps -------
@@ -433,9 +431,7 @@ def run(args):
         "plain": {"ms_per_rig": plain_ms, "rigs_per_s": 1e3 / plain_ms,
                   "value": plain_evals / (plain_ms * 1e-3) / 1e9},
         "batched_vs_plain": (B / step_ms) / (1.0 / plain_ms),
-        "default_forms_ms_per_step": default_ms,
-        "autotune": {"seconds": tune_s, "forms": ctx.tune_table().strip().splitlines()[1:],
-                     "note": "kernel_ms comes from eager steps in the default forms"},
+        "forms": ctx.tune_table().strip().splitlines()[1:],   # none: the automatic ones
         "batched_equals_plain": not bad,
         "batched_mismatched_rigs": len(bad),
         "batched_compared": f"disp and multiview maps of all {B} rigs against their scene computed alone",
@@ -474,12 +470,7 @@ def run_mixed(args):
         ctx.run_device([d["struct"]], 1)
         ctx.sync()
         alone.append(d["outs"]["disp"].clone())
-    ctx.graph_capture(structs, 1)
-    default_ms = time_graph(ctx, args, torch)
-    log(f"mixed32, default forms: {default_ms:.2f} ms per step")
-    t0 = time.perf_counter()
-    ctx.autotune(structs, 1)
-    tune_s = time.perf_counter() - t0
+    capture(ctx, structs, args)
     for d in dev:
         d["outs"]["disp"].zero_()
     step_ms = time_graph(ctx, args, torch)
@@ -488,13 +479,13 @@ def run_mixed(args):
     ctx.close()
     del dev
     torch.cuda.empty_cache()
-    log(f"mixed32, tuned forms: {step_ms:.2f} ms per step (tuning {tune_s:.1f} s)")
+    log(f"mixed32: {step_ms:.2f} ms per step")
     return {"workload": "32 rigs, sizes uniform over {640x480, 1280x720, 1920x1080, 2048x1536}, D uniform over "
                         "{64, 128, 192, 256} (seed 1000), one hipGraph",
             "ms_per_step": step_ms, "rigs_per_s": 32 / (step_ms * 1e-3),
             "value": evals / (step_ms * 1e-3) / 1e9, "unit": "G disparity-evals/s",
             "padded_cells_per_s": cells / (step_ms * 1e-3), "steps": args.steps,
-            "default_forms_ms_per_step": default_ms, "autotune_seconds": tune_s, "forms": forms,
+            "forms": forms,
             "rigs_differing_from_alone": bad}
 
 
@@ -635,6 +626,7 @@ def main():
     ap.add_argument("--workload", default="rig1080", choices=["rig1080", "mixed32", "large", "serve"])
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-extra", action="store_true", help="headline only (no mixed32 / serve blocks)")
+    ap.add_argument("--forms", help="launch-forms file that names the batch's shapes (default: the automatic forms)")
     ap.add_argument("--rate", type=float, default=200.0)
     ap.add_argument("--serve-seconds", type=float, default=10.0)
     ap.add_argument("--serve-host", action="store_true", help="serve host buffers instead of device-resident ones")

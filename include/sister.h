@@ -120,19 +120,20 @@ int sister_graph_launch(sister_ctx* ctx);
 
 /* ---- autotuning ----------------------------------------------------------- */
 /* No counterpart in the reference (its launch shapes are fixed by its SSE
-   loops).  Times on the device, as a captured graph of this batch, the launch
-   forms that leave results unchanged: first the graph's parts (1 to 4 parts
-   balanced by padded cells, or one part per disparity count, so that groups
-   of different D run side by side, and the parts started together or each
-   after the previous part's first stages), then for each disparity group of those
-   parts the SGM vertical families fused or separate.  The fastest of
-   each is kept in the context's table, which every later plan and capture
-   of a matching shape consults: groups are matched by D and the half-octaves
-   of their padded column total and tallest padded rig, batches by rig count,
-   distinct D count, half-octave of padded cells and modes.  Shapes already in
-   the table are not timed again.  path (nullable): a forms file, read first
-   and rewritten with the table.  The batch is left captured in its tuned
-   form (sister_graph_launch replays it). */
+   loops).  Launch forms that leave results unchanged: a batch's graph parts
+   (parts balanced by padded cells, or one part per disparity count, so that
+   groups of different D run side by side, and the parts started together or
+   each after the previous part's first stages), and for each disparity group
+   of those parts the SGM vertical families fused or separate.  They are kept in
+   the context's table, which every later plan and capture of a matching shape
+   consults: groups are matched by D and the half-octaves of their padded column
+   total and tallest padded rig, batches by rig count, distinct D count,
+   half-octave of padded cells and modes.  path (nullable): a forms file, read
+   into the table first and rewritten with it.  The batch is left captured in
+   its forms (sister_graph_launch replays it).  Timing the forms of shapes that
+   the table lacks is switched off (its repeated captures have ended in a crash
+   of the host process whose cause is not known): such a batch is refused with
+   SISTER_EINVAL, and sister_graph_capture runs it in the automatic forms. */
 int sister_autotune(sister_ctx* ctx, const sister_rig* rigs, int n, int modes, const char* path);
 /* The context's table of tuned forms as text, one form per line (the forms
    file's format). */

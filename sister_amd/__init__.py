@@ -226,9 +226,9 @@ class Context:
         self._check(lib().sister_graph_launch(self._h))
 
     def autotune(self, rigs, modes=MODE_MULTIVIEW, path=None):
-        """Time the launch forms of this batch (graph parts, then each D
-        group's SGM and cost-sum forms) and keep the fastest; the batch is
-        left captured in its tuned form.  path: forms file read and rewritten."""
+        """Capture the batch in the launch forms (graph parts, each D group's
+        SGM form) that the context's table holds for it, from the forms file
+        `path` or an earlier one; raises if a shape of the batch has none."""
         arr = (RigStruct * len(rigs))(*rigs)
         self._check(lib().sister_autotune(self._h, arr, len(rigs), modes,
                                           path.encode() if path else None))

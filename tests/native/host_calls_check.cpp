@@ -1,5 +1,6 @@
 // Drives the library's host code over the CPU stand-in of host_hip.cpp.
-//   host_calls_check NAME     runs one check; prints "ok"
+//   host_calls_check NAME [FILE]     runs one check; prints "ok"
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -141,6 +142,55 @@ void host_form_refused()
     CHECK(host_hip::pinned_bytes == 0);
 }
 
+int octave(double v) { return (int)std::floor(std::log2(v) * 2.0); }   // the forms file's half octaves
+double cells(const sister_rig& r)
+{
+    return (double)(r.width + 2 * r.disp_count) * (r.height + 2 * r.disp_count) * r.disp_count;
+}
+
+// sister_autotune captures a batch once, in the forms of a file; a batch with a
+// shape that no file names is refused before anything is captured.
+void forms_capture_once(const char* path)
+{
+    sister_ctx* c = create();
+    std::vector<Rig> rigs;
+    for (int k = 0; k < 4; k++) rigs.emplace_back(64 + 16 * k, 48, 8 * (k + 1), 30u + k);
+    std::vector<sister_rig> batch;
+    double total = 0;
+    for (Rig& r : rigs) {
+        batch.push_back(r.r);
+        total += cells(r.r);
+    }
+    CHECK(sister_graph_capture(c, batch.data(), 4, 1) == SISTER_OK);
+    CHECK(sister_autotune(c, batch.data(), 4, 1, nullptr) == SISTER_EINVAL);
+    CHECK(sister_autotune(c, batch.data(), 4, 1, path) == SISTER_EINVAL);
+    FILE* fp = std::fopen(path, "r");
+    CHECK(!fp);   // refused: no file is written
+    fp = std::fopen(path, "w");
+    std::fprintf(fp, "batch 4 4 %d 1 parts 2 by_d 0 stagger 0\n", octave(total));
+    for (Rig& r : rigs)
+        std::fprintf(fp, "group %d %d %d fused 0 kl 0 0 0 0 msum_split 0\n", r.D, octave(r.W + 2 * r.D), octave(r.H + 2 * r.D));
+    std::fclose(fp);
+    CHECK(host_hip::captures == 1);
+    // the first capture is still there
+    for (Rig& r : rigs) r.clear();
+    CHECK(sister_graph_launch(c) == SISTER_OK && sister_sync(c) == SISTER_OK);
+    for (Rig& r : rigs) CHECK(r.right(1));
+    CHECK(sister_autotune(c, batch.data(), 4, 1, path) == SISTER_OK);
+    CHECK(host_hip::captures == 2);
+    for (int i = 0; i < 3; i++) {
+        for (Rig& r : rigs) r.clear();
+        CHECK(sister_graph_launch(c) == SISTER_OK && sister_sync(c) == SISTER_OK);
+        for (Rig& r : rigs) CHECK(r.right(1));
+    }
+    // one more disparity count: not in the table
+    rigs.emplace_back(64, 48, 64, 40u);
+    batch.push_back(rigs.back().r);
+    CHECK(sister_autotune(c, batch.data(), 5, 1, path) == SISTER_EINVAL);
+    CHECK(host_hip::captures == 2);
+    sister_destroy(c);
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -149,6 +199,7 @@ int main(int argc, char** argv)
     if (name == "host_form_threads") host_form_threads();
     else if (name == "host_form_beside_batches") host_form_beside_batches();
     else if (name == "host_form_refused") host_form_refused();
+    else if (name == "forms_capture_once") forms_capture_once(argv[2]);
     else return 2;
     std::printf("ok\n");
     return 0;

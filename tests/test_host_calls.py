@@ -36,7 +36,8 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["host_form_threads", "host_form_beside_batches", "host_form_refused"])
-def test_host_calls(check, name):
-    r = subprocess.run([check, name], capture_output=True, text=True, timeout=120)
+@pytest.mark.parametrize("name", ["host_form_threads", "host_form_beside_batches", "host_form_refused",
+                                  "forms_capture_once"])
+def test_host_calls(check, name, tmp_path):
+    r = subprocess.run([check, name, str(tmp_path / "file")], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", (r.returncode, r.stdout + r.stderr)
