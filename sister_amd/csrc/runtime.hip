@@ -312,10 +312,11 @@ struct sister_ctx {
     // a captured batch runs as independent parts on their own streams
     // (parallel branches of the graph): one part's latency-bound stages (the
     // serial median, launch tails) overlap another part's work
-    static constexpr int kMaxParts = 8;
-    // a part per disparity count, up to one per hardware queue of the process:
-    // more branches would only share queues
-    static constexpr int kMaxDParts = 4;
+    // (at most four: the captures that ended in a crash of the host process,
+    // sister_autotune below, had five branches among them; that this was the
+    // cause is not shown.  Beyond four the branches share the process's four
+    // hardware queues.)
+    static constexpr int kMaxParts = 4;
     Plan graph_plan[kMaxParts];
     hipStream_t side[kMaxParts] = {};
     hipEvent_t ev_fork = nullptr, ev_join[kMaxParts] = {}, ev_stage[kMaxParts] = {};
@@ -1007,8 +1008,9 @@ static BatchKey batch_key(const sister_rig* rigs, int n, int modes)
 // under mu.  By default (or as tuned) the rigs are balanced by padded cells
 // over the parts, largest first to the lightest part; the tuned form may
 // instead give each disparity count a part of its own, so that groups of
-// different D run side by side.  SISTER_GRAPH_PARTS (1..8) overrides the
-// default part count (comparison runs).
+// different D run side by side (more counts than parts: kMaxParts balanced
+// ones).  SISTER_GRAPH_PARTS (1..kMaxParts) overrides the default part count
+// (comparison runs).  Larger counts, there or in a form, mean kMaxParts.
 static int partition_batch(sister_ctx* c, const sister_rig* rigs, int n, int modes,
                            std::vector<sister_rig> (&part)[sister_ctx::kMaxParts], int* stagger = nullptr)
 {
@@ -1033,11 +1035,12 @@ static int partition_batch(sister_ctx* c, const sister_rig* rigs, int n, int mod
         for (int i = 0; i < n; i++) ds.push_back(rigs[i].disp_count);
         std::sort(ds.begin(), ds.end());
         ds.erase(std::unique(ds.begin(), ds.end()), ds.end());
-        if ((int)ds.size() <= sister_ctx::kMaxDParts) {
+        if ((int)ds.size() <= sister_ctx::kMaxParts) {
             for (int i = 0; i < n; i++)
                 part[std::lower_bound(ds.begin(), ds.end(), rigs[i].disp_count) - ds.begin()].push_back(rigs[i]);
             return (int)ds.size();
         }
+        form.parts = sister_ctx::kMaxParts;
     }
     const int want = env_parts ? env_parts : form.parts > 0 ? form.parts : 2;
     const int nparts = std::max(1, std::min(std::min(want, (int)sister_ctx::kMaxParts), n));

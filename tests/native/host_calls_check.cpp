@@ -191,6 +191,37 @@ void forms_capture_once(const char* path)
     sister_destroy(c);
 }
 
+// Graph branches: as many as a form asks for, at most four.
+void graph_branches(const char* path)
+{
+    std::vector<Rig> rigs;
+    for (int k = 0; k < 9; k++) rigs.emplace_back(64, 48, 8 * (k % 6 + 1), 50u + k);
+    std::vector<sister_rig> batch;
+    double total = 0;
+    for (Rig& r : rigs) {
+        batch.push_back(r.r);
+        total += cells(r.r);
+    }
+    const struct { int n, parts, by_d, want; } cases[] = {{9, 1, 0, 1}, {9, 3, 0, 3}, {9, 4, 0, 4}, {9, 5, 0, 4}, {9, 8, 0, 4}, {9, 0, 1, 4}};
+    for (const auto& q : cases) {
+        sister_ctx* c = create();
+        FILE* fp = std::fopen(path, "w");
+        std::fprintf(fp, "batch %d 6 %d 1 parts %d by_d %d stagger 0\n", q.n, octave(total), q.parts, q.by_d);
+        // every split of the nine rigs: one or two of a disparity count in a part
+        for (int d = 8; d <= 48; d += 8)
+            for (int m = 1; m <= 2; m++)
+                std::fprintf(fp, "group %d %d %d fused 0 kl 0 0 0 0 msum_split 0\n", d, octave(m * (64 + 2 * d)), octave(48 + 2 * d));
+        std::fclose(fp);
+        host_hip::branches = 0;
+        CHECK(sister_autotune(c, batch.data(), q.n, 1, path) == SISTER_OK);
+        CHECK(host_hip::branches == q.want);
+        for (Rig& r : rigs) r.clear();
+        CHECK(sister_graph_launch(c) == SISTER_OK && sister_sync(c) == SISTER_OK);
+        for (Rig& r : rigs) CHECK(r.right(1));
+        sister_destroy(c);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -200,6 +231,7 @@ int main(int argc, char** argv)
     else if (name == "host_form_beside_batches") host_form_beside_batches();
     else if (name == "host_form_refused") host_form_refused();
     else if (name == "forms_capture_once") forms_capture_once(argv[2]);
+    else if (name == "graph_branches") graph_branches(argv[2]);
     else return 2;
     std::printf("ok\n");
     return 0;

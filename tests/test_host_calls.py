@@ -37,7 +37,7 @@ def check(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", ["host_form_threads", "host_form_beside_batches", "host_form_refused",
-                                  "forms_capture_once"])
+                                  "forms_capture_once", "graph_branches"])
 def test_host_calls(check, name, tmp_path):
     r = subprocess.run([check, name, str(tmp_path / "file")], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", (r.returncode, r.stdout + r.stderr)
