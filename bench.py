@@ -57,31 +57,56 @@ VALU_PEAK = 256 * 64 * 2.4e9      # int32 lane-ops/s: 256 CUs x 64 lanes/clk x 2
 HBM_PEAK = 8.0e12
 OPS_PER_CELL_PIPELINE = 97        # mode 0: costs 20, LR-check argmins 8, weighted sum 4, SGM 64, WTA 1
 
-# Algorithmic integer lane-ops per padded cell (W'*H'*D) of mode 0, split per
-# kernel: 4 directional costs (xor 2 + popcount 2 + invalid select 1 each = 20)
-# and the 8 LR-check argmins live in `wta`; the mask-weighted sum is 4; each
-# SGM path is 8 (+P1, min d-1, min d+1, min P2 term, -minL, +C, running min,
-# +S); the final argmin is 1.  Total 28 + 4 + 8*8 + 1 = 97.
-OPS_PER_CELL = {"wta": 28, "msum": 4, "sgm_rows": 16, "sgm_paths": 64, "winner": 1,
-                "sgm_vsweep": 49}   # the fused vertical sweep: 3 families x 2 sweeps x 8, + argmin
+# Integer lane-ops of mode 0 per cell that a kernel computes: 4 directional
+# costs (xor 2 + popcount 2 + invalid select 1 each = 20) and the 8 LR-check
+# argmins live in `wta`; the mask-weighted sum is 4; each SGM path is 8 (+P1,
+# min d-1, min d+1, min P2 term, -minL, +C, running min, +S); the final argmin
+# is 1.  Over every padded cell (W'*H'*D) that is 28 + 4 + 8*8 + 1 = 97.
+OPS_WTA, OPS_MSUM, OPS_PATH, OPS_ARGMIN = 28, 4, 8, 1
 
-# Algorithmic HBM bytes per padded cell of the HBM-bound kernels, with
-# `crop` the fraction of padded cells inside the crop (W*H of W'*H'): the
-# intermediates whose only reader is the final aggregate S are moved for those
-# cells alone, since S is read at the crop only.  The rows family ahead of the
-# fused sweep runs joined, reading M forward and again backward (2) and storing
-# one byte at crop cells (crop).  The fused vertical sweep (columns, diagonals,
-# anti-diagonals together) reads M going down and again going up (2) and, at
-# crop cells, the rows family's byte (1), the u16 partial sum P written going
-# down (2) and read going up (2): 2 + 5 crop.  The cost sum writes M once (1).
-# (The chains of smaller batches, sgm_paths, have forms that differ by group
-# and carry no figure here.)
-def bytes_per_cell(kernel, crop):
-    if kernel == "sgm_rows":
-        return 2 + crop
-    if kernel == "sgm_vsweep":
-        return 2 + 5 * crop
-    return {"msum": 1}.get(kernel)
+
+def kernel_work(rigs):
+    """Lane-ops and HBM bytes per padded cell of each kernel's work as the
+    kernels divide it, over the rigs (dicts with W, H, D): {kernel: (ops, bytes)},
+    bytes None where no figure is given; and `crop`, the crop's share of the cells.
+
+    S is read at the crop only, so a path runs from its border to its last crop
+    cell, and what only S needs is moved at crop cells:
+      wta        every row but the deep padding bands' copies
+      msum       every padded cell, M written once
+      sgm_rows   H rows of W + D cells a direction; M read at each, one byte
+                 stored at crop cells (joined, ahead of the fused sweep)
+      sgm_vsweep columns and both diagonals together, H' - D rows down and as
+                 many up, all W' columns; M read at each and, at crop cells, the
+                 rows family's byte read, the u16 partial sum P written and read
+      sgm_paths  all eight paths as chains; forms that differ by group move
+                 different bytes (no figure)
+      winner     the crop"""
+    total = 0
+    ops = dict.fromkeys(("wta", "msum", "sgm_rows", "sgm_vsweep", "sgm_paths", "winner"), 0.0)
+    rows_b = sweep_b = crop_cells = 0
+    for r in rigs:
+        W, H, D = r["W"], r["H"], r["D"]
+        Wp, Hp = W + 2 * D, H + 2 * D
+        total += Wp * Hp * D
+        crop = W * H * D
+        crop_cells += crop
+        rows = 2 * (W + D) * H * D
+        cols = 2 * (H + D) * W * D
+        sweep = 2 * (Hp - D) * Wp * D
+        # a diagonal x - y = k from its border to its last crop cell; the other
+        # three directions are reflections of it
+        diag = 4 * D * sum(min(D + H - 1, D + W - 1 - k) - max(0, -k) + 1 for k in range(1 - H, W))
+        ops["wta"] += OPS_WTA * (Wp * Hp - (D - 7) * (Wp + Hp)) * D
+        ops["msum"] += OPS_MSUM * Wp * Hp * D
+        ops["sgm_rows"] += OPS_PATH * rows
+        ops["sgm_vsweep"] += 3 * OPS_PATH * sweep + OPS_ARGMIN * crop
+        ops["sgm_paths"] += OPS_PATH * (rows + cols + diag)
+        ops["winner"] += OPS_ARGMIN * crop
+        rows_b += rows + crop
+        sweep_b += sweep + 5 * crop
+    byt = {"msum": 1.0, "sgm_rows": rows_b / total, "sgm_vsweep": sweep_b / total}
+    return {k: (v / total, byt.get(k)) for k, v in ops.items()}, crop_cells / total
 
 
 # per-kernel counter totals of one instrumented step (used when their batch
@@ -253,21 +278,8 @@ def run_single(args):
 # ---------------------------------------------------------------------------
 # headline: plain vs batched at 1920x1080 D=192
 # ---------------------------------------------------------------------------
-def wta_copied_fraction(rigs):
-    """Fraction of the WTA's cost evaluations (padded cells x 4 frames) that
-    fall on the deep padding bands' rows, [3, D-4] and [R-D+3, R-4] of every
-    frame, which copy the band's first row instead of computing it."""
-    done = total = 0
-    for r in rigs:
-        W, H, D = r["W"], r["H"], r["D"]
-        Wp, Hp = W + 2 * D, H + 2 * D
-        # copied: 2 bands x (D-7) rows x (2 W' + 2 H') columns x D, of 4 W' H' D
-        total += Wp * Hp * D
-        done += (D - 7) * (Wp + Hp) * D
-    return done / total
-
-
-def roofline_entry(kern, launches, cells, step_ms, B, workload, crop, wta_copied=0.0):
+def roofline_entry(kern, launches, cells, step_ms, B, workload, rigs):
+    work, crop = kernel_work(rigs)
     traffic = None
     per_kernel_traffic = {}
     valu = {}
@@ -282,9 +294,10 @@ def roofline_entry(kern, launches, cells, step_ms, B, workload, crop, wta_copied
             valu = v.get("kernels", {})
     step_s = step_ms * 1e-3
     achieved = OPS_PER_CELL_PIPELINE * cells / step_s
-    # the same without the WTA evaluations of the deep padding bands, which
-    # the kernels copy rather than compute
-    executed = OPS_PER_CELL_PIPELINE - OPS_PER_CELL["wta"] * wta_copied
+    # the same by the work that the batch's kernels compute: fused and separate
+    # groups in one batch count as separate, the smaller figure
+    ran = ("sgm_paths", "winner") if "sgm_paths" in kern else ("sgm_rows", "sgm_vsweep")
+    executed = sum(work[k][0] for k in ("wta", "msum") + ran)
     roof = {"bound": "valu", "scope": "whole step (every kernel of the batch)",
             "achieved": achieved / 1e12, "peak": VALU_PEAK / 1e12, "unit": "T int-lane-ops/s",
             "frac": achieved / VALU_PEAK, "ops_per_cell": OPS_PER_CELL_PIPELINE,
@@ -297,12 +310,12 @@ def roofline_entry(kern, launches, cells, step_ms, B, workload, crop, wta_copied
     dom = max(kern, key=lambda k: kern[k])
     n = launches.get(dom) or 1
     avg_ms = kern[dom] / n
-    ops = OPS_PER_CELL.get(dom, 0) * cells
-    d = {"kernel": dom, "bound": "valu", "ops_per_cell": OPS_PER_CELL.get(dom, 0),
+    dom_ops, bpc = work.get(dom, (0, None))
+    ops = dom_ops * cells
+    d = {"kernel": dom, "bound": "valu", "ops_per_cell": dom_ops,
          "launches_per_step": n, "avg_launch_ms": avg_ms,
          "achieved": ops / n / (avg_ms * 1e-3) / 1e12, "peak": VALU_PEAK / 1e12, "unit": "T int-lane-ops/s",
          "frac": ops / n / (avg_ms * 1e-3) / VALU_PEAK}
-    bpc = bytes_per_cell(dom, crop)
     if bpc is not None:
         alg = bpc * cells
         d.update({"bytes_per_cell": bpc, "crop_fraction": crop,
@@ -437,8 +450,7 @@ def run(args):
         "batched_compared": f"disp and multiview maps of all {B} rigs against their scene computed alone",
         "padded_cells_per_step": cells,
         "padded_cells_per_s": cells / (step_ms * 1e-3),
-        "roofline": roofline_entry(kern, launches, cells, step_ms, B, args.workload, evals / cells,
-                                   wta_copied_fraction(rigs)),
+        "roofline": roofline_entry(kern, launches, cells, step_ms, B, args.workload, rigs),
         "kernel_ms": kern,
         "kernel_launches_per_step": launches,
     }
