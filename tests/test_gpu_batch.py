@@ -436,3 +436,70 @@ def test_joined_chains_match_oracle(gpu_ctx, oracle_mod, W, H, D):
     for i in range(n):
         for k in names:
             assert np.array_equal(outs[i][k].cpu().numpy(), refs[i % 2][k]), (i, k)
+
+
+@pytest.mark.parametrize("W,H,D", [(320, 304, 64), (256, 4, 256), (4, 256, 256), (256, 8, 384), (8, 240, 384),
+                                   (256, 4, 512), (4, 256, 512)])
+def test_joined_chains_full_lanes(gpu_ctx, oracle_mod, W, H, D):
+    """The joined form with every lane full (8, 12 and 16 pairs) and with crops
+    of many segments, all three modes: equal to the rig alone, whose chains run
+    apart (that form is held against the oracle at these disparity counts by
+    the parity tests), and at D = 64 to the oracle."""
+    import torch
+    waves = (W + 3) // 4 + 2 * ((W + H + 2) // 4)
+    n = -(-1024 // waves)
+    assert waves < 1024 and n >= 2
+    rigs = [synth.rig_small(W, H, D, 900 + D + k) for k in range(2)]
+    views = [[torch.from_numpy(v).cuda() for v in r["views"]] for r in rigs]
+    names = ("multiview", "horizontal", "vertical", "disp")
+
+    def outputs():
+        o = {k: torch.zeros((H, W), dtype=torch.uint16, device="cuda") for k in names}
+        o["subpix"] = torch.zeros((H, W), dtype=torch.float32, device="cuda")
+        return o
+
+    alone = [outputs() for _ in range(2)]
+    for v, o in zip(views, alone):
+        gpu_ctx.run_device([gpu_ctx.rig_struct(v, D, o)], sister_amd.MODE_ALL)
+        gpu_ctx.sync()
+    outs = [outputs() for _ in range(n)]
+    print(f"[joined full] {n} rigs W={W} H={H} D={D}", flush=True)
+    gpu_ctx.vsweep(0)
+    try:
+        gpu_ctx.run_device([gpu_ctx.rig_struct(views[i % 2], D, outs[i]) for i in range(n)], sister_amd.MODE_ALL)
+        gpu_ctx.sync()
+    finally:
+        gpu_ctx.vsweep(-1)
+    for i in range(n):
+        for k in outs[i]:
+            assert np.array_equal(outs[i][k].cpu().numpy(), alone[i % 2][k].cpu().numpy()), (i, k)
+    if D == 64:
+        for k, r in enumerate(rigs):
+            ref = oracle_mod.compute(r["views"], D, modes=7)
+            for q in names:
+                assert np.array_equal(outs[k][q].cpu().numpy(), ref[q]), (k, q)
+
+
+def test_host_form_threads_share_a_context(gpu_ctx, oracle_mod):
+    """Threads in the class on one context, with rigs on both sides of the line
+    between one copy for all views and a copy per view: each gets its own maps."""
+    import threading
+    shapes = [(64, 48, 16), (516, 512, 8), (128, 96, 24)]
+    rigs = [synth.rig_small(W, H, D, 950 + D) for W, H, D in shapes]
+    refs = [oracle_mod.compute(r["views"], r["D"], modes=7) for r in rigs]
+    bad = []
+
+    def work(r, ref):
+        c = sister_amd.SisterMultiviewDisparities(*r["views"], context=gpu_ctx)
+        for i in range(6):
+            got = c.compute_disparities(r["D"])
+            bad.extend((r["W"], i, k) for k, g in zip(("multiview", "horizontal", "vertical"), got)
+                       if not np.array_equal(g, ref[k]))
+
+    print("[host threads] 3 threads, one context", flush=True)
+    threads = [threading.Thread(target=work, args=a) for a in zip(rigs, refs)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad
