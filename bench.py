@@ -6,7 +6,7 @@ mode 0 (multiview).  Two forms are measured on the same synthetic rigs, with
 inputs and outputs resident in HBM before the timed region:
 
   plain    one rig per call of the library (sister_run_device with n = 1),
-  batched  B rigs in one plan (default 64: 229 GB of workspace), captured
+  batched  B rigs in one plan (default 64: 192 GB of workspace), captured
            once as a hipGraph in the automatic launch forms (or those of a
            file, --forms) and replayed.
 

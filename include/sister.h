@@ -118,7 +118,7 @@ int sister_outside_reference_domain(int disp_count);
 int sister_graph_capture(sister_ctx* ctx, const sister_rig* rigs, int n, int modes);
 int sister_graph_launch(sister_ctx* ctx);
 
-/* ---- autotuning ----------------------------------------------------------- */
+/* ---- launch forms --------------------------------------------------------- */
 /* No counterpart in the reference (its launch shapes are fixed by its SSE
    loops).  Launch forms that leave results unchanged: a batch's graph parts
    (parts balanced by padded cells, or one part per disparity count, so that
@@ -135,8 +135,8 @@ int sister_graph_launch(sister_ctx* ctx);
    of the host process whose cause is not known): such a batch is refused with
    SISTER_EINVAL, and sister_graph_capture runs it in the automatic forms. */
 int sister_autotune(sister_ctx* ctx, const sister_rig* rigs, int n, int modes, const char* path);
-/* The context's table of tuned forms as text, one form per line (the forms
-   file's format). */
+/* The context's table of forms as text, one form per line (the forms file's
+   format). */
 int sister_tune_describe(sister_ctx* ctx, char* buf, size_t len);
 
 /* ---- serving: continuous batching by HBM footprint ---------------------- */
@@ -169,8 +169,10 @@ int sister_stats_get(sister_ctx* ctx, sister_stats* out);
 /* ---- instrumentation and test access ----------------------------------- */
 /* Per-kernel device time (HIP events around each kernel's launches on the
    stream they run on) accumulated while enabled: names[i] / ms[i] /
-   launches[i] (kernel dispatches issued) for i < returned count.  Profiled
-   runs issue the SGM families one after another. */
+   launches[i] (kernel dispatches issued) for i < returned count.  Names:
+   census, wta, median_prep, median_serial, mask, msum, sgm_rows and sgm_vsweep
+   (the rows paths and the fused vertical sweep), sgm_paths and winner (all
+   paths as separate chains).  Profiled runs issue the same launches. */
 int sister_profile_enable(sister_ctx* ctx, int on);
 int sister_profile_read(sister_ctx* ctx, const char** names, double* ms, int* launches, int max);
 /* Copy an intermediate of rig `index` of the last run to host memory:
@@ -182,15 +184,15 @@ int sister_debug_fetch(sister_ctx* ctx, int index, const char* what, int which, 
    last sweep consumes it for cells inside the crop). */
 int sister_debug_keep_sum(sister_ctx* ctx, int on);
 /* Form of the SGM vertical families (columns, diagonals, anti-diagonals) in
-   plans built afterwards: 0 = one chain sweep per family, 1 = the fused
+   plans built afterwards: 0 = all paths as separate chains, 1 = the fused
    vertical sweep wherever the disparity count allows it (D <= 384),
    -1 = automatic (fused for batches wide enough to fill the device).
    Results are identical either way. */
 int sister_debug_vsweep(sister_ctx* ctx, int mode);
 /* Plans built afterwards keep the fused vertical sweep's partial sums over
-   the rows family's bytes, the smaller layout (2.29 against 3.59 GB per
-   1920x1080 D=192 rig, 0.7% slower) that plans take by themselves when they
-   do not fit otherwise.  Results are identical either way. */
+   the rows family's bytes, the smaller layout (2.29 against 3.00 GB per
+   1920x1080 D=192 rig, 5% slower) that plans take by themselves when they do
+   not fit otherwise.  Results are identical either way. */
 int sister_debug_sweep_in_place(sister_ctx* ctx, int on);
 
 #ifdef __cplusplus

@@ -282,7 +282,7 @@ class Context:
         self._check(lib().sister_debug_keep_sum(self._h, 1 if on else 0))
 
     def vsweep(self, mode):
-        """Vertical SGM families: 0 separate sweeps, 1 fused sweep, -1 automatic."""
+        """Vertical SGM families: 0 separate chains, 1 fused sweep, -1 automatic."""
         self._check(lib().sister_debug_vsweep(self._h, int(mode)))
 
     def sweep_in_place(self, on=True):

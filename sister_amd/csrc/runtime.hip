@@ -232,7 +232,7 @@ constexpr size_t kScratchBytes = SISTER_NOALLOC_MAX_BYTES;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // ---------------------------------------------------------------------------
-// Launch forms chosen by the autotuner (sister_autotune).  A disparity group
+// Launch forms read from a forms file (sister_autotune).  A disparity group
 // of a plan (its rigs of one D) is keyed by D and the octaves of its padded
 // column total and tallest padded rig; a captured batch by its rig count, its
 // distinct D count, the octave of its padded cells and its modes.  Every form
@@ -240,13 +240,11 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 // ---------------------------------------------------------------------------
 struct GroupForm {
     int fused = -1;           // -1 automatic, 0 separate chains, 1 fused vertical sweep
-    int kl[4] = {0, 0, 0, 0}; // a field of the forms file; chains always take 16 lanes
-    int msum_split = 0;       // a field of the forms file; the cost sum has one form per disparity count
-    bool operator==(const GroupForm& o) const
-    {
-        return fused == o.fused && msum_split == o.msum_split && kl[0] == o.kl[0] && kl[1] == o.kl[1] &&
-               kl[2] == o.kl[2] && kl[3] == o.kl[3];
-    }
+    // fields of the file's format that choose nothing (chains always take 16
+    // lanes, the cost sum has one form per disparity count), held so that a file
+    // is written back as it was read
+    int kl[4] = {0, 0, 0, 0};
+    int msum_split = 0;
 };
 struct BatchForm {
     int parts = 0;            // independent graph parts (0: automatic)
@@ -304,8 +302,8 @@ struct sister_ctx {
     Plan last;                 // plan of the last sister_run_device (kept for debug fetch)
     uint64_t issued = 0;       // plans that `last` has held (under mu)
     Plan noalloc;              // plan of the last sister_run_device_noalloc (in the scratch array)
-    std::map<GroupKey, GroupForm> gforms;   // autotuned group forms (under mu)
-    std::map<BatchKey, BatchForm> bforms;   // autotuned batch forms (under mu)
+    std::map<GroupKey, GroupForm> gforms;   // group forms (under mu)
+    std::map<BatchKey, BatchForm> bforms;   // batch forms (under mu)
     char* scratch = nullptr;   // this device's scratch array (scratch_address)
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -435,7 +433,8 @@ constexpr long kJoinWaves = SISTER_JOIN_WAVES;
 // The rig table is ordered by D so that the SGM launches can take each group
 // of equal depth as one contiguous slice.
 // p_in_place: fused groups keep their partial sums over the rows family's
-// bytes (smaller workspaces, 0.7% slower): the retry of a plan that does not
+// bytes (smaller workspaces; an eager step of 64 rigs 1920x1080 D=192 takes
+// 140.5 ms against 133.2, for 147 GB against 192): the retry of a plan that does not
 // fit otherwise
 static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Carve* carve = nullptr,
                       bool p_in_place = false)
@@ -501,7 +500,7 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         GroupForm form;
         const auto it = c->gforms.find(GroupKey{D, octave((double)chains), octave((double)G.maxHp)});
         if (it != c->gforms.end()) form = it->second;
-        // the debug switch wins over a tuned form
+        // the debug switch wins over the table's form
         G.vcols = vsweep_pick_cols(chains, D, c->vsweep >= 0 ? c->vsweep : form.fused);
         long waves = 0;
         for (int j = k; j < e; j++)
@@ -510,8 +509,7 @@ static int build_plan(sister_ctx* c, const sister_rig* rigs, int n, Plan& p, Car
         groups.push_back(G);
         k = e;
     }
-    // workspaces: a rig of a fused group has four SGM volumes (two in place),
-    // the others five
+    // workspaces: ws_layout's forms by group
     std::vector<WsLayout> lay(n);
     for (GroupHost& G : groups) {
         bool lay_join = false;
@@ -1005,8 +1003,8 @@ static BatchKey batch_key(const sister_rig* rigs, int n, int modes)
 }
 
 // The independent parts of a captured batch (parallel branches of its graph),
-// under mu.  By default (or as tuned) the rigs are balanced by padded cells
-// over the parts, largest first to the lightest part; the tuned form may
+// under mu.  By default the rigs are balanced by padded cells over two parts,
+// largest first to the lightest part; a form may name another count, or
 // instead give each disparity count a part of its own, so that groups of
 // different D run side by side (more counts than parts: kMaxParts balanced
 // ones).  SISTER_GRAPH_PARTS (1..kMaxParts) overrides the default part count
@@ -1133,7 +1131,7 @@ int sister_graph_launch(sister_ctx* c)
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
-// autotuning
+// launch forms
 // ---------------------------------------------------------------------------
 static std::string forms_text(const sister_ctx* c)
 {
@@ -1232,7 +1230,7 @@ int sister_autotune(sister_ctx* c, const sister_rig* rigs, int n, int modes, con
         HIPCHK(c, hipStreamSynchronize(c->stream));
         free_plan(c, c->last);   // room for the capture
     }
-    // the batch captured in its tuned form
+    // the batch captured in its forms
     if ((rc = sister_graph_capture(c, rigs, n, modes))) return rc;
     if (path) {
         std::lock_guard<std::mutex> lk(c->mu);

@@ -188,10 +188,10 @@ def test_plain_640x480_d64(gpu_ctx, oracle_mod):
     assert float(np.abs(got["subpix"] - ref["subpix"]).max()) <= 1e-3
 
 
-# frames wider than 4096 pixels take the serial median's prepass form (8 slots
-# per thread up to 8192, 16 beyond); the others sort the six fixed values in
-# the serial kernel.  W' = 4136 and 8232 wide frames 0/180, H' = 4136 tall
-# (so 4136-wide frames 90/270).
+# frames wider than 4096 pixels: the serial median in strips of 6 and of 10 pairs
+# of columns a lane, up to eight waves (k_median_wide starts past 9920 columns).
+# W' = 4136 and 8216 wide frames 0/180, H' = 4136 tall (so 4136-wide frames
+# 90/270).
 @pytest.mark.parametrize("W,H,D,seed", [(4104, 16, 16, 21), (16, 4104, 16, 22), (8200, 12, 8, 23)])
 def test_stages_bit_exact_wide_frames(gpu_ctx, oracle_mod, W, H, D, seed):
     print(f"[parity wide] W={W} H={H} D={D} seed={seed}", flush=True)
@@ -199,10 +199,9 @@ def test_stages_bit_exact_wide_frames(gpu_ctx, oracle_mod, W, H, D, seed):
     assert not bad, bad
 
 
-# disparity counts beyond 192: wider SGM lane states, the tiled cost sum at 4
-# groups of 64 (D = 200, 256) and the two-launch cost sum beyond, the row WTA's
-# start-of-row segment when D > 256 (lane 63's leaving pixel before column 0),
-# and D = 512, the largest accepted.  Tiny visible sizes keep the oracle's
+# disparity counts beyond 192: 8, 12 and 16 pairs of disparities per lane of the
+# chains, the cost sum in two to four blocks of 128 disparities to a tile, the
+# median without its prepass (D > 256), and D = 512, the largest accepted.  Tiny visible sizes keep the oracle's
 # volumes in seconds (W' x H' x D up to 543 M cells at D = 512).
 @pytest.mark.parametrize("W,H,D,seed", [(16, 16, 200, 81), (16, 16, 256, 82), (16, 16, 264, 83),
                                         (16, 12, 320, 84), (8, 8, 384, 85), (8, 4, 512, 86)])
